@@ -51,28 +51,21 @@
 //     and (in the KTail instantiation, K % 64 != 0) K-contiguous chunks and
 //     MN-contiguous rows past K on the last step, get an offset past the
 //     range; the epilogue stores only rows < M and 8-column chunks < N.
-// Small-tile kernel (64 x 64 or 32 x 32 tiles): shapes with few 256 x 256
-// tiles, and any shape or alignment the fast kernel does not take.
+// Products with too few 256 x 256 tiles for the chip run smaller tiles
+// (k_gemm_f16_tile.hip, gemm_f16_tile).  Small-tile kernel below (64 x 64 or
+// 32 x 32 tiles): any shape or alignment the fast kernel does not take.
 #include "../../include/ipus.h"
 
 #include <mutex>
 
-#include "device_common.h"
+#include "gemm_f16_common.h"
 #include "kernels.h"
-
-#define LDS_AS __attribute__((address_space(3)))
 
 namespace ipus {
 namespace {
 
 constexpr int kBM = 256, kBN = 256;
 constexpr int kThreads = 256;
-constexpr int kBufferFlags = 0x00020000;  // raw buffer, dword 3 of the descriptor
-
-typedef short short4_t __attribute__((vector_size(8)));
-
-inline int hip_status(hipError_t e) { return e == hipSuccess ? 0 : IPUS_ERROR_HIP_BASE - (int)e; }
-
 // K-contiguous tile [256 rows][BK k]: byte offset of (row, 16-byte chunk).
 // A fragment read covers 16 consecutive rows and, per 16-lane group, one
 // chunk (4 chunks per instruction); XOR-ing the chunk with the row's low 3
@@ -94,11 +87,6 @@ __device__ __forceinline__ uint32_t mc_off(uint32_t k, uint32_t chunk) {
   return k * 512u + ((chunk ^ (x << 1)) << 4);
 }
 
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, uint8_t* lds, uint32_t voffset,
-                                      uint32_t soffset) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (LDS_AS void*)lds, 16, voffset, soffset, 0, 0);
-}
-
 template <int BK>
 struct Tile {
   static constexpr int kBytes = kBM * BK * 2;         // one operand tile
@@ -109,12 +97,6 @@ struct Tile {
 // offset) of the DMA instructions this wave issues for one operand tile.  The
 // DMA writes lane i at base + 16 i, so each lane fetches the global chunk
 // that the swizzle places at its LDS slot.
-// Offset of a chunk outside the operand (past M or N along an MN-contiguous
-// row, or past K on the last K step of a K-contiguous row): beyond every
-// buffer range (< 2^31) plus any K offset (< 2^31) without wrapping, so the
-// load returns 0.
-constexpr uint32_t kPadOffset = 0x80000000u;
-
 template <int BK, bool KContig>
 __device__ __forceinline__ void tile_offsets(uint32_t wave, uint32_t lane, uint32_t ld,
                                              uint32_t mn_limit, uint32_t* voff) {
@@ -163,34 +145,6 @@ __device__ __forceinline__ void issue_one(__amdgpu_buffer_rsrc_t rsrc, uint8_t* 
     }
   }
   dma16(rsrc, tile + inst * 1024, voff, soffset);
-}
-
-// Epilogues: the plain fp16 product; GELU of it; or the sum of it and an
-// addend element (C += A . B, the reference's accumulate mode).
-enum Epilogue : int { kEpiPlain = 0, kEpiGelu = 1, kEpiAdd = 2 };
-
-// fp16 result of one accumulator; with GELU, GELU of that fp16 value (the
-// same number the separate GELU kernel would produce from the stored GEMM
-// output).  The add epilogue applies add_f16 to this value afterwards.
-template <int Epi>
-__device__ __forceinline__ half_t epilogue(float acc) {
-  const half_t h = (half_t)acc;
-  if constexpr (Epi == kEpiGelu) return (half_t)gelu_tanh((float)h);
-  return h;
-}
-
-// The fp16 Add kernel's arithmetic (k_memory.hip add_kernel): both operands
-// widened to fp32, summed, rounded once to fp16, so a fused accumulate is
-// bit-identical to a GEMM followed by an Add.
-__device__ __forceinline__ half_t add_f16(half_t product, half_t addend) {
-  return (half_t)((float)addend + (float)product);
-}
-__device__ __forceinline__ u32x4 add_f16x8(u32x4 product, u32x4 addend) {
-  const half8_t p = __builtin_bit_cast(half8_t, product), a = __builtin_bit_cast(half8_t, addend);
-  half8_t r;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) r[e] = add_f16(p[e], a[e]);
-  return __builtin_bit_cast(u32x4, r);
 }
 
 // Split: workgroup z covers K range [z k_chunk, (z + 1) k_chunk) (k_chunk a
@@ -460,9 +414,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
   }
 }
 
-// Small fp16 GEMM: 64 x 64 or 32 x 32 output tiles, for shapes with fewer
-// 256 x 256 tiles than kSmallBelowTiles, which would keep few of the 256
-// CUs busy (configs[0]'s 256^3 is a single such tile).  256 threads = 4
+// Register-staged fp16 GEMM: 64 x 64 or 32 x 32 output tiles, for operands the
+// LDS-DMA kernels do not take (row pitches or addresses that are not 16-byte
+// multiples, operands past their 31-bit buffer ranges, K = 0).  256 threads = 4
 // waves in a 2 x 2 grid, each (Tile / 2)^2 of C as tiles of
 // v_mfma_f32_16x16x32_f16 (C^T as in the 256 x 256 kernel, so a lane holds
 // 4 consecutive columns).  K runs in chunks of 256: a chunk's
@@ -474,13 +428,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
 // MN-contiguous tiles [64 k][64 mn] are read with ds_read_b64_tr_b16.
 // Chunks past M, N or K are not loaded and stay 0.  Vec = 8: N and K, and
 // M when A is transposed, are multiples of 8 and the operands 16-byte
-// aligned, as for the 256 x 256 kernel.  Vec = 4 or 1 (any other shape or
+// aligned (operands past the 256 x 256 kernel's ranges).  Vec = 4 or 1 (any other shape or
 // alignment, where the 256 x 256 kernel cannot run): each 16-byte LDS chunk
 // is gathered from 8-byte or 2-byte loads, elements past M, N or K are 0,
 // and the epilogue stores element by element.
 constexpr uint32_t kSmallChunk = 256;
 constexpr uint32_t kSmallSteps = kSmallChunk / 64;
-constexpr uint64_t kSmallBelowTiles = 32;
 
 template <uint32_t Tile, bool TransposeLeft, bool TransposeRight, int Epi, int Vec = 8>
 __global__ __launch_bounds__(256) void gemm_f16_small_kernel(
@@ -844,17 +797,8 @@ int launch_gemm_f16(hipStream_t stream, const GemmArgs& a) {
   // Any M and N on the fast kernel: rows past the edge read as 0 and are not
   // stored.
   if (fast_ok(a)) {
-    // Fewer 256 x 256 tiles than kSmallBelowTiles: the small-tile kernel
-    // (measured: 256^3 10.7 -> 5.3 us a launch, 1024^3 22 -> 9.6, but
-    // 2048^3 with 64 tiles 40 -> 47).
-    const uint64_t tiles = (uint64_t)((a.rows + kBM - 1) / kBM) * ((a.columns + kBN - 1) / kBN);
-    if (tiles * a.batches < kSmallBelowTiles) {
-      switch (epilogue_of(a)) {
-        case kEpiGelu: return launch_small<kEpiGelu>(stream, a);
-        case kEpiAdd: return launch_small<kEpiAdd>(stream, a);
-        default: return launch_small<kEpiPlain>(stream, a);
-      }
-    }
+    const uint32_t tile = gemm_f16_tile(a.rows, a.columns, a.inner, a.batches);
+    if (tile != 256) return launch_gemm_f16_tile(stream, a, tile);
     switch (epilogue_of(a)) {
       case kEpiGelu: return dispatch_fast<kEpiGelu, false>(stream, a, 1, a.inner);
       case kEpiAdd: return dispatch_fast<kEpiAdd, false>(stream, a, 1, a.inner);

@@ -1,0 +1,79 @@
+"""The fp16 GEMM's 128 x 128, 64 x 64 and 32 x 32 tile kernels against float64, at
+the edges of their tiles and K steps, in every layout, batch form and epilogue
+(the launch picks the tile from the shape; each shape below names the tile it
+was chosen for)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def operands(ipus, oracle, M, N, K, tl, tr, batches, shared):
+    a = ipus.synth_f16(batches * M * K, 71, 1, 0, 1.0)
+    b = ipus.synth_f16((1 if shared else batches) * K * N, 71, 2, 0, 1.0)
+    af = oracle.f16_to_f32(a).astype(np.float64).reshape((batches, K, M) if tl else (batches, M, K))
+    bf = oracle.f16_to_f32(b).astype(np.float64).reshape((-1, N, K) if tr else (-1, K, N))
+    af = af.transpose(0, 2, 1) if tl else af
+    bf = bf.transpose(0, 2, 1) if tr else bf
+    return a, b, af, bf
+
+
+def assert_product(got, af, bf, K):
+    """One fp16 rounding (2^-11 of the value, 2^-25 below the normal range)
+    of an fp32 sum of K exact products, each addition within 2^-24 of the
+    running magnitude."""
+    want, magnitude = np.matmul(af, bf), np.matmul(np.abs(af), np.abs(bf))
+    bound = (np.abs(want) * 2.0 ** -11 + 2.0 ** -25) * 1.001 + magnitude * (K + 2) * 2.0 ** -24
+    assert np.all(np.abs(got - want) <= bound)
+
+
+SHAPES = [  # tile 128: a partial tile along M and N, a partial last K step
+          (1800, 2056, 584), (1792, 2048, 640),
+          # tile 64: fewer than four K steps left over, partial tiles
+          (520, 1160, 1160), (512, 1024, 1152),
+          # tile 32: one K step and part of one, single tiles, one row of tiles
+          (256, 256, 256), (8, 8, 8), (40, 72, 264), (32, 32, 128), (8, 4096, 1032)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("tl,tr", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_f16_tiles(ipus, oracle, ctx, M, N, K, tl, tr):
+    a, b, af, bf = operands(ipus, oracle, M, N, K, tl, tr, 1, True)
+    da, db = ctx.upload(a), ctx.upload(b)
+    out = ctx.upload(np.full(M * N + 8, 0x7E00, np.uint16))
+    ctx.launch("ipu_stack_gemm_f16", out, [da, db], [1, M, N, K, tl, tr, 0, 0])
+    raw = out.download(np.uint16)
+    assert np.all(raw[M * N:] == 0x7E00)  # nothing stored past C
+    assert_product(oracle.f16_to_f32(raw[:M * N]).reshape(1, M, N), af, bf, K)
+    for x in (da, db, out):
+        x.free()
+
+
+@pytest.mark.parametrize("M,N,K", [(601, 1032, 584), (264, 392, 1160), (33, 72, 200)])
+@pytest.mark.parametrize("shared", [True, False])
+@pytest.mark.parametrize("epilogue", ["none", "gelu", "add"])
+def test_gemm_f16_tiles_batches_and_epilogues(ipus, oracle, ctx, M, N, K, shared, epilogue):
+    """Batched, the right operand shared or not; the fused epilogues give the
+    bits of the product followed by the GELU or Add kernel."""
+    B = 5
+    a, b, af, bf = operands(ipus, oracle, M, N, K, 0, 1, B, shared)
+    n = B * M * N
+    da, db, out = ctx.upload(a), ctx.upload(b), ctx.alloc(n * 2)
+    sc = [B, M, N, K, 0, 1, M * K, 0 if shared else K * N]
+    ctx.launch("ipu_stack_gemm_f16", out, [da, db], sc)
+    if epilogue == "none":
+        got = oracle.f16_to_f32(out.download(np.uint16)).reshape(B, M, N)
+        assert_product(got, af, bf, K)
+    elif epilogue == "gelu":
+        want, fused = ctx.alloc(n * 2), ctx.alloc(n * 2)
+        ctx.launch("ipus_gelu_f16", want, [out], [n])
+        ctx.launch("ipu_stack_gemm_f16_gelu", fused, [da, db], sc)
+        assert np.array_equal(fused.download(np.uint16), want.download(np.uint16))
+    else:
+        d = ctx.upload(ipus.synth_f16(n, 71, 3, 0, 1.0))
+        want = ctx.alloc(n * 2)
+        ctx.launch("ipu_stack_add_f16", want, [out, d], [n, n, n])
+        ctx.launch("ipu_stack_gemm_f16_accumulate", d, [da, db, d], sc + [M * N, N])  # in place
+        assert np.array_equal(d.download(np.uint16), want.download(np.uint16))
