@@ -12,7 +12,8 @@
 // 128 or 256 columns wide with zero padding; for equal widths the MFMAs
 // cover the width rounded up to 32 columns):
 //   * 256 threads = 4 waves; a wave owns 32 queries (two tiles of 16; one
-//     tile at 256 columns), a workgroup 128 (64) queries of one stream; two
+//     tile at 256 columns, and where the launch would leave CUs idle, see
+//     fast_plan), a workgroup 128 (64) queries of one stream; two
 //     workgroups share a CU (launch bound), so one SIMD runs the softmax of
 //     one wave while the MFMA pipe serves the other;
 //   * keys stream through LDS in blocks of 64 (32 at 256 columns) with two
@@ -46,9 +47,9 @@
 //     one base), so the cluster's LDS reads take immediate offsets only;
 //   * causal: key blocks past the workgroup's last query are never loaded, a
 //     wave skips blocks past its own last query.
-//   * a workgroup runs two query blocks of one stream back to back (causal:
-//     n - 1 - i and then i, so every workgroup has the same number of key
-//     steps); the first block's last step prefetches the second's first K
+//   * a workgroup runs two query blocks of one stream back to back where the
+//     launch still fills the chip (causal: n - 1 - i and then i, so every
+//     workgroup has the same number of key steps); the first block's last step prefetches the second's first K
 //     tile and Q fragments;
 //     workgroups are remapped so each XCD (round-robin dispatch over 8) runs
 //     whole streams, sharing K and V in its L2.
@@ -62,14 +63,15 @@ namespace ipus {
 namespace {
 
 constexpr int kThreads = 256;
-// Fast-kernel shape for tile width D: 16-query tiles per wave and keys per
-// block.  Up to 128 columns a wave owns two query tiles (32 queries) and a
-// block is 64 keys; at 256 columns one tile and 32 keys keep the registers
-// (output accumulators, Q fragments) within two waves per SIMD and the two
-// LDS stages within two workgroups per CU.
-template <int D>
+// Fast-kernel shape for tile width D and QT 16-query tiles per wave: keys per
+// block.  Up to 128 columns a wave owns one or two query tiles (16 or 32
+// queries) and a block is 64 keys; at 256 columns one tile and 32 keys keep
+// the registers (output accumulators, Q fragments) within two waves per SIMD
+// and the two LDS stages within two workgroups per CU.
+template <int D, int QT>
 struct Fast {
-  static constexpr int kQT = D > 128 ? 1 : 2;           // 16-query tiles per wave
+  static_assert(QT == 1 || (QT == 2 && D <= 128), "two query tiles need 128 columns or fewer");
+  static constexpr int kQT = QT;                        // 16-query tiles per wave
   static constexpr int kKeys = D > 128 ? 32 : 64;       // keys per block
   static constexpr int kQueriesPerWave = 16 * kQT;
   static constexpr int kQueriesPerBlock = 4 * kQueriesPerWave;  // per workgroup
@@ -77,7 +79,6 @@ struct Fast {
   static constexpr int kHalves = kKeys / 32;            // 32-key output contractions per block
 };
 constexpr int kMaxKeysPerBlock = 64;
-constexpr uint32_t kBlocksPerGroup = 2;  // query blocks per workgroup, run back to back
 constexpr float kLog2e = 1.4426950408889634f;
 // A block whose probabilities, taken against the current reference point,
 // sum to at most 2^8 per lane is accepted without moving the reference.
@@ -154,9 +155,9 @@ __device__ __forceinline__ uint32_t kv_offset(uint32_t row_bytes, uint32_t width
 }
 
 // Key blocks of query block qb: causal blocks stop at the block's last query.
-template <int D, bool Causal>
+template <int D, int QT, bool Causal>
 __device__ __forceinline__ uint32_t key_blocks(uint32_t qb, uint32_t query_rows, uint32_t key_rows) {
-  constexpr uint32_t kQPB = Fast<D>::kQueriesPerBlock, kKeys = Fast<D>::kKeys;
+  constexpr uint32_t kQPB = Fast<D, QT>::kQueriesPerBlock, kKeys = Fast<D, QT>::kKeys;
   uint32_t key_end = key_rows;
   if (Causal) {
     const uint32_t q0 = qb * kQPB;
@@ -170,18 +171,18 @@ __device__ __forceinline__ uint32_t key_blocks(uint32_t qb, uint32_t query_rows,
 // scores): tile qt, k step ks holds Q[query][32 ks + 8 (l / 16) .. +7] of
 // query qb * kQueriesPerBlock + wave * kQueriesPerWave + 16 qt + l % 16
 // (clamped to the last row; padding columns are 0).
-template <int D, int DC>
-__device__ __forceinline__ void load_q(half8_t (&qf)[Fast<D>::kQT][DC / 32], const uint16_t* __restrict__ query,
+template <int D, int QT, int DC>
+__device__ __forceinline__ void load_q(half8_t (&qf)[QT][DC / 32], const uint16_t* __restrict__ query,
                                        uint32_t stream, uint32_t qb, uint32_t query_rows,
                                        uint32_t width, uint32_t q_heads) {
   const uint32_t lane = threadIdx.x % kWave;
   const uint32_t r16 = lane % 16, g4 = lane / 16;
   const uint32_t wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint32_t wq0 = qb * Fast<D>::kQueriesPerBlock + wave_s * Fast<D>::kQueriesPerWave;
+  const uint32_t wq0 = qb * Fast<D, QT>::kQueriesPerBlock + wave_s * Fast<D, QT>::kQueriesPerWave;
   const uint32_t q_pitch = q_heads * width;
   const uint16_t* Q = query + (uint64_t)(stream / q_heads) * query_rows * q_pitch + (stream % q_heads) * width;
 #pragma unroll
-  for (uint32_t qt = 0; qt < Fast<D>::kQT; ++qt) {
+  for (uint32_t qt = 0; qt < QT; ++qt) {
     uint32_t q = wq0 + 16 * qt + r16;
     q = q < query_rows ? q : query_rows - 1;
 #pragma unroll
@@ -196,14 +197,14 @@ __device__ __forceinline__ void load_q(half8_t (&qf)[Fast<D>::kQT][DC / 32], con
 // D / DC: K tile width and score columns (query/key width); DV / DVC: V
 // tile width and output columns (value width).  The block shape (query
 // tiles per wave, keys per block) follows the wider tile.
-template <int D, int DC, int DV, int DVC, bool Causal, bool OutF16>
+template <int D, int DC, int DV, int DVC, int QT, bool Causal, bool OutF16>
 __device__ __forceinline__ void attention_block(
     void* __restrict__ out, const uint16_t* __restrict__ query, const uint16_t* __restrict__ key,
     const uint16_t* __restrict__ value, uint32_t stream, uint32_t qb, uint32_t query_rows,
     uint32_t key_rows, uint32_t width, uint32_t value_width, float scale_log2, uint32_t q_heads,
-    uint32_t k_heads, uint32_t v_heads, half8_t (&qf)[Fast<(D > DV ? D : DV)>::kQT][DC / 32],
+    uint32_t k_heads, uint32_t v_heads, half8_t (&qf)[QT][DC / 32],
     bool k0_loaded, bool chain, uint32_t next_qb) {
-  using F = Fast<(D > DV ? D : DV)>;
+  using F = Fast<(D > DV ? D : DV), QT>;
   constexpr int kQT = F::kQT, kKT = F::kKT, kHalves = F::kHalves;
   constexpr uint32_t kKeys = F::kKeys;
   constexpr uint32_t kQPW = F::kQueriesPerWave, kQPB = F::kQueriesPerBlock;
@@ -250,7 +251,7 @@ __device__ __forceinline__ void attention_block(
   const uint32_t v_voff = kv_offset<DV, false>(v_row_bytes, value_width);
   static_assert(kVDmaRows % 8 == 0, "the V swizzle depends on row bits 0-2 only");
 
-  const uint32_t nblocks = key_blocks<(D > DV ? D : DV), Causal>(qb, query_rows, key_rows);
+  const uint32_t nblocks = key_blocks<(D > DV ? D : DV), QT, Causal>(qb, query_rows, key_rows);
   const uint32_t k_block_bytes = kKeys * k_row_bytes;
   const uint32_t v_block_bytes = kKeys * v_row_bytes;
   // Blocks this wave computes scores for (causal: keys <= its last query).
@@ -534,7 +535,7 @@ __device__ __forceinline__ void attention_block(
   if (kbi < nblocks) step(lds_k0, lds_v1, lds_k1, lds_v0, kbi);
   // V of the last block (and every DMA) has landed after this barrier.
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-  if (chain) load_q<(D > DV ? D : DV), DC>(qf, query, stream, next_qb, query_rows, width, q_heads);
+  if (chain) load_q<(D > DV ? D : DV), QT, DC>(qf, query, stream, next_qb, query_rows, width, q_heads);
   if (nproc == nblocks) pv_only((nblocks - 1) % 2 == 0 ? lds_v0 : lds_v1);
 
   // o[dt][qt][e] = O^T[d = 16 dt + 4 (l / 16) + e][qi[qt]], unnormalised.
@@ -604,38 +605,42 @@ __device__ __forceinline__ void attention_block(
   }
 }
 
-// One workgroup per pair of query blocks of one stream: 2 i and 2 i + 1
-// (non-causal), or n - 1 - i and i (causal: the pair's key steps add up to
-// the same count for every workgroup).  When the first block's key block
+// One workgroup per `group` (1 or 2, fast_plan) query blocks of one stream: i
+// (causal: n - 1 - i, the heaviest first), or 2 i and 2 i + 1 (non-causal),
+// or n - 1 - i and i (causal: the pair's key steps add up to the same count
+// for every workgroup).  When the first block's key block
 // count is even, its last step fetches the second block's first K tile and
 // its epilogue the second block's Q fragments, so the second block starts
 // without a load latency (and without the burst of loads that workgroups
 // starting together would issue).  Workgroups are remapped so each XCD
 // (round-robin dispatch over 8) runs whole streams, sharing K and V in its L2.
-template <int D, int DC, int DV, int DVC, bool Causal, bool OutF16>
+template <int D, int DC, int DV, int DVC, int QT, bool Causal, bool OutF16>
 __global__ __launch_bounds__(kThreads, 2) void attention_fwd_kernel(
     void* __restrict__ out, const uint16_t* __restrict__ query, const uint16_t* __restrict__ key,
     const uint16_t* __restrict__ value, uint32_t streams, uint32_t query_rows, uint32_t key_rows,
     uint32_t width, uint32_t value_width, float scale_log2, uint32_t q_heads, uint32_t k_heads,
-    uint32_t v_heads) {
+    uint32_t v_heads, uint32_t group) {
   constexpr int W = D > DV ? D : DV;
-  constexpr uint32_t kQPB = Fast<W>::kQueriesPerBlock;
+  constexpr uint32_t kQPB = Fast<W, QT>::kQueriesPerBlock;
   const uint32_t qblocks = (query_rows + kQPB - 1) / kQPB;
-  const uint32_t per_stream = (qblocks + kBlocksPerGroup - 1) / kBlocksPerGroup;
+  const uint32_t per_stream = (qblocks + group - 1) / group;
   const uint32_t total = per_stream * streams;
   uint32_t pid = blockIdx.x;
   if (total % 8 == 0) pid = (pid % 8) * (total / 8) + pid / 8;  // XCD-contiguous
   const uint32_t stream = pid / per_stream, i = pid % per_stream;
   // Block order within a stream: causal n - 1, 0, n - 2, 1, ... (the heavy
-  // block, then its mirror: each pair has the same key steps), otherwise
-  // 0, 1, 2, ...; this workgroup runs the pair at positions 2 i, 2 i + 1.
+  // block, then its mirror: each pair has the same key steps) in pairs, n - 1,
+  // n - 2, ... in singles, otherwise 0, 1, 2, ...; this workgroup runs the
+  // blocks at positions group * i on.
   auto qb_at = [&](uint32_t pos) {
-    return Causal ? (pos % 2 == 0 ? qblocks - 1 - pos / 2 : pos / 2) : pos;
+    if (!Causal) return pos;
+    if (group == 1) return qblocks - 1 - pos;
+    return pos % 2 == 0 ? qblocks - 1 - pos / 2 : pos / 2;
   };
-  const uint32_t pos0 = i * kBlocksPerGroup;
-  const uint32_t reps = qblocks - pos0 < kBlocksPerGroup ? qblocks - pos0 : kBlocksPerGroup;
-  half8_t qf[Fast<W>::kQT][DC / 32];
-  load_q<W, DC>(qf, query, stream, qb_at(pos0), query_rows, width, q_heads);
+  const uint32_t pos0 = i * group;
+  const uint32_t reps = qblocks - pos0 < group ? qblocks - pos0 : group;
+  half8_t qf[QT][DC / 32];
+  load_q<W, QT, DC>(qf, query, stream, qb_at(pos0), query_rows, width, q_heads);
   bool loaded = false;  // this block's first K tile and Q fragments were fetched by the last one
   for (uint32_t rep = 0; rep < reps; ++rep) {
     // Every wave is done with the LDS stages before the next block's DMA.
@@ -643,9 +648,9 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd_kernel(
     const uint32_t qb = qb_at(pos0 + rep);
     // A block with an even key block count ends in stage 1, so its last
     // step can fetch the next block's first K tile into stage 0.
-    const bool chain = rep + 1 < reps && key_blocks<W, Causal>(qb, query_rows, key_rows) % 2 == 0;
-    if (rep > 0 && !loaded) load_q<W, DC>(qf, query, stream, qb, query_rows, width, q_heads);
-    attention_block<D, DC, DV, DVC, Causal, OutF16>(out, query, key, value, stream, qb, query_rows,
+    const bool chain = rep + 1 < reps && key_blocks<W, QT, Causal>(qb, query_rows, key_rows) % 2 == 0;
+    if (rep > 0 && !loaded) load_q<W, QT, DC>(qf, query, stream, qb, query_rows, width, q_heads);
+    attention_block<D, DC, DV, DVC, QT, Causal, OutF16>(out, query, key, value, stream, qb, query_rows,
                                                     key_rows, width, value_width, scale_log2, q_heads,
                                                     k_heads, v_heads, qf, loaded, chain,
                                                     qb_at(pos0 + rep + 1));
@@ -924,29 +929,71 @@ __global__ __launch_bounds__(64) void attention_general_kernel(
   }
 }
 
-template <int D, int DC, int DV, int DVC, bool Causal, bool OutF16>
-int launch_fast(hipStream_t stream, const AttentionArgs& a, float scale_log2) {
-  constexpr uint32_t kQPB = Fast<(D > DV ? D : DV)>::kQueriesPerBlock;
+template <int D, int DC, int DV, int DVC, int QT, bool Causal, bool OutF16>
+int launch_fast(hipStream_t stream, const AttentionArgs& a, float scale_log2, uint32_t group) {
+  constexpr uint32_t kQPB = Fast<(D > DV ? D : DV), QT>::kQueriesPerBlock;
   const uint32_t qblocks = (a.query_rows + kQPB - 1) / kQPB;
-  const uint64_t blocks = (uint64_t)((qblocks + kBlocksPerGroup - 1) / kBlocksPerGroup) * a.streams;
+  const uint64_t blocks = (uint64_t)((qblocks + group - 1) / group) * a.streams;
   if (blocks > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
-  hipLaunchKernelGGL((attention_fwd_kernel<D, DC, DV, DVC, Causal, OutF16>), dim3((uint32_t)blocks),
+  hipLaunchKernelGGL((attention_fwd_kernel<D, DC, DV, DVC, QT, Causal, OutF16>), dim3((uint32_t)blocks),
                      dim3(kThreads), 0, stream, a.out, (const uint16_t*)a.query,
                      (const uint16_t*)a.key, (const uint16_t*)a.value, a.streams, a.query_rows,
                      a.key_rows, a.width, a.value_width, scale_log2, a.heads[0], a.heads[1],
-                     a.heads[2]);
+                     a.heads[2], group);
   return hip_status(hipGetLastError());
+}
+
+template <int D, int DC, int DV, int DVC, int QT>
+int dispatch_tiles(hipStream_t stream, const AttentionArgs& a, float scale_log2, uint32_t group) {
+  if (a.causal)
+    return a.output_f16 ? launch_fast<D, DC, DV, DVC, QT, true, true>(stream, a, scale_log2, group)
+                        : launch_fast<D, DC, DV, DVC, QT, true, false>(stream, a, scale_log2, group);
+  return a.output_f16 ? launch_fast<D, DC, DV, DVC, QT, false, true>(stream, a, scale_log2, group)
+                      : launch_fast<D, DC, DV, DVC, QT, false, false>(stream, a, scale_log2, group);
+}
+
+// Query tiles per wave and query blocks per workgroup.  Two 16-query tiles per
+// wave share every K and V fragment (half the LDS bytes per MFMA) and two
+// blocks per workgroup chain the second's first loads, but the chip holds 512
+// workgroups (two per CU) and a call with few streams or rows makes fewer:
+// then one block each, and one query tile per wave, make up to four times as
+// many.  Measured (us, two tiles / pairs, two tiles / singles, one tile /
+// pairs, one tile / singles):
+//   non-causal 16 x 729 x 72  26.3  14.4  17.5   9.9   (96 two-tile singles)
+//              64 x 729 x 72  26.7  20.9  22.8  21.8   (384)
+//             16 x 2048 x 128 67.1  37.3  44.3  38.1   (256)
+//            128 x 2048 x 128 246   244   293   295    (2048)
+//   causal    16 x 2048 x 128 42.1  36.3  27.7  31.4   (128 two-tile pairs)
+//             16 x 1024 x 128 26.5  21.2  17.9  14.7   (64)
+//             32 x 2048 x 128 44.1  52.7  43.3  51.6   (256)
+//              64 x 512 x 64  14.4  10.3   9.6   8.8   (128)
+// Causal singles leave the heavy blocks to the end of the launch, so pairs
+// stay while they fill half the chip.
+struct FastPlan {
+  int tiles;
+  uint32_t group;
+};
+inline FastPlan fast_plan(const AttentionArgs& a, bool one_tile_only) {
+  const uint64_t q64 = (a.query_rows + 63) / 64, q128 = (a.query_rows + 127) / 128;
+  const uint64_t pairs1 = (q64 + 1) / 2 * a.streams, pairs2 = (q128 + 1) / 2 * a.streams;
+  const bool two = !one_tile_only && q128 < q64;
+  if (a.causal) {
+    if (two && pairs2 >= 256) return {2, 2};
+    return {1, pairs1 >= 256 ? 2u : 1u};
+  }
+  if (two && q128 * a.streams >= 256) return {2, pairs2 >= 512 ? 2u : 1u};
+  return {1, pairs1 >= 512 ? 2u : 1u};
 }
 
 // Tile widths D / DV (LDS rows, DMA) and computed columns DC / DVC (score
 // k steps / output tiles) of the query-key and value widths.
 template <int D, int DC, int DV = D, int DVC = DC>
 int dispatch_fast(hipStream_t stream, const AttentionArgs& a, float scale_log2) {
-  if (a.causal)
-    return a.output_f16 ? launch_fast<D, DC, DV, DVC, true, true>(stream, a, scale_log2)
-                        : launch_fast<D, DC, DV, DVC, true, false>(stream, a, scale_log2);
-  return a.output_f16 ? launch_fast<D, DC, DV, DVC, false, true>(stream, a, scale_log2)
-                      : launch_fast<D, DC, DV, DVC, false, false>(stream, a, scale_log2);
+  constexpr bool kOne = (D > DV ? D : DV) > 128;
+  const FastPlan plan = fast_plan(a, kOne);
+  if constexpr (!kOne)
+    if (plan.tiles == 2) return dispatch_tiles<D, DC, DV, DVC, 2>(stream, a, scale_log2, plan.group);
+  return dispatch_tiles<D, DC, DV, DVC, 1>(stream, a, scale_log2, plan.group);
 }
 
 }  // namespace
