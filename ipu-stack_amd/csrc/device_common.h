@@ -57,6 +57,48 @@ __device__ __forceinline__ void store16(void* p, u32x4 v) {
   *reinterpret_cast<u32x4*>(p) = v;
 }
 
+// Device-coherent accesses, for partial results that one workgroup leaves for
+// another of the same launch on any XCD: written through and read past the
+// XCD's own L2 (agent-scope atomics without an order).  A plain store published
+// by __threadfence() instead writes back the whole L2 once per wave (about 0.1
+// us per workgroup, one after the other: 64 streams x 4096 keys in 8 splits 64
+// us against 25).  The order comes from arrive(): every store of the
+// workgroup is acknowledged by the device before its count, and the loads are
+// issued after the count of the last one has returned.
+__device__ __forceinline__ void store_device(float* p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float load_device(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_device4(float* p, float4_t v) {  // 8-byte aligned
+  const u32x4 w = __builtin_bit_cast(u32x4, v);
+  uint64_t* q = reinterpret_cast<uint64_t*>(p);
+  __hip_atomic_store(q, w[0] | (uint64_t)w[1] << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, w[2] | (uint64_t)w[3] << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float4_t load_device4(const float* p) {
+  const uint64_t* q = reinterpret_cast<const uint64_t*>(p);
+  const uint64_t a = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t b = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __builtin_bit_cast(float4_t, u32x4{(uint32_t)a, (uint32_t)(a >> 32), (uint32_t)b, (uint32_t)(b >> 32)});
+}
+// Counts this workgroup in after its store_device calls; true in every thread
+// of the last of `expected` workgroups, which also returns the counter to 0
+// for the next launch.  Called by all threads; `flag` is a word of LDS.
+__device__ __forceinline__ bool arrive(uint32_t* counter, uint32_t expected, uint32_t* flag) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have reached the device
+  __syncthreads();                                  // every wave's have
+  if (threadIdx.x == 0) {
+    const uint32_t before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (before + 1 == expected)
+      __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = before;
+  }
+  __syncthreads();
+  return *flag + 1 == expected;
+}
+
 // Wave-wide sum via cross-lane shuffles.
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -1499,7 +1499,9 @@ extern "C" int ipus_session_capture(ipus_session* s) {
   hipStream_t stream = s->ctx->stream;
   hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
+  s->ctx->capturing_session = true;
   const int status = launch_steps(s);
+  s->ctx->capturing_session = false;
   hipGraph_t graph = nullptr;
   e = hipStreamEndCapture(stream, &graph);  // always ends the capture
   if (status != 0) {

@@ -8,6 +8,7 @@
 
 #include "../../include/ipus.h"
 
+#include <atomic>
 #include <mutex>
 #include <unordered_map>
 
@@ -22,9 +23,25 @@ struct ipus_context {
   // inject_after more launches, the next one returns inject_status.
   uint32_t inject_after = 0;
   int inject_status = 0;
+  // Workspace of the kernels that split a reduction over workgroups
+  // (context_workspace): allocated with the context, not counted among the
+  // buffers above.
+  void* workspace = nullptr;
+  uint32_t* workspace_counters = nullptr;
+  // ipus_session_capture is recording this context's stream into a graph
+  // that will only be launched on it.
+  std::atomic<bool> capturing_session{false};
 };
 
 namespace ipus {
+
+struct Workspace;
+// The context's workspace, for a launch on its stream: launches there run one
+// after the other, whichever threads enqueue them, so they can share it.
+// Empty where the allocation failed, and while a caller records the stream
+// into a graph of its own (which it may launch on other streams, several at
+// once): the unsplit kernels run then.
+Workspace context_workspace(const ipus_context* ctx);
 
 // Records a formatted message as the thread's last error and returns `code`.
 int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));

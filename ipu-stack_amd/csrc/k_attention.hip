@@ -52,7 +52,9 @@
 //     workgroup has the same number of key steps); the first block's last step prefetches the second's first K
 //     tile and Q fragments;
 //     workgroups are remapped so each XCD (round-robin dispatch over 8) runs
-//     whole streams, sharing K and V in its L2.
+//     whole streams, sharing K and V in its L2;
+//   * few queries against many keys (decode): the keys are split over
+//     workgroups, and the last to finish merges their results (split_plan).
 #include "../../include/ipus.h"
 #include "device_common.h"
 #include "kernels.h"
@@ -194,16 +196,30 @@ __device__ __forceinline__ void load_q(half8_t (&qf)[QT][DC / 32], const uint16_
   }
 }
 
+// Split launches (non-causal, one query tile per wave, one query block per
+// workgroup): workgroup (x, z) takes the keys [z * chunk, (z + 1) * chunk) of
+// query block x and writes its unnormalised output rows (fp32), reference
+// points and row sums to the context's workspace; the last workgroup of a
+// query block to finish (a counter per block, returned to 0) merges the
+// `splits` partial results.  Every split holds at least one key.
+struct SplitKeys {
+  float* rows;         // [streams * query_rows][splits][value_width]
+  float* sums;         // [streams * query_rows][splits][2]: reference point, row sum
+  uint32_t* counters;  // one per query block of every stream, all 0 between launches
+  uint32_t splits, chunk;  // chunk: keys per split, a multiple of the key block
+};
+constexpr uint32_t kMaxSplits = 32;
+
 // D / DC: K tile width and score columns (query/key width); DV / DVC: V
 // tile width and output columns (value width).  The block shape (query
 // tiles per wave, keys per block) follows the wider tile.
-template <int D, int DC, int DV, int DVC, int QT, bool Causal, bool OutF16>
+template <int D, int DC, int DV, int DVC, int QT, bool Causal, bool OutF16, bool Split>
 __device__ __forceinline__ void attention_block(
     void* __restrict__ out, const uint16_t* __restrict__ query, const uint16_t* __restrict__ key,
     const uint16_t* __restrict__ value, uint32_t stream, uint32_t qb, uint32_t query_rows,
     uint32_t key_rows, uint32_t width, uint32_t value_width, float scale_log2, uint32_t q_heads,
     uint32_t k_heads, uint32_t v_heads, half8_t (&qf)[QT][DC / 32],
-    bool k0_loaded, bool chain, uint32_t next_qb) {
+    bool k0_loaded, bool chain, uint32_t next_qb, const SplitKeys& split) {
   using F = Fast<(D > DV ? D : DV), QT>;
   constexpr int kQT = F::kQT, kKT = F::kKT, kHalves = F::kHalves;
   constexpr uint32_t kKeys = F::kKeys;
@@ -241,6 +257,14 @@ __device__ __forceinline__ void attention_block(
   const uint16_t* K = key + (uint64_t)(stream / k_heads) * key_rows * k_heads * width + (stream % k_heads) * width;
   const uint16_t* V = value + (uint64_t)(stream / v_heads) * key_rows * v_heads * value_width +
                       (stream % v_heads) * value_width;
+  if constexpr (Split) {
+    static_assert(!Causal && QT == 1, "splits are non-causal, one query tile");
+    // From here on this split's keys are all there are.
+    const uint32_t first = blockIdx.y * split.chunk;
+    K += (uint64_t)first * k_heads * width;
+    V += (uint64_t)first * v_heads * value_width;
+    key_rows = key_rows - first < split.chunk ? key_rows - first : split.chunk;
+  }
   const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       (void*)K, 0, (int)((key_rows - 1) * k_row_bytes + width * 2u), kBufferFlags);
   const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -479,9 +503,13 @@ __device__ __forceinline__ void attention_block(
           for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[kt][qt][e]);
         mx = max_of_query(mx * scale_log2);
         const float m_new = mx > m_run[qt] ? mx : m_run[qt];
-        const float alpha = __builtin_amdgcn_exp2f(m_run[qt] - m_new);
+        // A split whose scores so far are all -inf (infinite operands) holds
+        // nothing yet: no NaN from (-inf) - (-inf), another split may hold the
+        // row's finite scores.
+        const float m_use = Split && m_new == -INFINITY ? 0.0f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_run[qt] - m_use);
         m_run[qt] = m_new;
-        neg_m[qt] = -m_new;
+        neg_m[qt] = -m_use;
         l_run[qt] *= alpha;
 #pragma unroll
         for (uint32_t dt = 0; dt < kDT; ++dt) o[dt][qt] *= alpha;
@@ -539,6 +567,80 @@ __device__ __forceinline__ void attention_block(
   if (nproc == nblocks) pv_only((nblocks - 1) % 2 == 0 ? lds_v0 : lds_v1);
 
   // o[dt][qt][e] = O^T[d = 16 dt + 4 (l / 16) + e][qi[qt]], unnormalised.
+  if constexpr (Split) {
+    const float l = sum_of_query(l_run[0]);
+    if (qi[0] < query_rows) {
+      const uint64_t part = ((uint64_t)stream * query_rows + qi[0]) * split.splits + blockIdx.y;
+      if (g4 == 0) {
+        store_device(split.sums + part * 2, m_run[0]);
+        store_device(split.sums + part * 2 + 1, l);
+      }
+#pragma unroll
+      for (uint32_t dt = 0; dt < kDT; ++dt) {
+        const uint32_t d = dt * 16 + 4 * g4;
+        if (d < value_width) store_device4(split.rows + part * value_width + d, o[dt][0]);
+      }
+    }
+    __shared__ uint32_t arrived;
+    uint32_t* counter = split.counters + (uint64_t)stream * ((query_rows + kQPB - 1) / kQPB) + qb;
+    if (!arrive(counter, split.splits, &arrived)) return;
+    const uint32_t nrows = query_rows - q0 < kQPB ? query_rows - q0 : kQPB;
+    // Weight of each split of each row, exp2(m - max m) / sum, in LDS: one
+    // thread loads each split's pair, one folds each row.
+    float* weight = reinterpret_cast<float*>(lds_k0);  // [row][kMaxSplits]
+    float* part_sum = reinterpret_cast<float*>(lds_k1);
+    static_assert(kQPB * kMaxSplits * 4 <= kTile, "the weights fit a K stage");
+    const uint32_t splits = split.splits;
+    const float* pairs = split.sums + ((uint64_t)stream * query_rows + q0) * splits * 2;
+    for (uint32_t i = threadIdx.x; i < nrows * splits; i += kThreads) {
+      const uint32_t at = i / splits * kMaxSplits + i % splits;
+      weight[at] = load_device(pairs + 2 * i);
+      part_sum[at] = load_device(pairs + 2 * i + 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < nrows) {
+      float* w = weight + threadIdx.x * kMaxSplits;
+      const float* l = part_sum + threadIdx.x * kMaxSplits;
+      float top = -INFINITY, sum = 0.0f;
+      for (uint32_t z = 0; z < splits; ++z) top = fmaxf(top, w[z]);
+      for (uint32_t z = 0; z < splits; ++z) {
+        w[z] = __builtin_amdgcn_exp2f(w[z] - top);
+        sum += w[z] * l[z];
+      }
+      const float inv = 1.0f / sum;
+      for (uint32_t z = 0; z < splits; ++z) w[z] *= inv;
+    }
+    __syncthreads();
+    const uint32_t quads = value_width / 4;
+    for (uint32_t i = threadIdx.x; i < nrows * quads; i += kThreads) {
+      const uint32_t r = i / quads, d = i % quads * 4;
+      const uint64_t row = (uint64_t)stream * query_rows + q0 + r;
+      const float* p = split.rows + row * splits * value_width + d;
+      const float* w = weight + r * kMaxSplits;
+      float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+      // Eight loads in flight (past the last split: the last one again, not added).
+      for (uint32_t z0 = 0; z0 < splits; z0 += 8) {
+        float4_t x[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) {
+          const uint32_t z = z0 + u < splits ? z0 + u : splits - 1;
+          x[u] = load_device4(p + (uint64_t)z * value_width);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+          if (z0 + u < splits) acc += x[u] * w[z0 + u];
+      }
+      if constexpr (OutF16) {
+        half4_t hv;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) hv[e] = (half_t)acc[e];
+        *reinterpret_cast<half4_t*>((uint16_t*)out + row * value_width + d) = hv;
+      } else {
+        *reinterpret_cast<float4_t*>((float*)out + row * value_width + d) = acc;
+      }
+    }
+    return;
+  }
   if constexpr (OutF16) {
 #pragma unroll
     for (int qt = 0; qt < kQT; ++qt) {
@@ -614,13 +716,15 @@ __device__ __forceinline__ void attention_block(
 // without a load latency (and without the burst of loads that workgroups
 // starting together would issue).  Workgroups are remapped so each XCD
 // (round-robin dispatch over 8) runs whole streams, sharing K and V in its L2.
-template <int D, int DC, int DV, int DVC, int QT, bool Causal, bool OutF16>
+template <int D, int DC, int DV, int DVC, int QT, bool Causal, bool OutF16, bool Split>
 __global__ __launch_bounds__(kThreads, 2) void attention_fwd_kernel(
     void* __restrict__ out, const uint16_t* __restrict__ query, const uint16_t* __restrict__ key,
     const uint16_t* __restrict__ value, uint32_t streams, uint32_t query_rows, uint32_t key_rows,
     uint32_t width, uint32_t value_width, float scale_log2, uint32_t q_heads, uint32_t k_heads,
-    uint32_t v_heads, uint32_t group) {
+    uint32_t v_heads, uint32_t group_arg, SplitKeys split) {
   constexpr int W = D > DV ? D : DV;
+  // Causal launches of two query tiles always take pairs (fast_plan).
+  const uint32_t group = Causal && QT == 2 ? 2 : group_arg;
   constexpr uint32_t kQPB = Fast<W, QT>::kQueriesPerBlock;
   const uint32_t qblocks = (query_rows + kQPB - 1) / kQPB;
   const uint32_t per_stream = (qblocks + group - 1) / group;
@@ -650,10 +754,10 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd_kernel(
     // step can fetch the next block's first K tile into stage 0.
     const bool chain = rep + 1 < reps && key_blocks<W, QT, Causal>(qb, query_rows, key_rows) % 2 == 0;
     if (rep > 0 && !loaded) load_q<W, QT, DC>(qf, query, stream, qb, query_rows, width, q_heads);
-    attention_block<D, DC, DV, DVC, QT, Causal, OutF16>(out, query, key, value, stream, qb, query_rows,
+    attention_block<D, DC, DV, DVC, QT, Causal, OutF16, Split>(out, query, key, value, stream, qb, query_rows,
                                                     key_rows, width, value_width, scale_log2, q_heads,
                                                     k_heads, v_heads, qf, loaded, chain,
-                                                    qb_at(pos0 + rep + 1));
+                                                    qb_at(pos0 + rep + 1), split);
     loaded = chain;
   }
 }
@@ -929,17 +1033,18 @@ __global__ __launch_bounds__(64) void attention_general_kernel(
   }
 }
 
-template <int D, int DC, int DV, int DVC, int QT, bool Causal, bool OutF16>
-int launch_fast(hipStream_t stream, const AttentionArgs& a, float scale_log2, uint32_t group) {
+template <int D, int DC, int DV, int DVC, int QT, bool Causal, bool OutF16, bool Split = false>
+int launch_fast(hipStream_t stream, const AttentionArgs& a, float scale_log2, uint32_t group,
+                const SplitKeys& split = {}) {
   constexpr uint32_t kQPB = Fast<(D > DV ? D : DV), QT>::kQueriesPerBlock;
   const uint32_t qblocks = (a.query_rows + kQPB - 1) / kQPB;
   const uint64_t blocks = (uint64_t)((qblocks + group - 1) / group) * a.streams;
   if (blocks > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
-  hipLaunchKernelGGL((attention_fwd_kernel<D, DC, DV, DVC, QT, Causal, OutF16>), dim3((uint32_t)blocks),
-                     dim3(kThreads), 0, stream, a.out, (const uint16_t*)a.query,
+  hipLaunchKernelGGL((attention_fwd_kernel<D, DC, DV, DVC, QT, Causal, OutF16, Split>),
+                     dim3((uint32_t)blocks, Split ? split.splits : 1), dim3(kThreads), 0, stream, a.out, (const uint16_t*)a.query,
                      (const uint16_t*)a.key, (const uint16_t*)a.value, a.streams, a.query_rows,
                      a.key_rows, a.width, a.value_width, scale_log2, a.heads[0], a.heads[1],
-                     a.heads[2], group);
+                     a.heads[2], group, split);
   return hip_status(hipGetLastError());
 }
 
@@ -985,12 +1090,57 @@ inline FastPlan fast_plan(const AttentionArgs& a, bool one_tile_only) {
   return {1, pairs1 >= 512 ? 2u : 1u};
 }
 
+// Key splits for a non-causal launch of at most 128 workgroups (decode: few
+// queries against a long cache), where each workgroup walks all key blocks one
+// after the other while the rest of the chip idles.  Modelled time, us, for
+// operands in HBM: a key block 1.2 (the latency of its loads; 0.8 up to 64
+// columns), the keys' and values' bytes at 5.5 TB/s at least, and for a split
+// launch 6 more for the partial results, the count and the merge, 0.5 per
+// split and 2.2 per MB of partial results (they go past L2).  Measured,
+// unsplit and at this choice, width 128, operands in HBM: 64 streams x 1 query x
+// 4096 keys 67.5 -> 28.9 us (8 splits 33.1), 128 x 1 x 4096 79.5 -> 50.2, 32 x 1 x
+// 8192 127 -> 29; in the caches 16 x 1 x 1024 12.4 -> 8.8, 16 x 64 x 4096 40.9 ->
+// 22.  Not worth it: 16 x 1 x 512 x 64 6.0 -> 7.1, 16 x 729 x 729 x 72 9.9 -> 19.7,
+// 256 x 1 x 2048 40.4 -> 41.3 (enough workgroups).
+inline bool split_plan(const AttentionArgs& a, uint32_t block_keys, SplitKeys* s) {
+  if (a.causal || !a.workspace.data) return false;
+  const uint64_t groups = (uint64_t)((a.query_rows + 63) / 64) * a.streams;
+  if (groups > 128 || groups > a.workspace.counter_count) return false;
+  const uint32_t blocks = (a.key_rows + block_keys - 1) / block_keys;
+  const double block_us = a.width <= 64 && a.value_width <= 64 ? 0.8 : 1.2;
+  const double memory_us = 2.0 * a.streams * a.key_rows * (a.width + a.value_width) / 5.5e6;
+  const uint64_t row_bytes = (uint64_t)a.streams * a.query_rows * (a.value_width + 2) * sizeof(float);
+  uint32_t best = 1;
+  double best_us = blocks * block_us;
+  for (uint32_t want = 2; want <= kMaxSplits && want * groups <= 512 && want * 2 <= blocks; ++want) {
+    const uint32_t per = (blocks + want - 1) / want, splits = (blocks + per - 1) / per;
+    if (row_bytes * splits > a.workspace.bytes) break;
+    const double walk_us = per * block_us > memory_us ? per * block_us : memory_us;
+    const double us = walk_us + 6.0 + 0.5 * splits + 2.2e-6 * (double)(row_bytes * splits);
+    if (splits >= 2 && us < best_us) {
+      best = splits;
+      best_us = us;
+      s->chunk = per * block_keys;
+    }
+  }
+  if (best < 2) return false;
+  s->splits = best;
+  s->rows = (float*)a.workspace.data;
+  s->sums = s->rows + (uint64_t)a.streams * a.query_rows * best * a.value_width;
+  s->counters = a.workspace.counters;
+  return true;
+}
+
 // Tile widths D / DV (LDS rows, DMA) and computed columns DC / DVC (score
 // k steps / output tiles) of the query-key and value widths.
 template <int D, int DC, int DV = D, int DVC = DC>
 int dispatch_fast(hipStream_t stream, const AttentionArgs& a, float scale_log2) {
   constexpr bool kOne = (D > DV ? D : DV) > 128;
   const FastPlan plan = fast_plan(a, kOne);
+  SplitKeys split;
+  if (plan.tiles == 1 && plan.group == 1 && split_plan(a, Fast<(D > DV ? D : DV), 1>::kKeys, &split))
+    return a.output_f16 ? launch_fast<D, DC, DV, DVC, 1, false, true, true>(stream, a, scale_log2, 1, split)
+                        : launch_fast<D, DC, DV, DVC, 1, false, false, true>(stream, a, scale_log2, 1, split);
   if constexpr (!kOne)
     if (plan.tiles == 2) return dispatch_tiles<D, DC, DV, DVC, 2>(stream, a, scale_log2, plan.group);
   return dispatch_tiles<D, DC, DV, DVC, 1>(stream, a, scale_log2, plan.group);

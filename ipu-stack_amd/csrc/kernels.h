@@ -9,6 +9,17 @@
 
 namespace ipus {
 
+// Device memory that launches on one stream share: partial results of kernels
+// that split a reduction over workgroups and merge it in the same launch.
+// Launches of one stream run one after the other, so each finds the counters
+// at 0 and leaves them so.  data = nullptr: none, the unsplit kernels run.
+struct Workspace {
+  void* data = nullptr;
+  uint64_t bytes = 0;
+  uint32_t* counters = nullptr;
+  uint32_t counter_count = 0;
+};
+
 struct GemmArgs {
   void* out;
   const void* left;
@@ -48,6 +59,7 @@ struct AttentionArgs {
   // Per operand (query, key, value): stream s is head s % h of matrix s / h
   // of a [streams / h, rows, h * width] tensor; 1 = contiguous streams.
   uint32_t heads[3] = {1, 1, 1};
+  Workspace workspace;
 };
 
 // Dense products (k_gemm_f16.hip, k_gemm_f32.hip).

@@ -45,6 +45,26 @@ int use_device(const ipus_context* ctx) {
   return e == hipSuccess ? 0 : hip_fail(e, "hipSetDevice");
 }
 
+// Partial results of one launch at most (a launch that would need more runs
+// unsplit), and a counter per group of workgroups that merges.
+constexpr size_t kWorkspaceBytes = 32u << 20;
+constexpr uint32_t kWorkspaceCounters = 16384;
+
+Workspace context_workspace(const ipus_context* ctx) {
+  Workspace w;
+  if (!ctx->workspace) return w;
+  if (!ctx->capturing_session.load(std::memory_order_relaxed)) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone)
+      return w;
+  }
+  w.data = ctx->workspace;
+  w.bytes = kWorkspaceBytes;
+  w.counters = ctx->workspace_counters;
+  w.counter_count = kWorkspaceCounters;
+  return w;
+}
+
 int check_launch(int status, const char* symbol) {
   if (status == 0) return 0;
   if (status <= IPUS_ERROR_HIP_BASE)
@@ -114,6 +134,21 @@ extern "C" int ipus_context_create(int device, ipus_context** out) {
     return fail(status, "device %d: looking up the split-K scratch array failed (%d)", device,
                 status);
   }
+  // The kernels' workspace, its counters at 0.  Without it (no memory left)
+  // every launch still runs, unsplit.
+  void* ws = nullptr;
+  if (hipMalloc(&ws, kWorkspaceBytes + kWorkspaceCounters * sizeof(uint32_t)) == hipSuccess) {
+    uint32_t* counters = (uint32_t*)((uint8_t*)ws + kWorkspaceBytes);
+    e = hipMemsetAsync(counters, 0, kWorkspaceCounters * sizeof(uint32_t), ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) {
+      ctx->workspace = ws;
+      ctx->workspace_counters = counters;
+    } else {
+      (void)hipFree(ws);
+    }
+  }
+  (void)hipGetLastError();
   *out = ctx;
   return 0;
 }
@@ -130,6 +165,10 @@ extern "C" int ipus_context_destroy(ipus_context* ctx) {
   // Buffers the caller did not free are released with the context.
   for (const auto& kv : ctx->live) {
     e = hipFree(kv.first);
+    if (e != hipSuccess && status == 0) status = hip_fail(e, "hipFree");
+  }
+  if (ctx->workspace) {
+    e = hipFree(ctx->workspace);
     if (e != hipSuccess && status == 0) status = hip_fail(e, "hipFree");
   }
   delete ctx;
@@ -413,6 +452,7 @@ int run_attention(ipus_context* c, void* o, const void* const* i, const uint32_t
   if (s[6] > 1 || s[7] > 1) return IPUS_ERROR_INVALID_ARGUMENT;
   if (heads)
     for (int k = 0; k < 3; ++k) a.heads[k] = heads[k];
+  a.workspace = context_workspace(c);
   return launch_attention_f16(c->stream, a);
 }
 
@@ -736,6 +776,7 @@ const std::vector<ShapeFamily>& shape_families() {
          a.scale = bits_to_float(f[5]);
          a.causal = false;
          a.output_f16 = false;
+         a.workspace = context_workspace(c);
          return launch_attention_f16(c->stream, a);
        }},
   };

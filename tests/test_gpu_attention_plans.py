@@ -65,3 +65,93 @@ def test_attention_plans(ipus, oracle, ctx, streams, heads, rows, keys, d, causa
         assert np.all(np.abs(got[s] - want) <= bound), s
     for x in bufs + [out]:
         x.free()
+
+
+SPLIT_SHAPES = [  # few queries, many keys: the keys are split over workgroups
+                (3, 1, 1, 1025, 128),     # a last split with a partial block
+                (16, 16, 5, 2048, 72), (2, 1, 64, 4000, 64),
+                (5, 1, 65, 3000, 96),     # a second query block of one row
+                (2, 2, 16, 1500, 256),    # 32-key blocks
+                (128, 16, 1, 1600, 32)]
+
+
+@pytest.mark.parametrize("streams,heads,rows,keys,d", SPLIT_SHAPES)
+@pytest.mark.parametrize("f16", [0, 1])
+def test_attention_key_splits(ipus, oracle, ctx, streams, heads, rows, keys, d, f16):
+    """Split launches against float64, and three in a row alike (the merge
+    leaves its counters as it found them)."""
+    q, k, v = (ipus.synth_f16(streams * n * d, 75, i, ipus.NORMAL, 1.0)
+               for i, n in ((1, rows), (2, keys), (3, keys)))
+    bufs = [ctx.upload(x) for x in (q, k, v)]
+    count = streams * rows * d
+    out = ctx.alloc(count * (2 if f16 else 4))
+    results = []
+    for _ in range(3):
+        ctx.memset(out, 0xFF)
+        ctx.launch("ipu_stack_flash_attention_heads_f16", out, bufs,
+                   [streams, rows, keys, d, d, 0, 0, f16, heads, heads, heads])
+        results.append(out.download(np.uint16))
+    assert np.array_equal(results[0], results[1]) and np.array_equal(results[0], results[2])
+    got = (oracle.f16_to_f32(results[0]) if f16 else results[0].view(np.float32))
+    got = got.reshape(streams, rows, d)
+
+    def stream(x, n, s):
+        x = oracle.f16_to_f32(x).astype(np.float64).reshape(streams // heads, n, heads, d)
+        return x[s // heads, :, s % heads, :]
+
+    for s in sorted({0, streams // 2, streams - 1}):
+        want, bound = attention64(stream(q, rows, s), stream(k, keys, s), stream(v, keys, s), 0)
+        if f16:
+            bound = bound + np.abs(want) * 2.0 ** -11 + 2.0 ** -24
+        assert np.all(np.abs(got[s] - want) <= bound), s
+    for x in bufs + [out]:
+        x.free()
+
+
+@pytest.mark.parametrize("dead", [64, 512, 1000])
+def test_attention_key_splits_with_minus_infinity_scores(ipus, oracle, ctx, dead):
+    """Keys whose scores are all -inf carry no weight, also where they fill a
+    split or its first blocks; a NaN key makes every output NaN."""
+    streams, rows, keys, d = 2, 3, 2048, 128
+    q, k, v = (ipus.synth_f16(streams * n * d, 76, i, ipus.NORMAL, 1.0).reshape(streams, n, d)
+               for i, n in ((1, rows), (2, keys), (3, keys)))
+    q[:, :, 0] = 0x3C00          # 1
+    k[:, :dead, 0] = 0xFC00      # -inf
+    args = [streams, rows, keys, d, d, 0, 0, 0]
+    bufs = [ctx.upload(x) for x in (q, k, v)]
+    out = ctx.alloc(streams * rows * d * 4)
+    ctx.launch("ipu_stack_flash_attention_online_f16", out, bufs, args)
+    got = out.download(np.float32).reshape(streams, rows, d)
+    qf, kf, vf = (oracle.f16_to_f32(x).astype(np.float64).reshape(x.shape) for x in (q, k, v))
+    for s in range(streams):
+        want, bound = attention64(qf[s], kf[s, dead:], vf[s, dead:], 0)
+        assert np.all(np.abs(got[s] - want) <= bound)
+    k[0, keys - 1, 5] = 0x7E00
+    ctx.write(bufs[1], k)
+    ctx.launch("ipu_stack_flash_attention_online_f16", out, bufs, args)
+    got = out.download(np.float32).reshape(streams, rows, d)
+    assert np.all(np.isnan(got[0])) and not np.any(np.isnan(got[1]))
+    for x in bufs + [out]:
+        x.free()
+
+
+def test_attention_key_splits_in_a_captured_session(ipus, ctx):
+    """A session's captured graph replays a split launch with the eager
+    result, with other launches on the stream in between."""
+    g = ipus.ComputeGraph()
+    q, k, v = (g.host_input(n, [4, r, 64]) for n, r in (("q", 2), ("k", 3000), ("v", 3000)))
+    g.set_outputs([g.flash_attention(q, k, v)])
+    pkg = ipus.build_package(g)
+    eager, replay = pkg.session(ctx), pkg.session(ctx)
+    replay.capture()
+    for seed in range(4):
+        for i, (name, r) in enumerate((("q", 2), ("k", 3000), ("v", 3000))):
+            x = ipus.synth_f16(4 * r * 64, 80 + seed, i, ipus.NORMAL, 1.0).reshape(4, r, 64)
+            eager.write(name, x)
+            replay.write(name, x)
+        replay.run()
+        eager.run()
+        replay.run()
+        assert np.array_equal(replay.read("output.0"), eager.read("output.0"))
+    eager.close()
+    replay.close()
