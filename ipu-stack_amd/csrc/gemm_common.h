@@ -1,5 +1,5 @@
-// Device helpers shared by the fp16 GEMM kernels (k_gemm_f16.hip,
-// k_gemm_f16_tile.hip): LDS DMA and the epilogues' arithmetic.
+// Device helpers shared by the GEMM kernels: LDS DMA, and the arithmetic of the
+// fp16 kernels' epilogues.
 #pragma once
 
 #include "device_common.h"

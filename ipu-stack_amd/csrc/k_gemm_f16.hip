@@ -58,7 +58,7 @@
 
 #include <mutex>
 
-#include "gemm_f16_common.h"
+#include "gemm_common.h"
 #include "kernels.h"
 
 namespace ipus {

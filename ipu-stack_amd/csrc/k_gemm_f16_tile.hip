@@ -31,7 +31,7 @@
 #include "../../include/ipus.h"
 
 #include "device_common.h"
-#include "gemm_f16_common.h"
+#include "gemm_common.h"
 #include "kernels.h"
 
 namespace ipus {

@@ -1,12 +1,14 @@
-// fp32 GEMM on gfx950 MFMA (v_mfma_f32_32x32x2_f32), fp32 accumulation and
-// output: replaces gemm_f32_64_amp (device/gemm_f32_64_amp.S:125-385), whose
-// init mode clears the output and accumulates in fp32 (gemm_f32_64_amp.S:40-56).
+// fp32 GEMM on gfx950 MFMA, fp32 accumulation and output: replaces
+// gemm_f32_64_amp (device/gemm_f32_64_amp.S:125-385), whose init mode clears the
+// output and accumulates in fp32 (gemm_f32_64_amp.S:40-56).
 //
-// One kernel for every shape (16-byte aligned operands whose contiguous
-// axes, and N, are multiples of 4 use 16-byte loads; the kEdge mode, used
-// off the 128 x 128 x 32 grid, zero-fills loads past M, N or K and stores
-// only rows < M and 4-column chunks < N; kScalar covers other shapes and
-// alignments with bounds-checked element loads and stores):
+// 16-byte aligned operands whose contiguous axes, and N, are multiples of 4
+// run the tile kernel (v_mfma_f32_16x16x4_f32, at the end of this file).  The
+// 128 x 128 kernel (v_mfma_f32_32x32x2_f32) runs the rest: other shapes and
+// alignments in its kScalar mode, with bounds-checked element loads and
+// stores, and operands past the tile kernel's 31-bit buffer ranges with
+// 16-byte loads (the kEdge mode, off the 128 x 128 x 32 grid, zero-fills loads
+// past M, N or K and stores only rows < M and 4-column chunks < N):
 //   * block tile 128 x 128 x 32, 4 waves in a 2 x 2 grid, each wave 64 x 64
 //     as 2 x 2 MFMA tiles;
 //   * each operand is staged in LDS in the layout it has in memory, so no
@@ -25,7 +27,10 @@
 //   * the MFMA computes C^T tiles so each lane holds 4 consecutive columns
 //     of C (one 16-byte store).
 #include "../../include/ipus.h"
-#include "device_common.h"
+
+#include <cmath>
+
+#include "gemm_common.h"
 #include "kernels.h"
 
 namespace ipus {
@@ -34,8 +39,6 @@ namespace {
 constexpr int kBM = 128, kBN = 128, kBK = 32;
 constexpr int kThreads = 256;
 constexpr int kTileBytes = kBK * kBM * 4;  // 16 KiB per operand tile
-
-inline int hip_status(hipError_t e) { return e == hipSuccess ? 0 : IPUS_ERROR_HIP_BASE - (int)e; }
 
 // Byte offset of element (k, x) in a [32 k][128 x] fp32 tile (k-major,
 // the layout of an operand whose x axis is contiguous in memory).
@@ -247,6 +250,304 @@ int launch_fast(hipStream_t stream, const GemmArgs& a, bool chunked) {
   return hip_status(hipGetLastError());
 }
 
+// ---------------------------------------------------------------------------
+// Tile kernel: 64 x 64 or 32 x 32 tiles of C, for aligned operands (below).
+// Bound by the matrix pipes: a 64 x 64 x 32 step is 16 KiB of operands for
+// 1,024 cycles of MFMA, so what counts is that no wave waits.  Operand tiles go
+// global -> LDS by DMA, four stages deep, and the fragments of step k + 1 are
+// read between the MFMAs of step k, as in k_gemm_f16_tile.hip; 64 x 64 tiles
+// run two K groups of four waves (group h takes substeps 4 h .. 4 h + 3 of
+// the eight k that each lane holds) and two workgroups per CU, four waves per
+// SIMD in all.  Small tiles cost nothing here and fill the chip: 4096^3 1,066
+// -> 918 us (129 -> 150 TFLOP/s, 95% of 157.3; 128 x 128 tiles 945), 1024^3 75
+// -> 19.2 (64 tiles of 128 x 128 before), 64 x 1024 x 1024 75 -> 7.0 (32 x 32),
+// 256^3 21 -> 3.6.  Errors against float64 are those of the kernel before (one
+// fp32 sum over K per element: 5.7e-7 normwise at K = 1024) or, with two K
+// groups, lower (4.1e-7).
+// ---------------------------------------------------------------------------
+// Tile of C (TM x TN), part of one wave (WM x WN), K groups, k per step.
+template <int BM, int BN, int WM_, int WN_, int KG_, int BK_>
+struct TileShapeF32 {
+  static constexpr int TM = BM, TN = BN, WM = WM_, WN = WN_, KG = KG_, BK = BK_;
+  static constexpr int S = 4;  // LDS stages
+  static constexpr int kWavesM = TM / WM, kWavesN = TN / WN;
+  static constexpr int kWaves = kWavesM * kWavesN * KG;
+  static constexpr int kThreads = kWaves * 64;
+  static constexpr int kABytes = TM * BK * 4, kBBytes = TN * BK * 4;
+  static constexpr int kStageBytes = kABytes + kBBytes;
+  static constexpr int kDmaA = kABytes / 1024 / kWaves, kDmaB = kBBytes / 1024 / kWaves;
+  static constexpr int kDma = kDmaA + kDmaB;
+  static constexpr int kMT = WM / 16, kNT = WN / 16;
+  static constexpr int kUnits = BK / 32;  // 32-k units per step
+  static constexpr int kP = 8 / KG;       // MFMA substeps of a unit that a K group takes
+  static_assert(kABytes % (1024 * kWaves) == 0 && kBBytes % (1024 * kWaves) == 0, "whole DMA instructions per wave");
+  static_assert(KG == 1 || KG == 2, "the exchange of partial sums is between two groups");
+};
+
+typedef TileShapeF32<64, 64, 32, 32, 2, 32> TileF32x64;
+typedef TileShapeF32<32, 32, 16, 16, 1, 64> TileF32x32;
+
+// LDS tiles.  K-contiguous operand: units of 32 k, each [rows][32 k] (128-byte
+// rows), 16-byte chunk XORed by row & 7.  MN-contiguous: [k][mn], the chunk
+// XORed by mn_swz32(k): a fragment read takes 16 consecutive columns (64
+// bytes) of the four rows 8 g + p (g = 0..3), which the XOR by row bits 3 and 4
+// puts on different quarters of the banks (128-byte rows: on two halves).
+template <int RowBytes>
+__device__ __forceinline__ uint32_t mn_swz32(uint32_t k) {
+  return RowBytes >= 256 ? ((k >> 3) & 3u) << 2 : ((k >> 3) & 1u) << 2;
+}
+
+template <class T, bool TransposeLeft, bool TransposeRight, bool KTail>
+__global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
+    float* __restrict__ out, const float* __restrict__ left, const float* __restrict__ right,
+    uint32_t M, uint32_t N, uint32_t K, uint64_t left_batch_stride, uint64_t right_batch_stride) {
+  constexpr int TM = T::TM, TN = T::TN, BK = T::BK, S = T::S, KG = T::KG;
+  constexpr int kMT = T::kMT, kNT = T::kNT, kUnits = T::kUnits, kP = T::kP;
+  constexpr int kDmaA = T::kDmaA, kDmaB = T::kDmaB;
+  // Distinct LDS objects: a DMA into one stage never aliases the reads of
+  // another.
+  __shared__ __attribute__((aligned(1024))) uint8_t lds0[T::kStageBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds1[T::kStageBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds2[T::kStageBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds3[T::kStageBytes];
+  constexpr bool kAK = !TransposeLeft;   // A rows (m) K-contiguous
+  constexpr bool kBK_ = TransposeRight;  // B^T rows (n) K-contiguous
+
+  const uint32_t nbm = (M + TM - 1) / TM, nbn = (N + TN - 1) / TN;
+  const uint32_t tiles = nbm * nbn;
+  // XCD-contiguous tiles, grouped 8 along M.
+  const uint32_t xcd = blockIdx.x % 8, per = tiles / 8, rest = tiles % 8;
+  const uint32_t pid = xcd * per + (xcd < rest ? xcd : rest) + blockIdx.x / 8;
+  constexpr uint32_t kGroup = 8;
+  const uint32_t group = pid / (kGroup * nbn);
+  const uint32_t first_m = group * kGroup;
+  const uint32_t group_rows = (nbm - first_m) < kGroup ? (nbm - first_m) : kGroup;
+  const uint32_t in_group = pid % (kGroup * nbn);
+  const uint32_t bm = first_m + in_group % group_rows;
+  const uint32_t bn = in_group / group_rows;
+  const uint32_t m0 = bm * TM, n0 = bn * TN;
+
+  const uint64_t batch = blockIdx.y;
+  const float* A = left + batch * left_batch_stride;
+  const float* B = right + batch * right_batch_stride;
+  float* C = out + batch * (uint64_t)M * N;
+  const float* a_base = kAK ? A + (uint64_t)m0 * K : A + m0;
+  const float* b_base = kBK_ ? B + (uint64_t)n0 * K : B + n0;
+  const uint64_t a_bytes = (uint64_t)M * K * 4 - (uint64_t)(a_base - A) * 4;
+  const uint64_t b_bytes = (uint64_t)N * K * 4 - (uint64_t)(b_base - B) * 4;
+  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)a_base, 0, (int)(a_bytes > 0x7fffffffull ? 0x7fffffff : a_bytes), kBufferFlags);
+  const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)b_base, 0, (int)(b_bytes > 0x7fffffffull ? 0x7fffffff : b_bytes), kBufferFlags);
+
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t kg = wave % KG, wmn = wave / KG;
+  const uint32_t wm = (wmn / T::kWavesN) * T::WM, wn = (wmn % T::kWavesN) * T::WN;
+  const uint32_t r16 = lane % 16, g4 = lane / 16;
+
+  // MFMA substep p of a unit contracts k = 8 (l / 16) + p of both operands (a
+  // permutation of the unit's 32 k), so a lane's eight k are contiguous.
+  // Chunk (row or k row, logical k or mn offset in elements) that the lane
+  // fetches for DMA instruction `inst` of a tile.
+  auto chunk_of = [&]<bool KContig, int TMN>(uint32_t inst, uint32_t* row, uint32_t* col) __attribute__((always_inline)) {
+    if constexpr (KContig) {
+      const uint32_t sub = inst / (TMN / 8), r = (inst % (TMN / 8)) * 8 + lane / 8;
+      *row = r;
+      *col = sub * 32 + ((lane % 8) ^ (r & 7u)) * 4;
+    } else {
+      const uint32_t k = inst * (256 / TMN) + lane / (TMN / 4);
+      *row = k;
+      *col = ((lane % (TMN / 4)) ^ mn_swz32<4 * TMN>(k)) * 4;
+    }
+  };
+  uint32_t a_voff[kDmaA], b_voff[kDmaB];
+  auto offsets = [&]<bool KContig, int TMN, int N_>(uint32_t ld, uint32_t mn_limit, uint32_t (&voff)[N_]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < N_; ++j) {
+      uint32_t row, col;
+      chunk_of.template operator()<KContig, TMN>(wave * N_ + j, &row, &col);
+      voff[j] = KContig || col < mn_limit ? (row * ld + col) * 4 : kPadOffset;
+    }
+  };
+  offsets.template operator()<kAK, TM>(kAK ? K : M, M - m0, a_voff);
+  offsets.template operator()<kBK_, TN>(kBK_ ? K : N, N - n0, b_voff);
+  const uint32_t a_kstep = kAK ? BK * 4 : BK * M * 4;
+  const uint32_t b_kstep = kBK_ ? BK * 4 : BK * N * 4;
+
+  const uint32_t ksteps = (K + BK - 1) / BK;
+  const uint32_t k_tail = K % BK;
+  auto clamp = [&](uint32_t k) { return k < ksteps ? k : ksteps - 1; };
+  // The DMA of step k into a stage; past the last step the last one again (a
+  // stage that is never read), so the wait counts stay exact.  KTail: chunks
+  // and rows past K on the last step get an offset past the range and read 0.
+  auto dma = [&](uint8_t* stage, uint32_t k) __attribute__((always_inline)) {
+    const uint32_t limit = KTail && k == ksteps - 1 ? k_tail : 0u;
+    auto one = [&]<bool KContig, int TMN>(__amdgpu_buffer_rsrc_t rsrc, uint8_t* tile, uint32_t inst, uint32_t voff, uint32_t soff) __attribute__((always_inline)) {
+      if (KTail && limit != 0) {
+        uint32_t row, col;
+        chunk_of.template operator()<KContig, TMN>(inst, &row, &col);
+        voff = (KContig ? col : row) < limit ? voff : kPadOffset;
+      }
+      dma16(rsrc, tile + inst * 1024, voff, soff);
+    };
+#pragma unroll
+    for (int j = 0; j < kDmaA; ++j)
+      one.template operator()<kAK, TM>(a_rsrc, stage, wave * kDmaA + j, a_voff[j], k * a_kstep);
+#pragma unroll
+    for (int j = 0; j < kDmaB; ++j)
+      one.template operator()<kBK_, TN>(b_rsrc, stage + T::kABytes, wave * kDmaB + j, b_voff[j], k * b_kstep);
+  };
+  dma(lds0, 0);
+  dma(lds1, clamp(1));
+  dma(lds2, clamp(2));
+  dma(lds3, clamp(3));
+
+  const uint32_t h0 = KG == 2 ? kg : 0;
+  auto k_base = [&](uint32_t w0) { return (w0 + r16) * 128 + (((2 * g4 + h0) ^ (r16 & 7)) << 4); };
+  auto m_base = [&]<int RB>(uint32_t w0) {
+    return (8 * g4 + 4 * h0) * RB + (((w0 / 4 + r16 / 4) ^ mn_swz32<RB>(8 * g4)) << 4) + (r16 % 4) * 4;
+  };
+  const uint32_t a_base_l = kAK ? k_base(wm) : m_base.template operator()<4 * TM>(wm);
+  const uint32_t b_base_l = kBK_ ? k_base(wn) : m_base.template operator()<4 * TN>(wn);
+  // Four substeps (half h of the lane's 8 k of unit u) of tile t.
+  auto frag = [&]<bool KContig, int TMN>(const uint8_t* tile, uint32_t base, uint32_t t, uint32_t u, uint32_t h) __attribute__((always_inline)) {
+    if constexpr (KContig) {
+      return *reinterpret_cast<const float4_t*>(tile + (base ^ (h << 4)) + 2048 * t + u * (TMN * 128));
+    } else {
+      constexpr uint32_t RB = 4 * TMN;
+      const uint8_t* p = tile + (base ^ (t << 6)) + (u * 32 + 4 * h) * RB;
+      float4_t v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = *reinterpret_cast<const float*>(p + e * RB);
+      return v;
+    }
+  };
+  constexpr int kH = kP / 4;  // halves a wave reads
+  constexpr int kItems = (kMT + kNT) * kH * kUnits;
+  float4_t fa[2][kUnits][kH][kMT], fb[2][kUnits][kH][kNT];
+  auto read_item = [&](const uint8_t* stage, int buf, int r) __attribute__((always_inline)) {
+    const int u = r / ((kMT + kNT) * kH), q = r % ((kMT + kNT) * kH), h = q / (kMT + kNT), x = q % (kMT + kNT);
+    if (x < kNT) fb[buf][u][h][x] = frag.template operator()<kBK_, TN>(stage + T::kABytes, b_base_l, x, u, h);
+    else fa[buf][u][h][x - kNT] = frag.template operator()<kAK, TM>(stage, a_base_l, x - kNT, u, h);
+  };
+
+  float4_t acc[kMT][kNT];
+#pragma unroll
+  for (int i = 0; i < kMT; ++i)
+#pragma unroll
+    for (int j = 0; j < kNT; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+  constexpr int kDma = T::kDma;
+  constexpr int kMfma = kUnits * kP * kMT * kNT;
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * kDma) : "memory");
+#pragma unroll
+  for (int r = 0; r < kItems; ++r) read_item(lds0, 0, r);
+  // After the barrier every wave's DMA of stage kt + 1 has landed and every
+  // wave's reads of stage kt have returned.
+  auto step = [&](uint8_t* cur, const uint8_t* next, int buf, uint32_t kt) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * kDma) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    dma(cur, clamp(kt + S));
+    __builtin_amdgcn_sched_barrier(0);
+    int r = 0;
+#pragma unroll
+    for (int m = 0; m < kMfma; ++m) {
+      const int u = m / (kP * kMT * kNT), p = m / (kMT * kNT) % kP, i = m / kNT % kMT, j = m % kNT;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[buf][u][p / 4][j][p % 4], fa[buf][u][p / 4][i][p % 4], acc[i][j], 0, 0, 0);
+      while (r < kItems && r * kMfma * 3 / 4 <= m * kItems) {
+        read_item(next, 1 - buf, r);
+        ++r;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  uint32_t kt = 0;
+  for (; kt + 3 < ksteps; kt += 4) {
+    step(lds0, lds1, 0, kt);
+    step(lds1, lds2, 1, kt + 1);
+    step(lds2, lds3, 0, kt + 2);
+    step(lds3, lds0, 1, kt + 3);
+  }
+  if (kt < ksteps) step(lds0, lds1, 0, kt);
+  if (kt + 1 < ksteps) step(lds1, lds2, 1, kt + 1);
+  if (kt + 2 < ksteps) step(lds2, lds3, 0, kt + 2);
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  // acc[i][j][e] = C[m0 + wm + 16 i + lane % 16][n0 + wn + 16 j + 4 (lane / 16) + e]
+  constexpr int kRowsT = kMT / KG;
+  if constexpr (KG == 2) {
+    // Each group hands the other half of its rows over through LDS.
+    constexpr uint32_t kSlot = kRowsT * kNT * 1024;
+    uint8_t* mine = (kg == 0 ? lds0 : lds1) + wmn * kSlot;
+    const uint8_t* theirs = (kg == 0 ? lds1 : lds0) + wmn * kSlot;
+    static_assert(T::kWavesM * T::kWavesN * kSlot <= T::kStageBytes, "exchange fits a stage");
+#pragma unroll
+    for (int i = 0; i < kMT; ++i) {
+      if ((uint32_t)i / kRowsT == kg) continue;
+#pragma unroll
+      for (int j = 0; j < kNT; ++j)
+        *reinterpret_cast<float4_t*>(mine + ((i % kRowsT) * kNT + j) * 1024 + lane * 16) = acc[i][j];
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < kMT; ++i) {
+      if ((uint32_t)i / kRowsT != kg) continue;
+#pragma unroll
+      for (int j = 0; j < kNT; ++j)
+        acc[i][j] += *reinterpret_cast<const float4_t*>(theirs + ((i % kRowsT) * kNT + j) * 1024 + lane * 16);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kMT; ++i) {
+    if (KG > 1 && (uint32_t)i / kRowsT != kg) continue;
+    const uint32_t row = m0 + wm + 16 * i + r16;
+    if (row >= M) continue;
+    float* crow = C + (uint64_t)row * N;
+#pragma unroll
+    for (int j = 0; j < kNT; ++j) {
+      const uint32_t col = n0 + wn + 16 * j + 4 * g4;
+      if (col < N) *reinterpret_cast<float4_t*>(crow + col) = acc[i][j];
+    }
+  }
+}
+
+template <class T>
+int launch_tile32(hipStream_t stream, const GemmArgs& a) {
+  const uint64_t tiles = (uint64_t)((a.rows + T::TM - 1) / T::TM) * ((a.columns + T::TN - 1) / T::TN);
+  if (tiles > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, a.batches), dim3(T::kThreads), 0, stream,
+                       (float*)a.out, (const float*)a.left, (const float*)a.right, a.rows,
+                       a.columns, a.inner, a.left_batch_stride, a.right_batch_stride);
+  };
+  const bool tl = a.transpose_left, tr = a.transpose_right;
+  if (a.inner % T::BK == 0) {
+    if (!tl && !tr) go(gemm_f32_tile_kernel<T, false, false, false>);
+    else if (!tl) go(gemm_f32_tile_kernel<T, false, true, false>);
+    else if (!tr) go(gemm_f32_tile_kernel<T, true, false, false>);
+    else go(gemm_f32_tile_kernel<T, true, true, false>);
+  } else {
+    if (!tl && !tr) go(gemm_f32_tile_kernel<T, false, false, true>);
+    else if (!tl) go(gemm_f32_tile_kernel<T, false, true, true>);
+    else if (!tr) go(gemm_f32_tile_kernel<T, true, false, true>);
+    else go(gemm_f32_tile_kernel<T, true, true, true>);
+  }
+  return hip_status(hipGetLastError());
+}
+
+// Modelled time of the two tile sizes: start-up and time per 32-k step and
+// round of 256 tiles (us).  729 x 1152 x 1152: 64 x 64 20.9, 32 x 32 21.7; 512^3
+// 10.6 / 5.1; 1000 x 1004 x 1000 20.9 / 23.1.
+bool smaller_tiles(const GemmArgs& a) {
+  auto us = [&](uint32_t tile, double start, double step) {
+    const double tiles = (double)((a.rows + tile - 1) / tile) * ((a.columns + tile - 1) / tile) * a.batches;
+    return start + std::ceil(tiles / 256) * ((a.inner + 31) / 32) * step;
+  };
+  return us(32, 2.5, 0.15) < us(64, 3.0, 0.50);
+}
+
 }  // namespace
 
 int launch_gemm_f32(hipStream_t stream, const GemmArgs& a) {
@@ -262,6 +563,12 @@ int launch_gemm_f32(hipStream_t stream, const GemmArgs& a) {
   // Other shapes and alignments, and K = 0 (every load masked, zeros
   // stored): the same kernel with element loads and stores.
   const bool vec = aligned && chunked && a.inner > 0;
+  // The tile kernel addresses an operand tile through a buffer descriptor
+  // with 31-bit offsets.
+  const uint64_t a_span = (a.transpose_left ? (uint64_t)a.rows : 64ull) * a.inner * 4;
+  const uint64_t b_span = (a.transpose_right ? 64ull : (uint64_t)a.columns) * a.inner * 4;
+  if (vec && a_span < (1ull << 31) && b_span < (1ull << 31))
+    return smaller_tiles(a) ? launch_tile32<TileF32x32>(stream, a) : launch_tile32<TileF32x64>(stream, a);
   if (!a.transpose_left && !a.transpose_right) return launch_fast<false, false>(stream, a, vec);
   if (!a.transpose_left && a.transpose_right) return launch_fast<false, true>(stream, a, vec);
   if (a.transpose_left && !a.transpose_right) return launch_fast<true, false>(stream, a, vec);

@@ -77,3 +77,43 @@ def test_gemm_f16_tiles_batches_and_epilogues(ipus, oracle, ctx, M, N, K, shared
         ctx.launch("ipu_stack_add_f16", want, [out, d], [n, n, n])
         ctx.launch("ipu_stack_gemm_f16_accumulate", d, [da, db, d], sc + [M * N, N])  # in place
         assert np.array_equal(d.download(np.uint16), want.download(np.uint16))
+
+
+@pytest.mark.parametrize("M,N,K", [
+    # 64 x 64 tiles: partial tiles, a partial last step, one step
+    (1000, 1004, 1000), (520, 1160, 72), (1024, 1024, 32),
+    # 32 x 32 tiles
+    (8, 4, 4), (36, 68, 100), (32, 32, 64), (1, 4096, 260)])
+@pytest.mark.parametrize("tl,tr", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_f32_tiles(ipus, ctx, M, N, K, tl, tr):
+    """Every element within K + 2 fp32 roundings of the running magnitude."""
+    if tl and M % 4:
+        pytest.skip("a transposed left operand of odd rows runs the scalar kernel")
+    a = ipus.synth_f32(M * K, 77, 1, 0, 1.0)
+    b = ipus.synth_f32(K * N, 77, 2, 0, 1.0)
+    pad = np.full(64 * max(M, N, K), np.nan, np.float32)  # read past an operand: NaN
+    da, db = ctx.upload(np.concatenate([a, pad])), ctx.upload(np.concatenate([b, pad]))
+    out = ctx.upload(np.full(M * N + 4, 7.0, np.float32))
+    ctx.launch("ipu_stack_gemm_f32", out, [da, db], [1, M, N, K, tl, tr, 0, 0])
+    raw = out.download(np.float32)
+    assert np.all(raw[M * N:] == 7.0)
+    af = a.astype(np.float64).reshape((K, M) if tl else (M, K))
+    bf = b.astype(np.float64).reshape((N, K) if tr else (K, N))
+    af, bf = af.T if tl else af, bf.T if tr else bf
+    bound = np.abs(af) @ np.abs(bf) * (K + 2) * 2.0 ** -24 + 1e-30
+    assert np.all(np.abs(raw[:M * N].reshape(M, N) - af @ bf) <= bound)
+    for x in (da, db, out):
+        x.free()
+
+
+def test_gemm_f32_tiles_batched(ipus, ctx):
+    B, M, N, K = 3, 100, 132, 200
+    a, b = ipus.synth_f32(B * M * K, 78, 1, 0, 1.0), ipus.synth_f32(K * N, 78, 2, 0, 1.0)
+    da, db, out = ctx.upload(a), ctx.upload(b), ctx.alloc(B * M * N * 4)
+    ctx.launch("ipu_stack_gemm_f32", out, [da, db], [B, M, N, K, 0, 0, M * K, 0])
+    got = out.download(np.float32).reshape(B, M, N)
+    af, bf = a.astype(np.float64).reshape(B, M, K), b.astype(np.float64).reshape(K, N)
+    bound = np.abs(af) @ np.abs(bf) * (K + 2) * 2.0 ** -24
+    assert np.all(np.abs(got - af @ bf) <= bound)
+    for x in (da, db, out):
+        x.free()
