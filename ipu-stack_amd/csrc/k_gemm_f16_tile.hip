@@ -30,6 +30,8 @@
 // x 64 tiles (2048^3 33.0 against 27.7).
 #include "../../include/ipus.h"
 
+#include <cmath>
+
 #include "device_common.h"
 #include "gemm_common.h"
 #include "kernels.h"
@@ -377,7 +379,8 @@ uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t
   for (const Class& c : kClasses) {
     const uint64_t m = ((uint64_t)rows + c.tile - 1) / c.tile, n = ((uint64_t)columns + c.tile - 1) / c.tile;
     const double tiles = (double)m * (double)n * (double)batches;
-    const double rounds = tiles <= 256 ? 1.0 : c.tile >= 128 ? (double)(uint64_t)((tiles + 255) / 256) : tiles / 256;
+    // Two workgroups of the smaller tiles share a CU.
+    const double rounds = tiles <= 256 ? 1.0 : c.tile >= 128 ? std::ceil(tiles / 256) : 2.0 * std::ceil(tiles / 512);
     const double us = c.start_us + rounds * (double)steps * c.step_us;
     if (c.tile == 256 || us < best_us) {
       best = c.tile;
