@@ -6,7 +6,8 @@
 // (crates/ipu-tests/src/diagnostic.rs:533-654, 841-847).
 //
 // Fast kernel (16-byte aligned operands; N and K multiples of 8, and M too
-// when A is transposed; any M, N, K otherwise):
+// when A is transposed; or, kDwords, 4-byte aligned operands with even row
+// pitches; any M, N, K otherwise):
 //   * block tile 256 x 256 x 64, 256 threads = 4 waves in a 2 x 2 grid, each
 //     wave owns 128 x 128 of C as 8 x 8 tiles of v_mfma_f32_16x16x32_f16
 //     (64 accumulators of 4 fp32, in AGPRs); a K step is two 32-k substeps.
@@ -50,7 +51,8 @@
 //     the buffer's range and read as 0; MN-contiguous chunks past M or N,
 //     and (in the KTail instantiation, K % 64 != 0) K-contiguous chunks and
 //     MN-contiguous rows past K on the last step, get an offset past the
-//     range; the epilogue stores only rows < M and 8-column chunks < N.
+//     range; the epilogue stores only rows < M and 8-column chunks < N
+//     (kDwords: columns < N, see gemm_common.h).
 // Products with too few 256 x 256 tiles for the chip run smaller tiles
 // (k_gemm_f16_tile.hip, gemm_f16_tile).  Small-tile kernel below (64 x 64 or
 // 32 x 32 tiles): any shape or alignment the fast kernel does not take.
@@ -159,13 +161,14 @@ __device__ __forceinline__ void mfma16(float4_t& acc, half8_t a, half8_t b) {
 
 // out may be the addend itself (in place: every element is read and then
 // written by the same lane), but not an operand.
-template <bool TransposeLeft, bool TransposeRight, int Epi, bool KTail, bool Split>
+template <bool TransposeLeft, bool TransposeRight, int Epi, int E, bool Split>
 __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
     uint16_t* out, const uint16_t* __restrict__ left, const uint16_t* __restrict__ right,
     uint32_t M, uint32_t N, uint32_t K, uint64_t left_batch_stride, uint64_t right_batch_stride,
     uint32_t k_chunk, const uint16_t* addend, uint64_t addend_batch_stride,
     uint32_t addend_row_stride) {
   constexpr int BK = 64;
+  constexpr bool KTail = E != kWhole;
   constexpr int kTileBytes = Tile<BK>::kBytes;
   constexpr int kDma = Tile<BK>::kDmaPerWave;
   // The two stages are distinct LDS objects: the compiler can then see that
@@ -308,16 +311,28 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  // kDwords: the chunk that K ends in, of K-contiguous rows of the last step's
+  // stage, is cleared past K before it is read.
+  auto clear_past_k = [&](uint8_t* ta, uint8_t* tb) __attribute__((always_inline)) {
+    const uint32_t chunk = k_tail / 8, valid = k_tail % 8;
+    if (valid == 0) return;
+    if constexpr (kAK) clear_chunk_past(ta + kc_off<BK>(threadIdx.x, chunk), valid);
+    if constexpr (kBK_) clear_chunk_past(tb + kc_off<BK>(threadIdx.x, chunk), valid);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  static_assert(kBM == kThreads && kBN == kThreads, "one row per thread");
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  if (E == kDwords && ksteps == 1) clear_past_k(lds_a0, lds_b0);
 #pragma unroll
   for (int r = 0; r < 16; ++r) read_item(lds_a0, lds_b0, 0, 0, r);
-  auto step = [&](uint8_t* ta, uint8_t* tb, const uint8_t* na, const uint8_t* nb, uint32_t kt)
+  auto step = [&](uint8_t* ta, uint8_t* tb, uint8_t* na, uint8_t* nb, uint32_t kt)
       __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
     substep(0, ta, tb, 1, nullptr, nullptr, -1);
     // This wave's reads of (ta, tb) have returned and its DMA of step kt + 1
     // has landed; after the barrier, every wave's have.
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (E == kDwords && kt + 2 == ksteps) clear_past_k(na, nb);
     __builtin_amdgcn_sched_barrier(0);
     substep(1, na, nb, 0, ta, tb, (int64_t)clamp(kt + 2));
   };
@@ -382,17 +397,20 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const uint32_t v = (k0 + k) * kWave + lane, r = v / 16, c = v % 16;
-        d[k] = m0 + wm + r < M && n0 + wn + c * 8 < N
-                   ? *reinterpret_cast<const u32x4*>(aw + (uint64_t)r * addend_row_stride + c * 8)
-                   : u32x4{0, 0, 0, 0};
+        const uint16_t* p = aw + (uint64_t)r * addend_row_stride + c * 8;
+        d[k] = u32x4{0, 0, 0, 0};
+        if (m0 + wm + r < M && n0 + wn + c * 8 < N)
+          d[k] = E == kDwords ? load_elements(p, N - (n0 + wn + c * 8)) : *reinterpret_cast<const u32x4*>(p);
       }
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const uint32_t v = (k0 + k) * kWave + lane, r = v / 16, c = v % 16;
         const u32x4 x = *reinterpret_cast<const u32x4*>(cst + r * 256 + ((c ^ (r & 15)) << 4));
-        if (m0 + wm + r < M && n0 + wn + c * 8 < N)
-          __builtin_nontemporal_store(add_f16x8(x, d[k]),
-                                      reinterpret_cast<u32x4*>(cw + (uint64_t)r * N + c * 8));
+        if (m0 + wm + r < M && n0 + wn + c * 8 < N) {
+          uint16_t* p = cw + (uint64_t)r * N + c * 8;
+          if constexpr (E == kDwords) store_dwords(p, add_f16x8(x, d[k]), N - (n0 + wn + c * 8));
+          else __builtin_nontemporal_store(add_f16x8(x, d[k]), reinterpret_cast<u32x4*>(p));
+        }
       }
     }
     return;
@@ -408,15 +426,16 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
     // product cost the 8192^3 GEMMs 1.5%.
     if (m0 + wm + r < M && n0 + wn + c * 8 < N) {
       u32x4* p = reinterpret_cast<u32x4*>(cw + (uint64_t)r * N + c * 8);
-      if constexpr (Epi == kEpiGelu) *p = x;
+      if constexpr (E == kDwords) store_dwords(reinterpret_cast<uint16_t*>(p), x, N - (n0 + wn + c * 8));
+      else if constexpr (Epi == kEpiGelu) *p = x;
       else __builtin_nontemporal_store(x, p);
     }
   }
 }
 
 // Register-staged fp16 GEMM: 64 x 64 or 32 x 32 output tiles, for operands the
-// LDS-DMA kernels do not take (row pitches or addresses that are not 16-byte
-// multiples, operands past their 31-bit buffer ranges, K = 0).  256 threads = 4
+// LDS-DMA kernels do not take (odd row pitches, addresses that are not
+// 4-byte multiples, operands past their 31-bit buffer ranges, K = 0).  256 threads = 4
 // waves in a 2 x 2 grid, each (Tile / 2)^2 of C as tiles of
 // v_mfma_f32_16x16x32_f16 (C^T as in the 256 x 256 kernel, so a lane holds
 // 4 consecutive columns).  K runs in chunks of 256: a chunk's
@@ -428,8 +447,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
 // MN-contiguous tiles [64 k][64 mn] are read with ds_read_b64_tr_b16.
 // Chunks past M, N or K are not loaded and stay 0.  Vec = 8: N and K, and
 // M when A is transposed, are multiples of 8 and the operands 16-byte
-// aligned (operands past the 256 x 256 kernel's ranges).  Vec = 4 or 1 (any other shape or
-// alignment, where the 256 x 256 kernel cannot run): each 16-byte LDS chunk
+// aligned (operands past the LDS-DMA kernels' ranges).  Vec = 4 or 1: each 16-byte LDS chunk
 // is gathered from 8-byte or 2-byte loads, elements past M, N or K are 0,
 // and the epilogue stores element by element.
 constexpr uint32_t kSmallChunk = 256;
@@ -665,55 +683,62 @@ int launch_small_any(hipStream_t stream, const GemmArgs& a) {
 }
 
 template <bool TL, bool TR, int Epi, bool Split>
-int launch_fast(hipStream_t stream, const GemmArgs& a, uint32_t splits, uint32_t k_chunk) {
+int launch_fast(hipStream_t stream, const GemmArgs& a, uint32_t splits, uint32_t k_chunk, bool dwords) {
   const uint32_t tiles = ((a.rows + kBM - 1) / kBM) * ((a.columns + kBN - 1) / kBN);
   const dim3 grid(tiles, a.batches, splits);
-  if (a.inner % 64 == 0)
-    hipLaunchKernelGGL((gemm_f16_256_kernel<TL, TR, Epi, false, Split>), grid, dim3(kThreads), 0,
-                       stream, (uint16_t*)a.out, (const uint16_t*)a.left, (const uint16_t*)a.right,
-                       a.rows, a.columns, a.inner, a.left_batch_stride, a.right_batch_stride,
-                       k_chunk, (const uint16_t*)a.addend, a.addend_batch_stride,
-                       a.addend_row_stride);
-  else
-    hipLaunchKernelGGL((gemm_f16_256_kernel<TL, TR, Epi, true, Split>), grid, dim3(kThreads), 0,
-                       stream, (uint16_t*)a.out, (const uint16_t*)a.left, (const uint16_t*)a.right,
-                       a.rows, a.columns, a.inner, a.left_batch_stride, a.right_batch_stride,
-                       k_chunk, (const uint16_t*)a.addend, a.addend_batch_stride,
-                       a.addend_row_stride);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, (uint16_t*)a.out,
+                       (const uint16_t*)a.left, (const uint16_t*)a.right, a.rows, a.columns,
+                       a.inner, a.left_batch_stride, a.right_batch_stride, k_chunk,
+                       (const uint16_t*)a.addend, a.addend_batch_stride, a.addend_row_stride);
+  };
+  if constexpr (!Split)
+    if (dwords) {
+      go(gemm_f16_256_kernel<TL, TR, Epi, kDwords, false>);
+      return hip_status(hipGetLastError());
+    }
+  if (a.inner % 64 == 0) go(gemm_f16_256_kernel<TL, TR, Epi, kWhole, Split>);
+  else go(gemm_f16_256_kernel<TL, TR, Epi, kKTail, Split>);
   return hip_status(hipGetLastError());
 }
 
 template <int Epi, bool Split>
-int dispatch_fast(hipStream_t stream, const GemmArgs& a, uint32_t splits, uint32_t k_chunk) {
+int dispatch_fast(hipStream_t stream, const GemmArgs& a, uint32_t splits, uint32_t k_chunk,
+                  bool dwords = false) {
   if (!a.transpose_left && !a.transpose_right)
-    return launch_fast<false, false, Epi, Split>(stream, a, splits, k_chunk);
+    return launch_fast<false, false, Epi, Split>(stream, a, splits, k_chunk, dwords);
   if (!a.transpose_left && a.transpose_right)
-    return launch_fast<false, true, Epi, Split>(stream, a, splits, k_chunk);
+    return launch_fast<false, true, Epi, Split>(stream, a, splits, k_chunk, dwords);
   if (a.transpose_left && !a.transpose_right)
-    return launch_fast<true, false, Epi, Split>(stream, a, splits, k_chunk);
-  return launch_fast<true, true, Epi, Split>(stream, a, splits, k_chunk);
+    return launch_fast<true, false, Epi, Split>(stream, a, splits, k_chunk, dwords);
+  return launch_fast<true, true, Epi, Split>(stream, a, splits, k_chunk, dwords);
 }
 
 int epilogue_of(const GemmArgs& a) {
   return a.addend ? kEpiAdd : a.gelu ? kEpiGelu : kEpiPlain;
 }
 
-// Conditions of the 256 x 256 kernel: 16-byte aligned operands, 32-bit
-// per-block buffer offsets, 16-byte chunks (N and K, and M when A is
-// transposed, multiples of 8).
-bool fast_ok(const GemmArgs& a) {
-  const bool aligned = ((uintptr_t)a.left % 16 == 0) && ((uintptr_t)a.right % 16 == 0) &&
-                       ((uintptr_t)a.out % 16 == 0) && a.left_batch_stride % 8 == 0 &&
-                       a.right_batch_stride % 8 == 0;
+// Conditions of the LDS-DMA kernels: `unit` 8 for 16-byte aligned operands and
+// rows (N and K, and M when A is transposed, multiples of 8), 2 for dword
+// aligned ones (every row pitch even, any other extent), and 32-bit
+// per-block buffer offsets.
+bool dma_ok(const GemmArgs& a, uint32_t unit) {
+  auto at = [&](const void* p) { return (uintptr_t)p % (2 * unit) == 0; };
+  const bool aligned = at(a.left) && at(a.right) && at(a.out) && a.left_batch_stride % unit == 0 &&
+                       a.right_batch_stride % unit == 0;
   const uint64_t a_span = a.transpose_left ? (uint64_t)a.inner * a.rows * 2 : 256ull * a.inner * 2;
   const uint64_t b_span = a.transpose_right ? 256ull * a.inner * 2 : (uint64_t)a.inner * a.columns * 2;
   const bool fits = a_span < (1ull << 31) && b_span < (1ull << 31);
-  const bool chunked = a.inner % 8 == 0 && a.columns % 8 == 0 && (!a.transpose_left || a.rows % 8 == 0);
-  // The add epilogue loads the addend as 16-byte chunks of 8 columns.
-  const bool addend_ok = !a.addend || ((uintptr_t)a.addend % 16 == 0 &&
-                                       a.addend_batch_stride % 8 == 0 && a.addend_row_stride % 8 == 0);
+  const uint32_t lda = a.transpose_left ? a.rows : a.inner, ldb = a.transpose_right ? a.inner : a.columns;
+  const bool chunked = unit == 8 ? a.inner % 8 == 0 && a.columns % 8 == 0 && (!a.transpose_left || a.rows % 8 == 0)
+                                 : lda % 2 == 0 && ldb % 2 == 0 && a.columns % 2 == 0;
+  // With 16-byte chunks the add epilogue loads the addend as chunks of 8
+  // columns, otherwise by element.
+  const bool addend_ok = unit != 8 || !a.addend || ((uintptr_t)a.addend % 16 == 0 &&
+                                                   a.addend_batch_stride % 8 == 0 && a.addend_row_stride % 8 == 0);
   return aligned && fits && chunked && addend_ok && a.inner > 0;
 }
+bool fast_ok(const GemmArgs& a) { return dma_ok(a, 8); }
 
 // fp32 partials [splits][count] -> fp16 (optionally GELU of the fp16 value):
 // 8 elements per thread, splits summed in order.
@@ -794,15 +819,17 @@ int launch_reduce_splits_f16(hipStream_t stream, void* dst, const void* parts, u
 int launch_gemm_f16(hipStream_t stream, const GemmArgs& a) {
   if (a.batches == 0 || a.rows == 0 || a.columns == 0) return 0;
   if (a.batches > 65535 || (a.gelu && a.addend)) return IPUS_ERROR_INVALID_ARGUMENT;
-  // Any M and N on the fast kernel: rows past the edge read as 0 and are not
-  // stored.
-  if (fast_ok(a)) {
+  // The LDS-DMA kernels take any M and N: rows past the edge read as 0 and are
+  // not stored.  Dword-aligned pitches run them too (kDwords): 4096 x 4096 x
+  // 4100 358 -> 108 us against the register-staged kernel.
+  const bool chunks = fast_ok(a);
+  if (chunks || dma_ok(a, 2)) {
     const uint32_t tile = gemm_f16_tile(a.rows, a.columns, a.inner, a.batches);
-    if (tile != 256) return launch_gemm_f16_tile(stream, a, tile);
+    if (tile != 256) return launch_gemm_f16_tile(stream, a, tile, !chunks);
     switch (epilogue_of(a)) {
-      case kEpiGelu: return dispatch_fast<kEpiGelu, false>(stream, a, 1, a.inner);
-      case kEpiAdd: return dispatch_fast<kEpiAdd, false>(stream, a, 1, a.inner);
-      default: return dispatch_fast<kEpiPlain, false>(stream, a, 1, a.inner);
+      case kEpiGelu: return dispatch_fast<kEpiGelu, false>(stream, a, 1, a.inner, !chunks);
+      case kEpiAdd: return dispatch_fast<kEpiAdd, false>(stream, a, 1, a.inner, !chunks);
+      default: return dispatch_fast<kEpiPlain, false>(stream, a, 1, a.inner, !chunks);
     }
   }
   // Any other shape or alignment (or operands past the 256 x 256 kernel's

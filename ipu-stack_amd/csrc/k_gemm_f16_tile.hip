@@ -78,7 +78,7 @@ __device__ __forceinline__ uint32_t mn_swz(uint32_t k) {
     return ((k >> 3) & 1u) << 1;
 }
 
-template <class T, bool TransposeLeft, bool TransposeRight, int Epi, bool KTail>
+template <class T, bool TransposeLeft, bool TransposeRight, int Epi, int E>
 __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
     uint16_t* out, const uint16_t* __restrict__ left, const uint16_t* __restrict__ right,
     uint32_t M, uint32_t N, uint32_t K, uint64_t left_batch_stride, uint64_t right_batch_stride,
@@ -86,6 +86,7 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   constexpr int TM = T::TM, TN = T::TN, BK = T::BK, S = T::S, KG = T::KG;
   constexpr int kMT = T::kMT, kNT = T::kNT, kSub = T::kSub;
   constexpr int kDmaA = T::kDmaA, kDmaB = T::kDmaB;
+  constexpr bool KTail = E != kWhole;
   // Four stages, each a distinct LDS object: the compiler can then see that
   // a DMA into one never aliases the fragment reads of another.
   __shared__ __attribute__((aligned(1024))) uint8_t lds0[T::kStageBytes];
@@ -223,20 +224,36 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
 #pragma unroll
     for (int j = 0; j < kNT; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
+  // kDwords: K-contiguous rows of the last step's stage hold elements past K
+  // in the chunk that K ends in; cleared once every wave's DMA has landed.
+  auto clear_past_k = [&](uint8_t* stage) __attribute__((always_inline)) {
+    const uint32_t chunk = k_tail / 8, valid = k_tail % 8;
+    if (valid == 0) return;
+    auto rows = [&](uint8_t* tile, uint32_t count) {
+      for (uint32_t r = threadIdx.x; r < count; r += T::kThreads)
+        clear_chunk_past(tile + chunk / 8 * (count * 128) + r * 128 + (((chunk % 8) ^ (r & 7u)) << 4), valid);
+    };
+    if constexpr (kAK) rows(stage, TM);
+    if constexpr (kBK_) rows(stage + T::kABytes, TN);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+
   constexpr int kDma = T::kDma;
   constexpr int kMfma = kSub * kMT * kNT, kReads = kSub * kItems;
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * kDma) : "memory");
+  if (E == kDwords && ksteps == 1) clear_past_k(lds0);
 #pragma unroll
   for (int r = 0; r < kReads; ++r) read_item(lds0, 0, r);
   // Step kt: its fragments are in register buffer buf.  After the barrier
   // every wave's DMA of stage kt + 1 (`next`) has landed and every wave's
   // reads of stage kt (`cur`) have returned, so cur takes the DMA of step
   // kt + 4 and next is read between the MFMAs.
-  auto step = [&](uint8_t* cur, const uint8_t* next, int buf, uint32_t kt) __attribute__((always_inline)) {
+  auto step = [&](uint8_t* cur, uint8_t* next, int buf, uint32_t kt) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * kDma) : "memory");
     __builtin_amdgcn_sched_barrier(0);
     dma(cur, clamp(kt + S));
+    if (E == kDwords && kt + 2 == ksteps) clear_past_k(next);
     __builtin_amdgcn_sched_barrier(0);
     int r = 0;
 #pragma unroll
@@ -313,19 +330,24 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
     const uint32_t v = k * kWave + lane, r = v / kRC, c = v % kRC;
     if (v >= 16 * kRowsT * kRC) break;  // 32 x 32 tiles: half a wave's lanes store
     u32x4 x = *reinterpret_cast<const u32x4*>(cst + r * kRB + ((c ^ (r & (kRC - 1))) << 4));
-    // Rows past M and 8-column chunks past N (N % 8 == 0) are not stored.  out
-    // may be the addend: the same lane reads each chunk and then writes it.
+    // Rows past M and columns past N are not stored (N % 8 == 0 except with
+    // kDwords).  out may be the addend: the same lane reads each chunk and then
+    // writes it.
     if (row0 + r < M && col0 + c * 8 < N) {
-      if constexpr (Epi == kEpiAdd)
-        x = add_f16x8(x, *reinterpret_cast<const u32x4*>(addend + batch * addend_batch_stride +
-                                                         (uint64_t)(row0 + r) * addend_row_stride + col0 + c * 8));
-      *reinterpret_cast<u32x4*>(C + (uint64_t)(row0 + r) * N + col0 + c * 8) = x;
+      const uint64_t at = (uint64_t)(row0 + r) * N + col0 + c * 8;
+      const uint32_t valid = N - (col0 + c * 8);
+      if constexpr (Epi == kEpiAdd) {
+        const uint16_t* d = addend + batch * addend_batch_stride + (uint64_t)(row0 + r) * addend_row_stride + col0 + c * 8;
+        x = add_f16x8(x, E == kDwords ? load_elements(d, valid) : *reinterpret_cast<const u32x4*>(d));
+      }
+      if constexpr (E == kDwords) store_dwords(C + at, x, valid);
+      else *reinterpret_cast<u32x4*>(C + at) = x;
     }
   }
 }
 
 template <class T, int Epi>
-int launch_tile(hipStream_t stream, const GemmArgs& a) {
+int launch_tile(hipStream_t stream, const GemmArgs& a, bool dwords) {
   const uint64_t tiles = (uint64_t)((a.rows + T::TM - 1) / T::TM) * ((a.columns + T::TN - 1) / T::TN);
   if (tiles > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
   auto go = [&](auto kernel) {
@@ -335,25 +357,23 @@ int launch_tile(hipStream_t stream, const GemmArgs& a) {
                        (const uint16_t*)a.addend, a.addend_batch_stride, a.addend_row_stride);
   };
   const bool tl = a.transpose_left, tr = a.transpose_right;
-  if (a.inner % T::BK == 0) {
-    if (!tl && !tr) go(gemm_f16_tile_kernel<T, false, false, Epi, false>);
-    else if (!tl) go(gemm_f16_tile_kernel<T, false, true, Epi, false>);
-    else if (!tr) go(gemm_f16_tile_kernel<T, true, false, Epi, false>);
-    else go(gemm_f16_tile_kernel<T, true, true, Epi, false>);
-  } else {
-    if (!tl && !tr) go(gemm_f16_tile_kernel<T, false, false, Epi, true>);
-    else if (!tl) go(gemm_f16_tile_kernel<T, false, true, Epi, true>);
-    else if (!tr) go(gemm_f16_tile_kernel<T, true, false, Epi, true>);
-    else go(gemm_f16_tile_kernel<T, true, true, Epi, true>);
-  }
+  auto layouts = [&]<int E>() {
+    if (!tl && !tr) go(gemm_f16_tile_kernel<T, false, false, Epi, E>);
+    else if (!tl) go(gemm_f16_tile_kernel<T, false, true, Epi, E>);
+    else if (!tr) go(gemm_f16_tile_kernel<T, true, false, Epi, E>);
+    else go(gemm_f16_tile_kernel<T, true, true, Epi, E>);
+  };
+  if (dwords) layouts.template operator()<kDwords>();
+  else if (a.inner % T::BK == 0) layouts.template operator()<kWhole>();
+  else layouts.template operator()<kKTail>();
   return hip_status(hipGetLastError());
 }
 
 template <class T>
-int launch_epilogue(hipStream_t stream, const GemmArgs& a) {
-  if (a.addend) return launch_tile<T, kEpiAdd>(stream, a);
-  if (a.gelu) return launch_tile<T, kEpiGelu>(stream, a);
-  return launch_tile<T, kEpiPlain>(stream, a);
+int launch_epilogue(hipStream_t stream, const GemmArgs& a, bool dwords) {
+  if (a.addend) return launch_tile<T, kEpiAdd>(stream, a, dwords);
+  if (a.gelu) return launch_tile<T, kEpiGelu>(stream, a, dwords);
+  return launch_tile<T, kEpiPlain>(stream, a, dwords);
 }
 
 }  // namespace
@@ -390,10 +410,10 @@ uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t
   return best;
 }
 
-int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile) {
-  if (tile == 128) return launch_epilogue<Tile128>(stream, a);
-  if (tile == 64) return launch_epilogue<Tile64>(stream, a);
-  return launch_epilogue<Tile32>(stream, a);
+int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, bool dwords) {
+  if (tile == 128) return launch_epilogue<Tile128>(stream, a, dwords);
+  if (tile == 64) return launch_epilogue<Tile64>(stream, a, dwords);
+  return launch_epilogue<Tile32>(stream, a, dwords);
 }
 
 }  // namespace ipus
