@@ -2,13 +2,13 @@
 // gemm_f32_64_amp (device/gemm_f32_64_amp.S:125-385), whose init mode clears the
 // output and accumulates in fp32 (gemm_f32_64_amp.S:40-56).
 //
-// 16-byte aligned operands whose contiguous axes, and N, are multiples of 4
-// run the tile kernel (v_mfma_f32_16x16x4_f32, at the end of this file).  The
-// 128 x 128 kernel (v_mfma_f32_32x32x2_f32) runs the rest: other shapes and
-// alignments in its kScalar mode, with bounds-checked element loads and
-// stores, and operands past the tile kernel's 31-bit buffer ranges with
-// 16-byte loads (the kEdge mode, off the 128 x 128 x 32 grid, zero-fills loads
-// past M, N or K and stores only rows < M and 4-column chunks < N):
+// Every shape runs the tile kernel (v_mfma_f32_16x16x4_f32, at the end of this
+// file) except K = 0 and operands past its 31-bit buffer ranges.  Those run
+// the 128 x 128 kernel (v_mfma_f32_32x32x2_f32): 16-byte aligned operands whose
+// contiguous axes, and N, are multiples of 4 with 16-byte loads (the kEdge
+// mode, off the 128 x 128 x 32 grid, zero-fills loads past M, N or K and stores
+// only rows < M and 4-column chunks < N), others in its kScalar mode with
+// bounds-checked element loads and stores:
 //   * block tile 128 x 128 x 32, 4 waves in a 2 x 2 grid, each wave 64 x 64
 //     as 2 x 2 MFMA tiles;
 //   * each operand is staged in LDS in the layout it has in memory, so no
@@ -251,7 +251,7 @@ int launch_fast(hipStream_t stream, const GemmArgs& a, bool chunked) {
 }
 
 // ---------------------------------------------------------------------------
-// Tile kernel: 64 x 64 or 32 x 32 tiles of C, for aligned operands (below).
+// Tile kernel: 64 x 64 or 32 x 32 tiles of C.
 // Bound by the matrix pipes: a 64 x 64 x 32 step is 16 KiB of operands for
 // 1,024 cycles of MFMA, so what counts is that no wave waits.  Operand tiles go
 // global -> LDS by DMA, four stages deep, and the fragments of step k + 1 are
@@ -297,13 +297,14 @@ __device__ __forceinline__ uint32_t mn_swz32(uint32_t k) {
   return RowBytes >= 256 ? ((k >> 3) & 3u) << 2 : ((k >> 3) & 1u) << 2;
 }
 
-template <class T, bool TransposeLeft, bool TransposeRight, bool KTail>
+template <class T, bool TransposeLeft, bool TransposeRight, int E>
 __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
     float* __restrict__ out, const float* __restrict__ left, const float* __restrict__ right,
     uint32_t M, uint32_t N, uint32_t K, uint64_t left_batch_stride, uint64_t right_batch_stride) {
   constexpr int TM = T::TM, TN = T::TN, BK = T::BK, S = T::S, KG = T::KG;
   constexpr int kMT = T::kMT, kNT = T::kNT, kUnits = T::kUnits, kP = T::kP;
   constexpr int kDmaA = T::kDmaA, kDmaB = T::kDmaB;
+  constexpr bool KTail = E != kWhole;
   // Distinct LDS objects: a DMA into one stage never aliases the reads of
   // another.
   __shared__ __attribute__((aligned(1024))) uint8_t lds0[T::kStageBytes];
@@ -438,18 +439,34 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
 #pragma unroll
     for (int j = 0; j < kNT; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
+  // kDwords (gemm_common.h): the chunk that K ends in, of K-contiguous rows of
+  // the last step's stage, is cleared past K once every DMA has landed.
+  auto clear_past_k = [&](uint8_t* stage) __attribute__((always_inline)) {
+    const uint32_t chunk = k_tail / 4, valid = k_tail % 4;
+    if (valid == 0) return;
+    auto rows = [&](uint8_t* tile, uint32_t count) {
+      for (uint32_t r = threadIdx.x; r < count; r += T::kThreads)
+        clear_chunk_past(tile + chunk / 8 * (count * 128) + r * 128 + (((chunk % 8) ^ (r & 7u)) << 4), 2 * valid);
+    };
+    if constexpr (kAK) rows(stage, TM);
+    if constexpr (kBK_) rows(stage + T::kABytes, TN);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+
   constexpr int kDma = T::kDma;
   constexpr int kMfma = kUnits * kP * kMT * kNT;
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * kDma) : "memory");
+  if (E == kDwords && ksteps == 1) clear_past_k(lds0);
 #pragma unroll
   for (int r = 0; r < kItems; ++r) read_item(lds0, 0, r);
   // After the barrier every wave's DMA of stage kt + 1 has landed and every
   // wave's reads of stage kt have returned.
-  auto step = [&](uint8_t* cur, const uint8_t* next, int buf, uint32_t kt) __attribute__((always_inline)) {
+  auto step = [&](uint8_t* cur, uint8_t* next, int buf, uint32_t kt) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * kDma) : "memory");
     __builtin_amdgcn_sched_barrier(0);
     dma(cur, clamp(kt + S));
+    if (E == kDwords && kt + 2 == ksteps) clear_past_k(next);
     __builtin_amdgcn_sched_barrier(0);
     int r = 0;
 #pragma unroll
@@ -508,13 +525,25 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
 #pragma unroll
     for (int j = 0; j < kNT; ++j) {
       const uint32_t col = n0 + wn + 16 * j + 4 * g4;
-      if (col < N) *reinterpret_cast<float4_t*>(crow + col) = acc[i][j];
+      if (E != kDwords) {
+        if (col < N) *reinterpret_cast<float4_t*>(crow + col) = acc[i][j];
+      } else {
+        // Rows start dword-aligned and N is any count.
+        typedef float4_t __attribute__((aligned(4))) float4_dwords;
+        if (col + 4 <= N) {
+          *reinterpret_cast<float4_dwords*>(crow + col) = acc[i][j];
+        } else {
+#pragma unroll
+          for (uint32_t e = 0; e < 4; ++e)
+            if (col + e < N) crow[col + e] = acc[i][j][e];
+        }
+      }
     }
   }
 }
 
 template <class T>
-int launch_tile32(hipStream_t stream, const GemmArgs& a) {
+int launch_tile32(hipStream_t stream, const GemmArgs& a, bool chunked) {
   const uint64_t tiles = (uint64_t)((a.rows + T::TM - 1) / T::TM) * ((a.columns + T::TN - 1) / T::TN);
   if (tiles > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
   auto go = [&](auto kernel) {
@@ -523,17 +552,15 @@ int launch_tile32(hipStream_t stream, const GemmArgs& a) {
                        a.columns, a.inner, a.left_batch_stride, a.right_batch_stride);
   };
   const bool tl = a.transpose_left, tr = a.transpose_right;
-  if (a.inner % T::BK == 0) {
-    if (!tl && !tr) go(gemm_f32_tile_kernel<T, false, false, false>);
-    else if (!tl) go(gemm_f32_tile_kernel<T, false, true, false>);
-    else if (!tr) go(gemm_f32_tile_kernel<T, true, false, false>);
-    else go(gemm_f32_tile_kernel<T, true, true, false>);
-  } else {
-    if (!tl && !tr) go(gemm_f32_tile_kernel<T, false, false, true>);
-    else if (!tl) go(gemm_f32_tile_kernel<T, false, true, true>);
-    else if (!tr) go(gemm_f32_tile_kernel<T, true, false, true>);
-    else go(gemm_f32_tile_kernel<T, true, true, true>);
-  }
+  auto layouts = [&]<int E>() {
+    if (!tl && !tr) go(gemm_f32_tile_kernel<T, false, false, E>);
+    else if (!tl) go(gemm_f32_tile_kernel<T, false, true, E>);
+    else if (!tr) go(gemm_f32_tile_kernel<T, true, false, E>);
+    else go(gemm_f32_tile_kernel<T, true, true, E>);
+  };
+  if (!chunked) layouts.template operator()<kDwords>();
+  else if (a.inner % T::BK == 0) layouts.template operator()<kWhole>();
+  else layouts.template operator()<kKTail>();
   return hip_status(hipGetLastError());
 }
 
@@ -564,11 +591,15 @@ int launch_gemm_f32(hipStream_t stream, const GemmArgs& a) {
   // stored): the same kernel with element loads and stores.
   const bool vec = aligned && chunked && a.inner > 0;
   // The tile kernel addresses an operand tile through a buffer descriptor
-  // with 31-bit offsets.
+  // with 31-bit offsets.  Any pitch of fp32 rows is dword-aligned, which its
+  // kDwords form takes: 4096 x 4096 x 4097 1,490 -> 1,035 us, 1000 x 1001 x 1003 106
+  // -> 22, 100 x 1001 x 1000 100 -> 8.4, against the 128 x 128 kernel's element
+  // loads.
   const uint64_t a_span = (a.transpose_left ? (uint64_t)a.rows : 64ull) * a.inner * 4;
   const uint64_t b_span = (a.transpose_right ? 64ull : (uint64_t)a.columns) * a.inner * 4;
-  if (vec && a_span < (1ull << 31) && b_span < (1ull << 31))
-    return smaller_tiles(a) ? launch_tile32<TileF32x32>(stream, a) : launch_tile32<TileF32x64>(stream, a);
+  const bool floats = (uintptr_t)a.left % 4 == 0 && (uintptr_t)a.right % 4 == 0 && (uintptr_t)a.out % 4 == 0;
+  if (floats && a.inner > 0 && a_span < (1ull << 31) && b_span < (1ull << 31))
+    return smaller_tiles(a) ? launch_tile32<TileF32x32>(stream, a, vec) : launch_tile32<TileF32x64>(stream, a, vec);
   if (!a.transpose_left && !a.transpose_right) return launch_fast<false, false>(stream, a, vec);
   if (!a.transpose_left && a.transpose_right) return launch_fast<false, true>(stream, a, vec);
   if (a.transpose_left && !a.transpose_right) return launch_fast<true, false>(stream, a, vec);
