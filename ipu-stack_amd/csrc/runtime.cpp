@@ -13,7 +13,9 @@
 #include <mutex>
 #include <set>
 #include <string>
+#include <string_view>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 #include "internal.h"
@@ -838,13 +840,22 @@ struct Resolved {
   }
 };
 
+const std::unordered_map<std::string_view, const KernelEntry*>& registry_index() {
+  static const auto* index = [] {
+    auto* m = new std::unordered_map<std::string_view, const KernelEntry*>();
+    for (const auto& e : registry()) m->emplace(e.symbol, &e);
+    return m;
+  }();
+  return *index;
+}
+
 int resolve(const char* symbol, Resolved* r) {
   if (!symbol) return fail(IPUS_ERROR_UNKNOWN_SYMBOL, "kernel symbol is null");
-  for (const auto& e : registry())
-    if (strcmp(e.symbol, symbol) == 0) {
-      r->entry = &e;
-      return 0;
-    }
+  const auto found = registry_index().find(symbol);
+  if (found != registry_index().end()) {
+    r->entry = found->second;
+    return 0;
+  }
   for (const auto& f : shape_families()) {
     const size_t n = strlen(f.prefix);
     if (strncmp(symbol, f.prefix, n) != 0) continue;

@@ -130,3 +130,21 @@ def test_failure_injection_and_live_buffer_calls_validate_arguments(ipus):
     n = ipus.ctypes.c_uint64()
     assert lib.ipus_context_live_buffers(None, ipus.ctypes.byref(n), ipus.ctypes.byref(n)) == \
         ipus.ERROR_INVALID_ARGUMENT
+
+
+def test_launch_marshals_every_integer_form(ipus):
+    """Context.launch packs plain unsigned integers and falls back to ctypes
+    conversion for the rest; both reach the same ABI checks (a null context is
+    refused before any device work, an unknown value type before the call)."""
+    import numpy as np
+
+    context = ipus.Context.__new__(ipus.Context)
+    context.handle, context._buffers, context._sessions = None, set(), set()
+    for scalars in ([2], (2,), [np.int64(2)], [2.0], [True], [-1], [1 << 33], list(range(40))):
+        for inputs in ([1], [np.uint64(1)], [1] * 9):
+            with pytest.raises(ipus.IpusError) as e:
+                context.launch("ipu_stack_gelu_tanh_approx_f16", 1, inputs, scalars)
+            assert e.value.status == ipus.ERROR_INVALID_ARGUMENT
+    for bad in ("x", None):
+        with pytest.raises((TypeError, ValueError)):
+            context.launch("ipu_stack_gelu_tanh_approx_f16", 1, [1], [bad])
