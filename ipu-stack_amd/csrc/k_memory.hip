@@ -68,6 +68,29 @@ __device__ __forceinline__ void store16_nt(void* p, u32x4 v) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
 
+// 16-byte accesses at element (2-byte) alignment: one global_load/store_dwordx4
+// (the device runs in unaligned access mode), which costs a second cache line
+// where it crosses one.
+typedef u32x4 __attribute__((aligned(2))) u32x4_elements;
+// Elements c .. c + 7 of a row of `limit` elements, zero past it.
+__device__ __forceinline__ u32x4 load_row8(const uint16_t* row, uint32_t c, uint32_t limit) {
+  if (c + 8 <= limit) return *reinterpret_cast<const u32x4_elements*>(row + c);
+  u32x4 v = {0, 0, 0, 0};
+#pragma unroll
+  for (uint32_t e = 0; e < 8; ++e)
+    if (c + e < limit) v[e / 2] |= (uint32_t)row[c + e] << (16 * (e % 2));
+  return v;
+}
+__device__ __forceinline__ void store_row8(uint16_t* row, uint32_t c, uint32_t limit, u32x4 v) {
+  if (c + 8 <= limit) {
+    *reinterpret_cast<u32x4_elements*>(row + c) = v;
+    return;
+  }
+#pragma unroll
+  for (uint32_t e = 0; e < 8; ++e)
+    if (c + e < limit) row[c + e] = (uint16_t)(v[e / 2] >> (16 * (e % 2)));
+}
+
 // ---------------------------------------------------------------------------
 // Transpose: [matrices][rows][columns] -> [matrices][columns][rows].
 // A wave owns a 64x64 tile; lane (rc = lane % 8, cc = lane / 8) owns the 8x8
@@ -83,16 +106,23 @@ __device__ __forceinline__ void store16_nt(void* p, u32x4 v) {
 // 512 x 128 with one: 5.36, 5.43, 5.39; 128 x 128 with 3-4: 5.21; a
 // persistent grid loading the next tile before storing the current one:
 // 4.9-5.5).
+// Matrices with too few such tiles for the chip take one wave per workgroup
+// (64 x 64 tiles), so that every CU has some.  Any: rows, columns or addresses
+// that are no multiple of 8 elements, with the same blocks read and written at
+// element alignment and by element at the edges (a kernel with one element per
+// thread, reading a column per wave, before: 4313 x 7213 149 -> 33.7 us, 8191 x
+// 8190 208 -> 47.8, 729 x 1152 5.4 -> 4.3 a launch).
 // ---------------------------------------------------------------------------
 constexpr uint32_t kTransposeWaves = 8;
-__global__ __launch_bounds__(64 * kTransposeWaves) void transpose_f16_kernel(
+template <uint32_t Waves, bool Any>
+__global__ __launch_bounds__(64 * Waves) void transpose_f16_kernel(
     uint16_t* __restrict__ dst, const uint16_t* __restrict__ src, uint32_t rows, uint32_t columns,
     uint32_t tiles_c) {
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x % kWave;
   uint32_t tr, tc;
   tile_of_block(tiles_c, 7, &tr, &tc);
-  const uint32_t block_r = tr * (64 * kTransposeWaves) + wave * 64;
+  const uint32_t block_r = tr * (64 * Waves) + wave * 64;
   const uint32_t block_c = tc * 64;
   const uint64_t matrix = blockIdx.y;
   const uint32_t r0 = block_r + (lane % 8) * 8;
@@ -102,23 +132,21 @@ __global__ __launch_bounds__(64 * kTransposeWaves) void transpose_f16_kernel(
   uint16_t* d = dst + matrix * rows * (uint64_t)columns;
   u32x4 in[8], out[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) in[j] = load16_nt(s + (uint64_t)(r0 + j) * columns + c0);
+  for (int j = 0; j < 8; ++j) {
+    if constexpr (Any)
+      in[j] = r0 + j < rows ? load_row8(s + (uint64_t)(r0 + j) * columns, c0, columns) : u32x4{0, 0, 0, 0};
+    else
+      in[j] = load16_nt(s + (uint64_t)(r0 + j) * columns + c0);
+  }
   transpose8x8_u16(in, out);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) store16_nt(d + (uint64_t)(c0 + i) * rows + r0, out[i]);
-}
-
-__global__ __launch_bounds__(kThreads) void transpose_f16_scalar_kernel(
-    uint16_t* __restrict__ dst, const uint16_t* __restrict__ src, uint32_t rows, uint32_t columns,
-    uint64_t total) {
-  const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= total) return;
-  const uint64_t me = (uint64_t)rows * columns;
-  const uint64_t matrix = idx / me;
-  const uint64_t within = idx % me;  // index in the destination [columns][rows]
-  const uint32_t c = (uint32_t)(within / rows);
-  const uint32_t r = (uint32_t)(within % rows);
-  dst[idx] = src[matrix * me + (uint64_t)r * columns + c];
+  for (int i = 0; i < 8; ++i) {
+    if constexpr (Any) {
+      if (c0 + i < columns) store_row8(d + (uint64_t)(c0 + i) * rows, r0, rows, out[i]);
+    } else {
+      store16_nt(d + (uint64_t)(c0 + i) * rows + r0, out[i]);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -128,20 +156,31 @@ __global__ __launch_bounds__(kThreads) void transpose_f16_scalar_kernel(
 // covers 16 rows x 256 columns: lane % 2 picks the row half, lane / 2 the
 // 8-column chunk.
 // ---------------------------------------------------------------------------
+// Padded: source rows of any extent and alignment, [logical_rows,
+// logical_columns], zero up to [rows, columns].
+template <bool Padded>
 __global__ __launch_bounds__(kThreads) void block_major_f16_kernel(
     uint16_t* __restrict__ dst, const uint16_t* __restrict__ src, uint32_t rows, uint32_t columns,
-    uint32_t row_block, uint32_t column_block, uint32_t tiles_c) {
+    uint32_t row_block, uint32_t column_block, uint32_t tiles_c, uint32_t logical_rows,
+    uint32_t logical_columns) {
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x % kWave;
   const uint32_t r0 = (blockIdx.x / tiles_c) * 64 + wave * 16 + (lane % 2) * 8;
   const uint32_t c0 = (blockIdx.x % tiles_c) * 256 + (lane / 2) * 8;
   if (r0 >= rows || c0 >= columns) return;
   const uint64_t me = (uint64_t)rows * columns;
-  const uint16_t* s = src + blockIdx.y * me;
+  const uint16_t* s = src + blockIdx.y * (Padded ? (uint64_t)logical_rows * logical_columns : me);
   uint16_t* d = dst + blockIdx.y * me;
   u32x4 in[8], out[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) in[j] = load16(s + (uint64_t)(r0 + j) * columns + c0);
+  for (int j = 0; j < 8; ++j) {
+    if constexpr (Padded)
+      in[j] = r0 + j < logical_rows
+                  ? load_row8(s + (uint64_t)(r0 + j) * logical_columns, c0, logical_columns)
+                  : u32x4{0, 0, 0, 0};
+    else
+      in[j] = load16(s + (uint64_t)(r0 + j) * columns + c0);
+  }
   transpose8x8_u16(in, out);
 #pragma unroll
   for (int i = 0; i < 8; ++i)
@@ -300,6 +339,33 @@ __global__ __launch_bounds__(kThreads) void amp_tile_f16_kernel(uint16_t* __rest
 #pragma unroll
   for (uint32_t i = 0; i < kPer; ++i)
     if (ok[i]) store16_nt(dst + to[i], v[i]);
+}
+
+// Row-major rows of any extent and alignment -> AMP-Left or AMP-TransposedRight
+// padded to [physical_rows, physical_columns]: the same chunks, each thread one,
+// the source read at element alignment and zero past its rows and columns.
+// us against one element per thread with the inverse map: 4313 x 7213 to
+// AMP-Left 61.8 -> 27.5, to AMP-TransposedRight 66 -> 26.8, to 64 x 64 blocks
+// (block_major_f16_kernel) 95 -> 28; 2000 x 2001 to AMP-Left 10.7 -> 3.9.
+template <uint32_t Order>
+__global__ __launch_bounds__(kThreads) void amp_padded_f16_kernel(
+    uint16_t* __restrict__ dst, const uint16_t* __restrict__ src, uint32_t rows,
+    uint32_t logical_rows, uint32_t physical_rows, uint32_t logical_columns,
+    uint32_t physical_columns, uint32_t tiles_c) {
+  // 32 x 64 tiles; AMP-Left: `rows` is every matrix's physical rows.
+  const uint32_t tr = blockIdx.x / tiles_c, tc = blockIdx.x % tiles_c;
+  const uint32_t r = tr * 32 + threadIdx.x / 8, c = tc * 64 + threadIdx.x % 8 * 8;
+  if (r >= rows || c >= physical_columns) return;
+  const uint32_t matrix = Order == kOrderAmpLeft ? r / physical_rows : blockIdx.y;
+  const uint32_t row = Order == kOrderAmpLeft ? r % physical_rows : r;
+  u32x4 v = {0, 0, 0, 0};
+  if (row < logical_rows)
+    v = load_row8(src + ((uint64_t)matrix * logical_rows + row) * logical_columns, c, logical_columns);
+  const uint64_t to = Order == kOrderAmpLeft
+                          ? amp_left_index(rows, r, c)
+                          : (uint64_t)matrix * physical_rows * physical_columns +
+                                amp_transposed_right_index(physical_rows, physical_columns, r, c);
+  store16(dst + to, v);
 }
 
 // Unpack AMP-Output (pair-permuted 16-column micros, storage.rs:329-340),
@@ -855,15 +921,30 @@ inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 int launch_transpose_f16(hipStream_t stream, void* dst, const void* src, uint32_t matrices,
                          uint32_t rows, uint32_t columns) {
   if (matrices == 0 || rows == 0 || columns == 0) return 0;
-  if (rows % 8 == 0 && columns % 8 == 0 && aligned16(dst) && aligned16(src) && matrices <= 65535) {
-    const uint32_t tiles_r = ceil_div(rows, 64 * kTransposeWaves), tiles_c = ceil_div(columns, 64);
-    hipLaunchKernelGGL(transpose_f16_kernel, dim3(tiles_r * tiles_c, matrices),
-                       dim3(64 * kTransposeWaves), occupancy_lds(1, 0), stream, (uint16_t*)dst,
-                       (const uint16_t*)src, rows, columns, tiles_c);
-  } else {
-    const uint64_t total = (uint64_t)matrices * rows * columns;
-    hipLaunchKernelGGL(transpose_f16_scalar_kernel, dim3(ceil_div(total, kThreads)), dim3(kThreads),
-                       0, stream, (uint16_t*)dst, (const uint16_t*)src, rows, columns, total);
+  const bool chunks = rows % 8 == 0 && columns % 8 == 0 && aligned16(dst) && aligned16(src);
+  const uint32_t tiles_c = ceil_div(columns, 64);
+  const uint64_t tall = (uint64_t)ceil_div(rows, 64 * kTransposeWaves) * tiles_c;
+  const uint64_t small = (uint64_t)ceil_div(rows, 64) * tiles_c;
+  if (small > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
+  // Matrices beyond the grid's second dimension: one launch per 65535.
+  for (uint32_t first = 0; first < matrices; first += 65535) {
+    const uint32_t count = matrices - first < 65535 ? matrices - first : 65535;
+    uint16_t* d = (uint16_t*)dst + (uint64_t)first * rows * columns;
+    const uint16_t* s = (const uint16_t*)src + (uint64_t)first * rows * columns;
+    auto go = [&](auto kernel, uint64_t tiles, uint32_t waves, uint32_t lds) {
+      hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, count), dim3(64 * waves), lds, stream, d, s, rows,
+                         columns, tiles_c);
+    };
+    // Up to two rounds of the tall tiles (one workgroup per CU), 64 x 64 tiles
+    // are as fast or faster: 2048^2 5.2 -> 4.4 us a launch, 2048 x 4096 6.8 -> 5.9,
+    // 4096^2 13.4 -> 12.1-13.3; beyond, the tall ones hold (8192^2 45.5).
+    if (tall * count > 512) {
+      if (chunks) go(transpose_f16_kernel<kTransposeWaves, false>, tall, kTransposeWaves, occupancy_lds(1, 0));
+      else go(transpose_f16_kernel<kTransposeWaves, true>, tall, kTransposeWaves, occupancy_lds(1, 0));
+    } else {
+      if (chunks) go(transpose_f16_kernel<1, false>, small, 1, 0);
+      else go(transpose_f16_kernel<1, true>, small, 1, 0);
+    }
   }
   return hip_status(hipGetLastError());
 }
@@ -899,6 +980,40 @@ bool launch_amp_tile(hipStream_t stream, void* dst, const void* src, uint32_t or
   return true;
 }
 
+// Any source extent and alignment into an aligned destination padded to its
+// order's blocks; false where a block or the grid does not fit (the
+// one-element-per-thread kernel then).
+bool launch_padded(hipStream_t stream, void* dst, const void* src, uint32_t order,
+                   uint32_t row_block, uint32_t column_block, uint32_t matrices,
+                   uint32_t logical_rows, uint32_t physical_rows, uint32_t logical_columns,
+                   uint32_t physical_columns) {
+  if (!aligned16(dst)) return false;
+  if (order == kOrderBlockMajor) {
+    const uint32_t tiles_c = ceil_div(physical_columns, 256);
+    const uint64_t tiles = (uint64_t)ceil_div(physical_rows, 64) * tiles_c;
+    // Below 96 tiles the element kernel's many small workgroups are as fast
+    // (1152 x 729: 54 tiles 5.3 us a launch, elements 5.1).
+    if (column_block % 8 != 0 || matrices > 65535 || tiles > 0x7fffffffull || tiles * matrices < 96) return false;
+    hipLaunchKernelGGL(block_major_f16_kernel<true>, dim3((uint32_t)tiles, matrices), dim3(kThreads), 0,
+                       stream, (uint16_t*)dst, (const uint16_t*)src, physical_rows, physical_columns,
+                       row_block, column_block, tiles_c, logical_rows, logical_columns);
+    return true;
+  }
+  const bool left = order == kOrderAmpLeft;
+  const uint64_t rows = left ? (uint64_t)matrices * physical_rows : physical_rows;
+  const uint32_t tiles_c = ceil_div(physical_columns, 64);
+  const uint64_t tiles = ceil_div(rows, 32) * (uint64_t)tiles_c;
+  if (rows > 0xffffffffull || tiles > 0x7fffffffull || (!left && matrices > 65535)) return false;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, left ? 1 : matrices), dim3(kThreads), 0, stream,
+                       (uint16_t*)dst, (const uint16_t*)src, (uint32_t)rows, logical_rows, physical_rows,
+                       logical_columns, physical_columns, tiles_c);
+  };
+  if (left) go(amp_padded_f16_kernel<kOrderAmpLeft>);
+  else go(amp_padded_f16_kernel<kOrderAmpTransposedRight>);
+  return true;
+}
+
 int launch_rearrange_f16(hipStream_t stream, void* dst, const void* src, uint32_t target_order,
                          uint32_t row_block, uint32_t column_block, uint32_t matrices,
                          uint32_t logical_rows, uint32_t physical_rows, uint32_t logical_columns,
@@ -930,14 +1045,18 @@ int launch_rearrange_f16(hipStream_t stream, void* dst, const void* src, uint32_
                        column_block, tiles_c);
   } else if (fast_block_major) {
     const uint32_t tiles_r = ceil_div(physical_rows, 64), tiles_c = ceil_div(physical_columns, 256);
-    hipLaunchKernelGGL(block_major_f16_kernel, dim3(tiles_r * tiles_c, matrices), dim3(kThreads), 0,
+    hipLaunchKernelGGL(block_major_f16_kernel<false>, dim3(tiles_r * tiles_c, matrices), dim3(kThreads), 0,
                        stream, (uint16_t*)dst, (const uint16_t*)src, physical_rows,
-                       physical_columns, row_block, column_block, tiles_c);
+                       physical_columns, row_block, column_block, tiles_c, physical_rows,
+                       physical_columns);
   } else if (target_order != kOrderBlockMajor && logical_rows == physical_rows &&
              logical_columns == physical_columns && aligned16(dst) && aligned16(src) &&
              launch_amp_tile<false>(stream, dst, src, target_order, matrices, physical_rows,
                                     physical_columns)) {
     // launched by launch_amp_tile
+  } else if (launch_padded(stream, dst, src, target_order, row_block, column_block, matrices,
+                           logical_rows, physical_rows, logical_columns, physical_columns)) {
+    // launched by launch_padded
   } else {
     hipLaunchKernelGGL(rearrange_f16_general_kernel, dim3(ceil_div(total, kThreads)),
                        dim3(kThreads), 0, stream, (uint16_t*)dst, (const uint16_t*)src,

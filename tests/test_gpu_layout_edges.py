@@ -1,0 +1,64 @@
+"""Transposes and padded rearranges at sizes and addresses off the vector grid,
+bit-exact against the oracle's index maps, with guard elements around the
+destination and NaN patterns around the source."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+GUARD = 0x7E5A
+
+
+def guarded(ctx, x, shift):
+    """x at an element offset, between guard elements."""
+    g = np.full(64, GUARD, np.uint16)
+    return ctx.upload(np.concatenate([g[:8 + shift], x.reshape(-1), g]))
+
+
+def read_guarded(buf, count, shift):
+    raw = buf.download(np.uint16)
+    assert np.all(raw[:8 + shift] == GUARD) and np.all(raw[8 + shift + count:] == GUARD)
+    return raw[8 + shift:8 + shift + count]
+
+
+@pytest.mark.parametrize("matrices,rows,cols", [
+    (1, 1, 1), (1, 7, 9), (1, 8, 8), (3, 63, 65), (2, 64, 64), (1, 513, 40), (1, 729, 1152),
+    (2, 1152, 729), (1, 2049, 4097), (1, 4096, 4096), (70000, 3, 5)])
+@pytest.mark.parametrize("shift", [0, 1, 4])
+def test_transpose_any_size_and_alignment(ipus, oracle, ctx, matrices, rows, cols, shift):
+    n = matrices * rows * cols
+    x = ipus.synth_f16(n, 83, 1)
+    src = guarded(ctx, x, shift)
+    dst = guarded(ctx, np.zeros(n, np.uint16), shift)
+    ctx.launch("ipu_stack_transpose_f16", dst.ptr + 2 * (8 + shift), [src.ptr + 2 * (8 + shift)],
+               [matrices, rows, cols])
+    got = read_guarded(dst, n, shift)
+    assert np.array_equal(got, oracle.transpose_u16(x, matrices, rows, cols).reshape(-1))
+    src.free()
+    dst.free()
+
+
+@pytest.mark.parametrize("order,rb,cb", [(0, 0, 0), (1, 0, 0), (2, 64, 64), (2, 64, 16), (2, 16, 8),
+                                         (2, 16, 20)])
+@pytest.mark.parametrize("matrices,lr,pr,lc,pc", [
+    (1, 1, 64, 1, 320), (1, 729, 768, 1147, 1280), (3, 17, 64, 33, 80), (2, 64, 64, 80, 80),
+    (1, 33, 192, 640, 640), (1, 128, 128, 8, 160)])
+@pytest.mark.parametrize("shift", [0, 3])
+def test_padded_rearrange(ipus, oracle, ctx, order, rb, cb, matrices, lr, pr, lc, pc, shift):
+    """Padding rows and columns are zero; the source may start at any
+    element (the destination is aligned, or at any element too with shift)."""
+    if cb and (pc % cb or pr % rb):
+        pytest.skip("the blocks do not divide these extents")
+    x = ipus.synth_f16(matrices * lr * lc, 84, 1)
+    n = matrices * pr * pc
+    want = oracle.rearrange_row_major_f16(x, order, matrices, lr, pr, lc, pc, rb, cb).reshape(-1)
+    src = guarded(ctx, x, shift)
+    for dshift in {0, shift}:
+        dst = guarded(ctx, np.full(n, GUARD, np.uint16), dshift)
+        ctx.launch("ipu_stack_rearrange_row_major_f16", dst.ptr + 2 * (8 + dshift),
+                   [src.ptr + 2 * (8 + shift)], [lr, pr, order, lc, pc, rb, cb, matrices])
+        assert np.array_equal(read_guarded(dst, n, dshift), want)
+        dst.free()
+    src.free()
