@@ -55,26 +55,39 @@ __device__ __forceinline__ u32x4 add_f16x8(u32x4 product, u32x4 addend) {
 
 // Operand edges of the LDS-DMA kernels.  kWhole: K a multiple of the K step,
 // every row pitch a multiple of 8 elements, 16-byte aligned addresses.  kKTail:
-// the same with a partial last step.  kDwords: pitches and addresses that are
-// only multiples of 4 bytes (and any K): the DMA fetches the same 16-byte
+// the same with a partial last step.  kDwords: operand pitches and addresses that
+// are only multiples of 4 bytes (any K, and any C): the DMA fetches the same 16-byte
 // chunks, dword-aligned; a chunk that runs past M or N along a row holds
 // elements of the next row, which reach only rows or columns of C that are not
 // stored, and a chunk that runs past K along a row is cleared past K in LDS
 // (clear_past_k) before the last step reads it.
-enum Edge : int { kWhole = 0, kKTail = 1, kDwords = 2 };
+// kElements (k_gemm_f16_tile.hip only): any pitch, address and extent; the
+// chunks go through registers instead, read at element alignment.
+enum Edge : int { kWhole = 0, kKTail = 1, kDwords = 2, kElements = 3 };
 
-// 16 bytes of C (8 columns of one row) at a dword-aligned address, `valid` of
-// them inside the row.
-__device__ __forceinline__ void store_dwords(uint16_t* p, u32x4 v, uint32_t valid) {
-  typedef u32x4 __attribute__((aligned(4))) u32x4_dwords;
+// 16-byte access at element (2-byte) alignment: one global_load/store_dwordx4
+// (the device runs in unaligned access mode).
+typedef u32x4 __attribute__((aligned(2))) u32x4_elements;
+// Elements at .. at + 7 of an operand of `total` elements, zero past its end.
+__device__ __forceinline__ u32x4 load_chunk(const uint16_t* x, uint64_t at, uint64_t total) {
+  if (at + 8 <= total) return *reinterpret_cast<const u32x4_elements*>(x + at);
+  u32x4 v = {0, 0, 0, 0};
+#pragma unroll
+  for (uint32_t e = 0; e < 8; ++e)
+    if (at + e < total) v[e / 2] |= (uint32_t)x[at + e] << (16 * (e % 2));
+  return v;
+}
+// 16 bytes of C (8 columns of one row), `valid` columns of them inside the row.
+__device__ __forceinline__ void store_elements(uint16_t* p, u32x4 v, uint32_t valid) {
   if (valid >= 8) {
-    *reinterpret_cast<u32x4_dwords*>(p) = v;
+    *reinterpret_cast<u32x4_elements*>(p) = v;
   } else {
 #pragma unroll
-    for (uint32_t w = 0; w < 4; ++w)  // N is even, so words are whole
-      if (2 * w < valid) *reinterpret_cast<uint32_t*>(p + 2 * w) = v[w];
+    for (uint32_t e = 0; e < 8; ++e)
+      if (e < valid) p[e] = (uint16_t)(v[e / 2] >> (16 * (e % 2)));
   }
 }
+
 // Eight elements of an addend row of any alignment, `valid` of them inside it.
 __device__ __forceinline__ u32x4 load_elements(const uint16_t* p, uint32_t valid) {
   u32x4 v = {0, 0, 0, 0};
@@ -83,13 +96,17 @@ __device__ __forceinline__ u32x4 load_elements(const uint16_t* p, uint32_t valid
     if (e < valid) v[e / 2] |= (uint32_t)p[e] << (16 * (e % 2));
   return v;
 }
-// Keeps the first `valid` elements of a 16-byte chunk in LDS (0 <= valid < 8).
-__device__ __forceinline__ void clear_chunk_past(uint8_t* chunk, uint32_t valid) {
-  u32x4 v = *reinterpret_cast<const u32x4*>(chunk);
+// The first `valid` elements of a chunk, zero past them.
+__device__ __forceinline__ u32x4 keep_elements(u32x4 v, uint32_t valid) {
 #pragma unroll
   for (uint32_t w = 0; w < 4; ++w)
     v[w] &= (2 * w < valid ? 0xffffu : 0u) | (2 * w + 1 < valid ? 0xffff0000u : 0u);
-  *reinterpret_cast<u32x4*>(chunk) = v;
+  return v;
+}
+// The same on a chunk in LDS.
+__device__ __forceinline__ void clear_chunk_past(uint8_t* chunk, uint32_t valid) {
+  u32x4* p = reinterpret_cast<u32x4*>(chunk);
+  *p = keep_elements(*p, valid);
 }
 
 }  // namespace ipus

@@ -53,9 +53,8 @@
 //     MN-contiguous rows past K on the last step, get an offset past the
 //     range; the epilogue stores only rows < M and 8-column chunks < N
 //     (kDwords: columns < N, see gemm_common.h).
-// Products with too few 256 x 256 tiles for the chip run smaller tiles
-// (k_gemm_f16_tile.hip, gemm_f16_tile).  Small-tile kernel below (64 x 64 or
-// 32 x 32 tiles): any shape or alignment the fast kernel does not take.
+// Products with too few 256 x 256 tiles for the chip, and any shape or alignment
+// this kernel does not take, run smaller tiles (k_gemm_f16_tile.hip).
 #include "../../include/ipus.h"
 
 #include <mutex>
@@ -408,7 +407,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
         const u32x4 x = *reinterpret_cast<const u32x4*>(cst + r * 256 + ((c ^ (r & 15)) << 4));
         if (m0 + wm + r < M && n0 + wn + c * 8 < N) {
           uint16_t* p = cw + (uint64_t)r * N + c * 8;
-          if constexpr (E == kDwords) store_dwords(p, add_f16x8(x, d[k]), N - (n0 + wn + c * 8));
+          if constexpr (E == kDwords) store_elements(p, add_f16x8(x, d[k]), N - (n0 + wn + c * 8));
           else __builtin_nontemporal_store(add_f16x8(x, d[k]), reinterpret_cast<u32x4*>(p));
         }
       }
@@ -426,259 +425,10 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
     // product cost the 8192^3 GEMMs 1.5%.
     if (m0 + wm + r < M && n0 + wn + c * 8 < N) {
       u32x4* p = reinterpret_cast<u32x4*>(cw + (uint64_t)r * N + c * 8);
-      if constexpr (E == kDwords) store_dwords(reinterpret_cast<uint16_t*>(p), x, N - (n0 + wn + c * 8));
+      if constexpr (E == kDwords) store_elements(reinterpret_cast<uint16_t*>(p), x, N - (n0 + wn + c * 8));
       else if constexpr (Epi == kEpiGelu) *p = x;
       else __builtin_nontemporal_store(x, p);
     }
-  }
-}
-
-// Register-staged fp16 GEMM: 64 x 64 or 32 x 32 output tiles, for operands the
-// LDS-DMA kernels do not take (odd row pitches, addresses that are not
-// 4-byte multiples, operands past their 31-bit buffer ranges, K = 0).  256 threads = 4
-// waves in a 2 x 2 grid, each (Tile / 2)^2 of C as tiles of
-// v_mfma_f32_16x16x32_f16 (C^T as in the 256 x 256 kernel, so a lane holds
-// 4 consecutive columns).  K runs in chunks of 256: a chunk's
-// operand tiles (4 steps of 64) are loaded to registers, 16 loads of 16
-// bytes per thread in flight at once, stored to four LDS stages, and
-// computed while the next chunk's loads are in flight; a K of at most 256
-// takes one memory round trip.  K-contiguous tiles are stored [64 rows][64 k]
-// with the 256 x 256 kernel's XOR swizzle and read with ds_read_b128;
-// MN-contiguous tiles [64 k][64 mn] are read with ds_read_b64_tr_b16.
-// Chunks past M, N or K are not loaded and stay 0.  Vec = 8: N and K, and
-// M when A is transposed, are multiples of 8 and the operands 16-byte
-// aligned (operands past the LDS-DMA kernels' ranges).  Vec = 4 or 1: each 16-byte LDS chunk
-// is gathered from 8-byte or 2-byte loads, elements past M, N or K are 0,
-// and the epilogue stores element by element.
-constexpr uint32_t kSmallChunk = 256;
-constexpr uint32_t kSmallSteps = kSmallChunk / 64;
-
-template <uint32_t Tile, bool TransposeLeft, bool TransposeRight, int Epi, int Vec = 8>
-__global__ __launch_bounds__(256) void gemm_f16_small_kernel(
-    uint16_t* out, const uint16_t* __restrict__ left, const uint16_t* __restrict__ right,
-    uint32_t M, uint32_t N, uint32_t K, uint64_t left_batch_stride, uint64_t right_batch_stride,
-    uint32_t tiles_n, const uint16_t* addend, uint64_t addend_batch_stride,
-    uint32_t addend_row_stride) {
-  constexpr uint32_t kWT = Tile / 32;                 // 16 x 16 tiles per wave and dimension
-  constexpr uint32_t kStepBytes = Tile * 64 * 2;      // one operand, one 64-k step
-  constexpr uint32_t kMnRow = Tile * 2;               // bytes of an MN-contiguous k row
-  constexpr uint32_t kMnChunks = Tile / 8;            // 16-byte chunks of such a row
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2][kSmallSteps][kStepBytes];
-  constexpr bool kAK = !TransposeLeft;   // A rows (m) K-contiguous
-  constexpr bool kBK_ = TransposeRight;  // B^T rows (n) K-contiguous
-  const uint64_t batch = blockIdx.y;
-  const uint16_t* A = left + batch * left_batch_stride;
-  const uint16_t* B = right + batch * right_batch_stride;
-  uint16_t* C = out + batch * (uint64_t)M * N;
-  const uint32_t m0 = blockIdx.x / tiles_n * Tile, n0 = blockIdx.x % tiles_n * Tile;
-  const uint32_t wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const uint32_t wm = (wave / 2) * (Tile / 2), wn = (wave % 2) * (Tile / 2);
-  const uint32_t r16 = lane % 16, g4 = lane / 16;
-
-  // Chunk q = threadIdx.x + 256 i of an operand's 4 steps: step q / (steps'
-  // chunks), then (row, k chunk) for a K-contiguous tile (8 chunks a row) or
-  // (k row, mn chunk) for an MN-contiguous one (Tile / 8 chunks a row).
-  constexpr uint32_t kStepChunks = kStepBytes / 16;
-  constexpr uint32_t kPer = kSmallSteps * kStepChunks / 256;
-  u32x4 ra[kPer], rb[kPer];
-  auto load_operand = [&]<bool KContig>(const uint16_t* X, uint32_t mn0, uint32_t mn_limit,
-                                        uint32_t ld, uint32_t k0, u32x4* r) __attribute__((always_inline)) {
-#pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i) {
-      const uint32_t q = threadIdx.x + 256 * i, step = q / kStepChunks, w = q % kStepChunks;
-      const uint32_t per_row = KContig ? 8 : kMnChunks;
-      const uint32_t major = w / per_row, minor = w % per_row * 8;
-      const uint32_t k = KContig ? k0 + step * 64 + minor : k0 + step * 64 + major;
-      const uint32_t mn = KContig ? mn0 + major : mn0 + minor;
-      const uint16_t* p = X + (KContig ? (uint64_t)mn * ld + k : (uint64_t)k * ld + mn);
-      if constexpr (Vec == 8) {
-        const bool ok = k < K && mn < mn_limit;
-        r[i] = ok ? load16(p) : u32x4{0, 0, 0, 0};
-      } else {
-        // The chunk's 8 elements run along the contiguous axis (k or mn);
-        // groups of Vec are wholly in or out, as Vec divides that extent.
-        const bool row_ok = KContig ? mn < mn_limit : k < K;
-        const uint32_t c0 = KContig ? k : mn, c_limit = KContig ? K : mn_limit;
-        uint16_t e[8];
-#pragma unroll
-        for (uint32_t g = 0; g < 8; g += Vec) {
-          const bool ok = row_ok && c0 + g < c_limit;
-          if constexpr (Vec == 4) {
-            const u32x2 v = ok ? *reinterpret_cast<const u32x2*>(p + g) : u32x2{0, 0};
-            e[g] = (uint16_t)v[0];
-            e[g + 1] = (uint16_t)(v[0] >> 16);
-            e[g + 2] = (uint16_t)v[1];
-            e[g + 3] = (uint16_t)(v[1] >> 16);
-          } else {
-            e[g] = ok ? p[g] : (uint16_t)0;
-          }
-        }
-        r[i] = u32x4{e[0] | (uint32_t)e[1] << 16, e[2] | (uint32_t)e[3] << 16,
-                     e[4] | (uint32_t)e[5] << 16, e[6] | (uint32_t)e[7] << 16};
-      }
-    }
-  };
-  auto store_operand = [&]<bool KContig>(uint8_t (*stage)[kStepBytes], const u32x4* r) __attribute__((always_inline)) {
-#pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i) {
-      const uint32_t q = threadIdx.x + 256 * i, step = q / kStepChunks, w = q % kStepChunks;
-      const uint32_t per_row = KContig ? 8 : kMnChunks;
-      const uint32_t major = w / per_row, chunk = w % per_row;
-      const uint32_t off = KContig ? kc_off<64>(major, chunk) : major * kMnRow + chunk * 16;
-      *reinterpret_cast<u32x4*>(stage[step] + off) = r[i];
-    }
-  };
-  auto load_chunk = [&](uint32_t k0) __attribute__((always_inline)) {
-    load_operand.template operator()<kAK>(A, m0, M, kAK ? K : M, k0, ra);
-    load_operand.template operator()<kBK_>(B, n0, N, kBK_ ? K : N, k0, rb);
-  };
-  auto store_chunk = [&]() __attribute__((always_inline)) {
-    store_operand.template operator()<kAK>(lds[0], ra);
-    store_operand.template operator()<kBK_>(lds[1], rb);
-  };
-  // Fragment of 16 rows (m or n) w0 + 16 t + .., k 32 ss + 8 (lane / 16) ..+7.
-  auto frag = [&]<bool KContig>(const uint8_t* tile, uint32_t w0, uint32_t t, uint32_t ss) __attribute__((always_inline)) {
-    if constexpr (KContig) {
-      const uint32_t row = w0 + 16 * t + r16;
-      return __builtin_bit_cast(
-          half8_t, *reinterpret_cast<const u32x4*>(tile + kc_off<64>(row, 4 * ss + g4)));
-    } else {
-      // 16-lane group g reads k rows 32 ss + 8 g + {0..3} (then +4): lane s
-      // addresses k row + s / 4, columns w0 + 16 t + 4 (s % 4) .. +3.
-      const uint32_t k = 32 * ss + 8 * g4 + r16 / 4;
-      const uint32_t a = k * kMnRow + (w0 + 16 * t + 4 * (r16 % 4)) * 2;
-      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS short4_t*)(tile + a));
-      const short4_t hi =
-          __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS short4_t*)(tile + a + 4 * kMnRow));
-      return __builtin_bit_cast(half8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    }
-  };
-
-  float4_t acc[kWT][kWT];
-#pragma unroll
-  for (uint32_t i = 0; i < kWT; ++i)
-#pragma unroll
-    for (uint32_t j = 0; j < kWT; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  const uint32_t chunks = (K + kSmallChunk - 1) / kSmallChunk;
-  load_chunk(0);
-  store_chunk();
-  __syncthreads();
-  for (uint32_t c = 0; c < chunks; ++c) {
-    if (c + 1 < chunks) load_chunk((c + 1) * kSmallChunk);
-#pragma unroll
-    for (uint32_t step = 0; step < kSmallSteps; ++step)
-#pragma unroll
-      for (uint32_t ss = 0; ss < 2; ++ss) {
-        half8_t fa[kWT], fb[kWT];
-#pragma unroll
-        for (uint32_t t = 0; t < kWT; ++t) {
-          fa[t] = frag.template operator()<kAK>(lds[0][step], wm, t, ss);
-          fb[t] = frag.template operator()<kBK_>(lds[1][step], wn, t, ss);
-        }
-#pragma unroll
-        for (uint32_t i = 0; i < kWT; ++i)
-#pragma unroll
-          for (uint32_t j = 0; j < kWT; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[j], fa[i], acc[i][j], 0, 0, 0);
-      }
-    if (c + 1 < chunks) {
-      __syncthreads();  // every wave is done reading the stages
-      store_chunk();
-      __syncthreads();
-    }
-  }
-  // acc[i][j][e] = C[m0 + wm + 16 i + lane % 16][n0 + wn + 16 j + 4 (lane / 16) + e]
-#pragma unroll
-  for (uint32_t i = 0; i < kWT; ++i) {
-    const uint32_t m = m0 + wm + 16 * i + r16;
-    if (m >= M) continue;
-#pragma unroll
-    for (uint32_t j = 0; j < kWT; ++j) {
-      const uint32_t n = n0 + wn + 16 * j + 4 * g4;
-      if (n >= N) continue;
-      half4_t h;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) h[e] = epilogue<Epi>(acc[i][j][e]);
-      if constexpr (Vec == 8) {
-        // N % 8 == 0: a lane's 4 columns are all in or all out.
-        if constexpr (Epi == kEpiAdd) {
-          const half4_t d = *reinterpret_cast<const half4_t*>(
-              addend + batch * addend_batch_stride + (uint64_t)m * addend_row_stride + n);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) h[e] = add_f16(h[e], d[e]);
-        }
-        *reinterpret_cast<half4_t*>(C + (uint64_t)m * N + n) = h;
-      } else {
-#pragma unroll
-        for (uint32_t e = 0; e < 4; ++e) {
-          if (n + e >= N) break;
-          half_t v = h[e];
-          if constexpr (Epi == kEpiAdd)
-            v = add_f16(v, __builtin_bit_cast(half_t, addend[batch * addend_batch_stride +
-                                                             (uint64_t)m * addend_row_stride + n + e]));
-          C[(uint64_t)m * N + n + e] = __builtin_bit_cast(uint16_t, v);
-        }
-      }
-    }
-  }
-}
-
-// 64 x 64 tiles, or 32 x 32 when there are fewer 64 x 64 tiles than a
-// quarter of the CUs (256^3: 64 workgroups instead of 16).
-template <int Epi, int Vec = 8>
-int launch_small(hipStream_t stream, const GemmArgs& a) {
-  const uint64_t tiles64 = (uint64_t)((a.rows + 63) / 64) * ((a.columns + 63) / 64);
-  const uint32_t tile = tiles64 * a.batches < 64 ? 32 : 64;
-  const uint32_t tiles_m = (a.rows + tile - 1) / tile;
-  const uint32_t tiles_n = (a.columns + tile - 1) / tile;
-  if ((uint64_t)tiles_m * tiles_n > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
-  const dim3 grid(tiles_m * tiles_n, a.batches);
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, (uint16_t*)a.out,
-                       (const uint16_t*)a.left, (const uint16_t*)a.right, a.rows, a.columns,
-                       a.inner, a.left_batch_stride, a.right_batch_stride, tiles_n,
-                       (const uint16_t*)a.addend, a.addend_batch_stride, a.addend_row_stride);
-  };
-  const bool tl = a.transpose_left, tr = a.transpose_right;
-  if (tile == 32) {
-    if (!tl && !tr) go(gemm_f16_small_kernel<32, false, false, Epi, Vec>);
-    else if (!tl) go(gemm_f16_small_kernel<32, false, true, Epi, Vec>);
-    else if (!tr) go(gemm_f16_small_kernel<32, true, false, Epi, Vec>);
-    else go(gemm_f16_small_kernel<32, true, true, Epi, Vec>);
-  } else {
-    if (!tl && !tr) go(gemm_f16_small_kernel<64, false, false, Epi, Vec>);
-    else if (!tl) go(gemm_f16_small_kernel<64, false, true, Epi, Vec>);
-    else if (!tr) go(gemm_f16_small_kernel<64, true, false, Epi, Vec>);
-    else go(gemm_f16_small_kernel<64, true, true, Epi, Vec>);
-  }
-  return hip_status(hipGetLastError());
-}
-
-// Elements per global load (8, 4 or 1) that every operand row, batch and
-// base address allows, and 8 only where the addend and output allow the
-// 16-byte epilogue too.
-uint32_t small_vec(const GemmArgs& a) {
-  auto fits = [&](uint32_t v) {
-    const uint32_t lda = a.transpose_left ? a.rows : a.inner;
-    const uint32_t ldb = a.transpose_right ? a.inner : a.columns;
-    bool ok = lda % v == 0 && ldb % v == 0 && (uintptr_t)a.left % (2 * v) == 0 &&
-              (uintptr_t)a.right % (2 * v) == 0 && a.left_batch_stride % v == 0 &&
-              a.right_batch_stride % v == 0;
-    if (v == 8)
-      ok = ok && a.inner % 8 == 0 && a.columns % 8 == 0 && (uintptr_t)a.out % 16 == 0 &&
-           (!a.addend || ((uintptr_t)a.addend % 16 == 0 && a.addend_batch_stride % 8 == 0 &&
-                          a.addend_row_stride % 8 == 0));
-    return ok;
-  };
-  return fits(8) ? 8u : fits(4) ? 4u : 1u;
-}
-
-template <int Epi>
-int launch_small_any(hipStream_t stream, const GemmArgs& a) {
-  switch (small_vec(a)) {
-    case 8: return launch_small<Epi, 8>(stream, a);
-    case 4: return launch_small<Epi, 4>(stream, a);
-    default: return launch_small<Epi, 1>(stream, a);
   }
 }
 
@@ -718,24 +468,23 @@ int epilogue_of(const GemmArgs& a) {
   return a.addend ? kEpiAdd : a.gelu ? kEpiGelu : kEpiPlain;
 }
 
-// Conditions of the LDS-DMA kernels: `unit` 8 for 16-byte aligned operands and
-// rows (N and K, and M when A is transposed, multiples of 8), 2 for dword
-// aligned ones (every row pitch even, any other extent), and 32-bit
-// per-block buffer offsets.
+// Conditions of the LDS-DMA kernels: `unit` 8 for 16-byte aligned operands, C
+// and rows (N and K, and M when A is transposed, multiples of 8), 2 for
+// operands whose addresses and row pitches are multiples of 4 bytes (any C),
+// and 32-bit per-block buffer offsets.
 bool dma_ok(const GemmArgs& a, uint32_t unit) {
   auto at = [&](const void* p) { return (uintptr_t)p % (2 * unit) == 0; };
-  const bool aligned = at(a.left) && at(a.right) && at(a.out) && a.left_batch_stride % unit == 0 &&
-                       a.right_batch_stride % unit == 0;
+  const uint32_t lda = a.transpose_left ? a.rows : a.inner, ldb = a.transpose_right ? a.inner : a.columns;
+  const bool aligned = at(a.left) && at(a.right) && a.left_batch_stride % unit == 0 &&
+                       a.right_batch_stride % unit == 0 && lda % unit == 0 && ldb % unit == 0;
   const uint64_t a_span = a.transpose_left ? (uint64_t)a.inner * a.rows * 2 : 256ull * a.inner * 2;
   const uint64_t b_span = a.transpose_right ? 256ull * a.inner * 2 : (uint64_t)a.inner * a.columns * 2;
   const bool fits = a_span < (1ull << 31) && b_span < (1ull << 31);
-  const uint32_t lda = a.transpose_left ? a.rows : a.inner, ldb = a.transpose_right ? a.inner : a.columns;
-  const bool chunked = unit == 8 ? a.inner % 8 == 0 && a.columns % 8 == 0 && (!a.transpose_left || a.rows % 8 == 0)
-                                 : lda % 2 == 0 && ldb % 2 == 0 && a.columns % 2 == 0;
-  // With 16-byte chunks the add epilogue loads the addend as chunks of 8
-  // columns, otherwise by element.
-  const bool addend_ok = unit != 8 || !a.addend || ((uintptr_t)a.addend % 16 == 0 &&
-                                                   a.addend_batch_stride % 8 == 0 && a.addend_row_stride % 8 == 0);
+  // With 16-byte chunks K ends whole chunks, C is stored in chunks and the add
+  // epilogue loads the addend as chunks of 8 columns, otherwise by element.
+  const bool chunked = unit != 8 || (a.inner % 8 == 0 && a.columns % 8 == 0 && at(a.out));
+  const bool addend_ok = unit != 8 || !a.addend || (at(a.addend) && a.addend_batch_stride % 8 == 0 &&
+                                                   a.addend_row_stride % 8 == 0);
   return aligned && fits && chunked && addend_ok && a.inner > 0;
 }
 bool fast_ok(const GemmArgs& a) { return dma_ok(a, 8); }
@@ -822,23 +571,19 @@ int launch_gemm_f16(hipStream_t stream, const GemmArgs& a) {
   // The LDS-DMA kernels take any M and N: rows past the edge read as 0 and are
   // not stored.  Dword-aligned pitches run them too (kDwords): 4096 x 4096 x
   // 4100 358 -> 108 us against the register-staged kernel.
-  const bool chunks = fast_ok(a);
-  if (chunks || dma_ok(a, 2)) {
-    const uint32_t tile = gemm_f16_tile(a.rows, a.columns, a.inner, a.batches);
-    if (tile != 256) return launch_gemm_f16_tile(stream, a, tile, !chunks);
-    switch (epilogue_of(a)) {
-      case kEpiGelu: return dispatch_fast<kEpiGelu, false>(stream, a, 1, a.inner, !chunks);
-      case kEpiAdd: return dispatch_fast<kEpiAdd, false>(stream, a, 1, a.inner, !chunks);
-      default: return dispatch_fast<kEpiPlain, false>(stream, a, 1, a.inner, !chunks);
-    }
-  }
-  // Any other shape or alignment (or operands past the 256 x 256 kernel's
-  // 31-bit buffer ranges): the small-tile kernel with the widest loads the
-  // operands allow.
+  const GemmAccess access = fast_ok(a) ? GemmAccess::kChunk : dma_ok(a, 2) ? GemmAccess::kDword : GemmAccess::kElement;
+  // Odd pitches or addresses, K = 0 and operands past the buffer ranges go
+  // through registers, in tiles of at most 128 x 128 (us, against a kernel
+  // with one 256-k chunk in flight and 2-byte loads: 4095 x 4097 x 4099 1,505 ->
+  // 285, 2048 x 2047 x 2048 228 -> 33, 1000 x 1001 x 1003 26.8 -> 10, 129 x 129 x 2001
+  // 37 -> 12).
+  const uint32_t tile = gemm_f16_tile(a.rows, a.columns, a.inner, a.batches, access == GemmAccess::kElement ? 128 : 256);
+  if (tile != 256) return launch_gemm_f16_tile(stream, a, tile, access);
+  const bool dwords = access == GemmAccess::kDword;
   switch (epilogue_of(a)) {
-    case kEpiGelu: return launch_small_any<kEpiGelu>(stream, a);
-    case kEpiAdd: return launch_small_any<kEpiAdd>(stream, a);
-    default: return launch_small_any<kEpiPlain>(stream, a);
+    case kEpiGelu: return dispatch_fast<kEpiGelu, false>(stream, a, 1, a.inner, dwords);
+    case kEpiAdd: return dispatch_fast<kEpiAdd, false>(stream, a, 1, a.inner, dwords);
+    default: return dispatch_fast<kEpiPlain, false>(stream, a, 1, a.inner, dwords);
   }
 }
 

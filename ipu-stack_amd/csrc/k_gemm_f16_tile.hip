@@ -28,6 +28,10 @@
 // load per wave (2048^3 21.1 -> 22.1, 729 x 1152 x 4304 on 64 x 64 17.7 ->
 // 20.9), two stages and two workgroups per CU (2048^3 24.9), 128-k steps on 64
 // x 64 tiles (2048^3 33.0 against 27.7).
+//
+// Operands the DMA cannot fetch (odd row pitches or addresses, kElements) take
+// the same kernel with the tiles going through registers: chunks are read at
+// element alignment two steps before they are stored to LDS.
 #include "../../include/ipus.h"
 
 #include <cmath>
@@ -86,7 +90,8 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   constexpr int TM = T::TM, TN = T::TN, BK = T::BK, S = T::S, KG = T::KG;
   constexpr int kMT = T::kMT, kNT = T::kNT, kSub = T::kSub;
   constexpr int kDmaA = T::kDmaA, kDmaB = T::kDmaB;
-  constexpr bool KTail = E != kWhole;
+  constexpr bool KTail = E == kKTail || E == kDwords;
+  constexpr bool kRegs = E == kElements;  // operands through registers, not by DMA
   // Four stages, each a distinct LDS object: the compiler can then see that
   // a DMA into one never aliases the fragment reads of another.
   __shared__ __attribute__((aligned(1024))) uint8_t lds0[T::kStageBytes];
@@ -182,10 +187,53 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
       one.template operator()<kBK_, TN>(b_rsrc, stage + T::kABytes, wave * kDmaB + j, b_voff[j], k * b_kstep);
   };
 
-  dma(lds0, 0);
-  dma(lds1, clamp(1));
-  dma(lds2, clamp(2));
-  dma(lds3, clamp(3));
+  // kElements: this thread's chunks of step k, read at element alignment.  Rows
+  // past M or N repeat the last one and chunks run on into the next row (both
+  // reach only elements of C that are not stored); k past K is zero.
+  auto load_regs = [&](uint32_t k, u32x4 (&v)[kDmaA + kDmaB]) __attribute__((always_inline)) {
+    auto one = [&]<bool KContig, int TMN>(const uint16_t* X, uint32_t inst, uint32_t mn0, uint32_t MN) __attribute__((always_inline)) {
+      uint32_t row, col;
+      chunk_of.template operator()<KContig, TMN>(inst, &row, &col);
+      const uint64_t total = (uint64_t)MN * K, k0 = (uint64_t)k * BK;
+      const u32x4 zero = {0, 0, 0, 0};
+      if constexpr (KContig) {
+        const uint64_t at_k = k0 + col;
+        const uint32_t mn = mn0 + row < MN ? mn0 + row : MN - 1;
+        if (at_k >= K) return zero;
+        const u32x4 x = load_chunk(X, (uint64_t)mn * K + at_k, total);
+        return at_k + 8 <= K ? x : keep_elements(x, (uint32_t)(K - at_k));
+      } else {
+        const uint64_t at_k = k0 + row;
+        return at_k < K && mn0 + col < MN ? load_chunk(X, at_k * MN + mn0 + col, total) : zero;
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < kDmaA; ++j) v[j] = one.template operator()<kAK, TM>(A, wave * kDmaA + j, m0, M);
+#pragma unroll
+    for (int j = 0; j < kDmaB; ++j) v[kDmaA + j] = one.template operator()<kBK_, TN>(B, wave * kDmaB + j, n0, N);
+  };
+  auto store_regs = [&](uint8_t* stage, const u32x4 (&v)[kDmaA + kDmaB]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kDmaA; ++j)
+      *reinterpret_cast<u32x4*>(stage + (wave * kDmaA + j) * 1024 + lane * 16) = v[j];
+#pragma unroll
+    for (int j = 0; j < kDmaB; ++j)
+      *reinterpret_cast<u32x4*>(stage + T::kABytes + (wave * kDmaB + j) * 1024 + lane * 16) = v[kDmaA + j];
+  };
+  u32x4 regs[2][kRegs ? kDmaA + kDmaB : 1];
+  if constexpr (kRegs) {
+    load_regs(0, regs[0]);
+    load_regs(1, regs[1]);
+    store_regs(lds0, regs[0]);
+    store_regs(lds1, regs[1]);
+    load_regs(2, regs[0]);
+    load_regs(3, regs[1]);
+  } else {
+    dma(lds0, 0);
+    dma(lds1, clamp(1));
+    dma(lds2, clamp(2));
+    dma(lds3, clamp(3));
+  }
 
   auto k_base = [&](uint32_t w0) { return (w0 + r16) * 128 + ((g4 ^ (r16 & 7)) << 4); };
   auto m_base = [&]<int RB>(uint32_t w0) {
@@ -240,7 +288,8 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
 
   constexpr int kDma = T::kDma;
   constexpr int kMfma = kSub * kMT * kNT, kReads = kSub * kItems;
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * kDma) : "memory");
+  if constexpr (kRegs) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * kDma) : "memory");
   if (E == kDwords && ksteps == 1) clear_past_k(lds0);
 #pragma unroll
   for (int r = 0; r < kReads; ++r) read_item(lds0, 0, r);
@@ -248,11 +297,21 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   // every wave's DMA of stage kt + 1 (`next`) has landed and every wave's
   // reads of stage kt (`cur`) have returned, so cur takes the DMA of step
   // kt + 4 and next is read between the MFMAs.
-  auto step = [&](uint8_t* cur, uint8_t* next, int buf, uint32_t kt) __attribute__((always_inline)) {
+  // kElements: the step stores the chunks of step kt + 2, loaded two steps ago,
+  // into their stage (`ahead`, last read in step kt - 2) and loads those of
+  // step kt + 4; the barrier publishes the stores of the step before.
+  auto step = [&](uint8_t* cur, uint8_t* next, uint8_t* ahead, int buf, uint32_t kt) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * kDma) : "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    dma(cur, clamp(kt + S));
+    if constexpr (kRegs) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      store_regs(ahead, regs[buf]);
+      load_regs(kt + S, regs[buf]);
+    } else {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * kDma) : "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      dma(cur, clamp(kt + S));
+    }
     if (E == kDwords && kt + 2 == ksteps) clear_past_k(next);
     __builtin_amdgcn_sched_barrier(0);
     int r = 0;
@@ -270,14 +329,14 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   };
   uint32_t kt = 0;
   for (; kt + 3 < ksteps; kt += 4) {
-    step(lds0, lds1, 0, kt);
-    step(lds1, lds2, 1, kt + 1);
-    step(lds2, lds3, 0, kt + 2);
-    step(lds3, lds0, 1, kt + 3);
+    step(lds0, lds1, lds2, 0, kt);
+    step(lds1, lds2, lds3, 1, kt + 1);
+    step(lds2, lds3, lds0, 0, kt + 2);
+    step(lds3, lds0, lds1, 1, kt + 3);
   }
-  if (kt < ksteps) step(lds0, lds1, 0, kt);
-  if (kt + 1 < ksteps) step(lds1, lds2, 1, kt + 1);
-  if (kt + 2 < ksteps) step(lds2, lds3, 0, kt + 2);
+  if (kt < ksteps) step(lds0, lds1, lds2, 0, kt);
+  if (kt + 1 < ksteps) step(lds1, lds2, lds3, 1, kt + 1);
+  if (kt + 2 < ksteps) step(lds2, lds3, lds0, 0, kt + 2);
   // The redundant prefetches have landed and every wave is done with the stages.
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
@@ -331,23 +390,23 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
     if (v >= 16 * kRowsT * kRC) break;  // 32 x 32 tiles: half a wave's lanes store
     u32x4 x = *reinterpret_cast<const u32x4*>(cst + r * kRB + ((c ^ (r & (kRC - 1))) << 4));
     // Rows past M and columns past N are not stored (N % 8 == 0 except with
-    // kDwords).  out may be the addend: the same lane reads each chunk and then
+    // kDwords and kElements).  out may be the addend: the same lane reads each chunk and then
     // writes it.
     if (row0 + r < M && col0 + c * 8 < N) {
       const uint64_t at = (uint64_t)(row0 + r) * N + col0 + c * 8;
       const uint32_t valid = N - (col0 + c * 8);
       if constexpr (Epi == kEpiAdd) {
         const uint16_t* d = addend + batch * addend_batch_stride + (uint64_t)(row0 + r) * addend_row_stride + col0 + c * 8;
-        x = add_f16x8(x, E == kDwords ? load_elements(d, valid) : *reinterpret_cast<const u32x4*>(d));
+        x = add_f16x8(x, E >= kDwords ? load_elements(d, valid) : *reinterpret_cast<const u32x4*>(d));
       }
-      if constexpr (E == kDwords) store_dwords(C + at, x, valid);
+      if constexpr (E >= kDwords) store_elements(C + at, x, valid);
       else *reinterpret_cast<u32x4*>(C + at) = x;
     }
   }
 }
 
 template <class T, int Epi>
-int launch_tile(hipStream_t stream, const GemmArgs& a, bool dwords) {
+int launch_tile(hipStream_t stream, const GemmArgs& a, GemmAccess access) {
   const uint64_t tiles = (uint64_t)((a.rows + T::TM - 1) / T::TM) * ((a.columns + T::TN - 1) / T::TN);
   if (tiles > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
   auto go = [&](auto kernel) {
@@ -363,17 +422,18 @@ int launch_tile(hipStream_t stream, const GemmArgs& a, bool dwords) {
     else if (!tr) go(gemm_f16_tile_kernel<T, true, false, Epi, E>);
     else go(gemm_f16_tile_kernel<T, true, true, Epi, E>);
   };
-  if (dwords) layouts.template operator()<kDwords>();
+  if (access == GemmAccess::kElement) layouts.template operator()<kElements>();
+  else if (access == GemmAccess::kDword) layouts.template operator()<kDwords>();
   else if (a.inner % T::BK == 0) layouts.template operator()<kWhole>();
   else layouts.template operator()<kKTail>();
   return hip_status(hipGetLastError());
 }
 
 template <class T>
-int launch_epilogue(hipStream_t stream, const GemmArgs& a, bool dwords) {
-  if (a.addend) return launch_tile<T, kEpiAdd>(stream, a, dwords);
-  if (a.gelu) return launch_tile<T, kEpiGelu>(stream, a, dwords);
-  return launch_tile<T, kEpiPlain>(stream, a, dwords);
+int launch_epilogue(hipStream_t stream, const GemmArgs& a, GemmAccess access) {
+  if (a.addend) return launch_tile<T, kEpiAdd>(stream, a, access);
+  if (a.gelu) return launch_tile<T, kEpiGelu>(stream, a, access);
+  return launch_tile<T, kEpiPlain>(stream, a, access);
 }
 
 }  // namespace
@@ -387,22 +447,23 @@ int launch_epilogue(hipStream_t stream, const GemmArgs& a, bool dwords) {
 // 128 9.4, 32 x 32 9.2; 128 x 4096 x 4096 64 x 64 15.8, 32 x 32 18.3.  The choice
 // does not depend on the epilogue, so a fused epilogue gives the bits of the
 // separate kernels.
-uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches) {
+uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches, uint32_t largest) {
   struct Class {
     uint32_t tile;
     double start_us, step_us;
   };
   constexpr Class kClasses[] = {{256, 7.0, 1.35}, {128, 5.0, 0.50}, {64, 3.0, 0.19}, {32, 2.4, 0.10}};
   const uint64_t steps = ((uint64_t)inner + 63) / 64;
-  uint32_t best = 256;
+  uint32_t best = 0;
   double best_us = 0;
   for (const Class& c : kClasses) {
+    if (c.tile > largest) continue;
     const uint64_t m = ((uint64_t)rows + c.tile - 1) / c.tile, n = ((uint64_t)columns + c.tile - 1) / c.tile;
     const double tiles = (double)m * (double)n * (double)batches;
     // Two workgroups of the smaller tiles share a CU.
     const double rounds = tiles <= 256 ? 1.0 : c.tile >= 128 ? std::ceil(tiles / 256) : 2.0 * std::ceil(tiles / 512);
     const double us = c.start_us + rounds * (double)steps * c.step_us;
-    if (c.tile == 256 || us < best_us) {
+    if (best == 0 || us < best_us) {
       best = c.tile;
       best_us = us;
     }
@@ -410,10 +471,10 @@ uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t
   return best;
 }
 
-int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, bool dwords) {
-  if (tile == 128) return launch_epilogue<Tile128>(stream, a, dwords);
-  if (tile == 64) return launch_epilogue<Tile64>(stream, a, dwords);
-  return launch_epilogue<Tile32>(stream, a, dwords);
+int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, GemmAccess access) {
+  if (tile == 128) return launch_epilogue<Tile128>(stream, a, access);
+  if (tile == 64) return launch_epilogue<Tile64>(stream, a, access);
+  return launch_epilogue<Tile32>(stream, a, access);
 }
 
 }  // namespace ipus

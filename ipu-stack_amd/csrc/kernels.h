@@ -66,10 +66,13 @@ struct AttentionArgs {
 int launch_gemm_f16(hipStream_t stream, const GemmArgs& a);
 // Tile edge (256, 128, 64 or 32) for an fp16 product that meets the LDS-DMA
 // kernels' conditions; the smaller ones are launched by launch_gemm_f16_tile
-// (k_gemm_f16_tile.hip), which does not check those conditions again.  dwords:
-// pitches and addresses are multiples of 4 bytes, not of 16.
-uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches);
-int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, bool dwords);
+// (k_gemm_f16_tile.hip), which does not check those conditions again.  access:
+// what every row pitch and address of the operands allows; kElement also
+// takes K = 0 and operands past the DMA's buffer ranges.
+uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches,
+                       uint32_t largest);
+enum class GemmAccess { kChunk, kDword, kElement };  // 16, 4, 2 bytes
+int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, GemmAccess access);
 // Split-K: fp32 partials float[splits][batches][M][N] into a.out (a.gelu must
 // be false), then launch_reduce_splits_f16 to fp16.  gemm_f16_split_chunk
 // gives the k range per split (a multiple of 64); the plan picks splits so

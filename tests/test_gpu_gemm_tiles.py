@@ -129,32 +129,54 @@ def test_gemm_f32_tiles_batched(ipus, ctx):
 @pytest.mark.parametrize("tl,tr", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_gemm_f16_dword_aligned_pitches(ipus, oracle, ctx, M, N, K, tl, tr):
     """Row pitches that are even but no multiple of 8, at 4-byte-aligned
-    addresses; NaN after both operands, so that an element read from past
+    addresses."""
+    check_unaligned(ipus, oracle, ctx, M, N, K, tl, tr, 2)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1801, 2057, 585),    # tile 128
+    (521, 1161, 1155),    # tile 64
+    (41, 73, 265), (1, 1, 1), (33, 4097, 61), (257, 263, 129), (64, 64, 192)])  # tile 32
+@pytest.mark.parametrize("tl,tr", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_f16_odd_pitches(ipus, oracle, ctx, M, N, K, tl, tr):
+    """Odd row pitches, or any at 2-byte-aligned addresses."""
+    check_unaligned(ipus, oracle, ctx, M, N, K, tl, tr, 1)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 5001, 768), (1030, 777, 1090), (130, 67, 64)])
+def test_gemm_f16_odd_output_rows(ipus, oracle, ctx, M, N, K):
+    """Dword-aligned operands (the right one transposed), C with odd rows."""
+    check_unaligned(ipus, oracle, ctx, M, N, K, 0, 1, 2)
+
+
+def check_unaligned(ipus, oracle, ctx, M, N, K, tl, tr, shift_elements):
+    """Operands and output `shift_elements` into their allocations; NaN after both operands, so that an element read from past
     them (rather than masked or cleared) shows.  Rows at both ends and
     sampled between are checked, and nothing is stored past C."""
     a = ipus.synth_f16(M * K, 79, 1, 0, 1.0)
     b = ipus.synth_f16(K * N, 79, 2, 0, 1.0)
-    shift = np.zeros(2, np.uint16)
+    at = shift_elements
+    shift = np.zeros(at, np.uint16)
     pad = np.full(64 * max(M, N, K), 0x7E00, np.uint16)
     da, db = (ctx.upload(np.concatenate([shift, x, pad])) for x in (a, b))
     out = ctx.upload(np.full(M * N + 16, 0x7E00, np.uint16))
     sc = [1, M, N, K, tl, tr, 0, 0]
-    ctx.launch("ipu_stack_gemm_f16", out.ptr + 4, [da.ptr + 4, db.ptr + 4], sc)
+    ctx.launch("ipu_stack_gemm_f16", out.ptr + 2 * at, [da.ptr + 2 * at, db.ptr + 2 * at], sc)
     raw = out.download(np.uint16)
-    assert np.all(raw[:2] == 0x7E00) and np.all(raw[2 + M * N:] == 0x7E00)
+    assert np.all(raw[:at] == 0x7E00) and np.all(raw[at + M * N:] == 0x7E00)
     rows = np.unique(np.concatenate([np.arange(min(M, 20)), np.arange(max(0, M - 20), M),
                                      np.random.default_rng(3).integers(0, M, 40)]))
     af = oracle.f16_to_f32(a).astype(np.float64).reshape((K, M) if tl else (M, K))
     bf = oracle.f16_to_f32(b).astype(np.float64).reshape((N, K) if tr else (K, N))
     af, bf = (af.T if tl else af)[rows], bf.T if tr else bf
-    got = oracle.f16_to_f32(raw[2:2 + M * N]).reshape(M, N)
+    got = oracle.f16_to_f32(raw[at:at + M * N]).reshape(M, N)
     assert_product(got[rows], af, bf, K)
     # The add epilogue, its addend (any alignment) read by element
     d = ctx.upload(np.concatenate([np.zeros(1, np.uint16), ipus.synth_f16(M * N, 79, 3, 0, 1.0)]))
     want = ctx.alloc(M * N * 2)
     fused = ctx.alloc(M * N * 2)
-    ctx.launch("ipu_stack_add_f16", want, [out.ptr + 4, d.ptr + 2], [M * N, M * N, M * N])
-    ctx.launch("ipu_stack_gemm_f16_accumulate", fused, [da.ptr + 4, db.ptr + 4, d.ptr + 2],
+    ctx.launch("ipu_stack_add_f16", want, [out.ptr + 2 * at, d.ptr + 2], [M * N, M * N, M * N])
+    ctx.launch("ipu_stack_gemm_f16_accumulate", fused, [da.ptr + 2 * at, db.ptr + 2 * at, d.ptr + 2],
                sc + [0, N])
     assert np.array_equal(fused.download(np.uint16), want.download(np.uint16))
     for x in (da, db, d, out, want, fused):
