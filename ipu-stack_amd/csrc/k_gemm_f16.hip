@@ -565,9 +565,24 @@ int launch_reduce_splits_f16(hipStream_t stream, void* dst, const void* parts, u
   return hip_status(hipGetLastError());
 }
 
-int launch_gemm_f16(hipStream_t stream, const GemmArgs& a) {
+int launch_gemm_f16(hipStream_t stream, const GemmArgs& args) {
+  GemmArgs a = args;
   if (a.batches == 0 || a.rows == 0 || a.columns == 0) return 0;
   if (a.batches > 65535 || (a.gelu && a.addend)) return IPUS_ERROR_INVALID_ARGUMENT;
+  // Batches that follow each other in memory and share the right operand (x .
+  // W over [batch, rows, width]) are one product of batches * rows rows: no
+  // partial tile per batch.  The tile is chosen for that product also where
+  // the addend does not follow the same rows, so that the sums (and the bits)
+  // do not depend on the epilogue.
+  const uint64_t rows = (uint64_t)a.batches * a.rows;
+  const bool shared = a.batches > 1 && !a.transpose_left && a.right_batch_stride == 0 &&
+                      a.left_batch_stride == (uint64_t)a.rows * a.inner && rows <= 0xffffffffull;
+  if (shared && (!a.addend || a.addend_batch_stride == (uint64_t)a.rows * a.addend_row_stride)) {
+    a.rows = (uint32_t)rows;
+    a.batches = 1;
+    a.left_batch_stride = 0;
+    a.addend_batch_stride = 0;
+  }
   // The LDS-DMA kernels take any M and N: rows past the edge read as 0 and are
   // not stored.  Dword-aligned pitches run them too (kDwords): 4096 x 4096 x
   // 4100 358 -> 108 us against the register-staged kernel.
@@ -577,7 +592,8 @@ int launch_gemm_f16(hipStream_t stream, const GemmArgs& a) {
   // with one 256-k chunk in flight and 2-byte loads: 4095 x 4097 x 4099 1,505 ->
   // 285, 2048 x 2047 x 2048 228 -> 33, 1000 x 1001 x 1003 26.8 -> 10, 129 x 129 x 2001
   // 37 -> 12).
-  const uint32_t tile = gemm_f16_tile(a.rows, a.columns, a.inner, a.batches, access == GemmAccess::kElement ? 128 : 256);
+  const uint32_t tile = gemm_f16_tile(shared ? (uint32_t)rows : a.rows, a.columns, a.inner,
+                                      shared ? 1 : a.batches, access == GemmAccess::kElement ? 128 : 256);
   if (tile != 256) return launch_gemm_f16_tile(stream, a, tile, access);
   const bool dwords = access == GemmAccess::kDword;
   switch (epilogue_of(a)) {

@@ -79,6 +79,33 @@ def test_gemm_f16_tiles_batches_and_epilogues(ipus, oracle, ctx, M, N, K, shared
         assert np.array_equal(d.download(np.uint16), want.download(np.uint16))
 
 
+@pytest.mark.parametrize("B,M,N,K", [(5, 141, 1032, 584), (2, 700, 1280, 1160), (7, 9, 73, 66)])
+@pytest.mark.parametrize("addend", ["none", "full", "matrix", "rows"])
+def test_gemm_f16_batches_as_rows(ipus, oracle, ctx, B, M, N, K, addend):
+    """Contiguous batches that share the right operand run as one product of
+    B M rows; an addend per matrix (which cannot) gives the same sums."""
+    a, b, af, bf = operands(ipus, oracle, M, N, K, 0, 0, B, True)
+    n = B * M * N
+    da, db, out = ctx.upload(a), ctx.upload(b), ctx.upload(np.full(n + 8, 0x7E00, np.uint16))
+    sc = [B, M, N, K, 0, 0, M * K, 0]
+    ctx.launch("ipu_stack_gemm_f16", out, [da, db], sc)
+    raw = out.download(np.uint16)
+    assert np.all(raw[n:] == 0x7E00)
+    if addend == "none":
+        assert_product(oracle.f16_to_f32(raw[:n]).reshape(B, M, N), af, bf, K)
+        # the same bits as each batch's rows of one 2-D product
+        one = ctx.alloc(n * 2)
+        ctx.launch("ipu_stack_gemm_f16", one, [da, db], [1, B * M, N, K, 0, 0, 0, 0])
+        assert np.array_equal(one.download(np.uint16), raw[:n])
+    else:
+        count, strides = {"full": (n, [M * N, N]), "matrix": (M * N, [0, N]), "rows": (N, [0, 0])}[addend]
+        d = ctx.upload(ipus.synth_f16(count, 71, 3, 0, 1.0))
+        want, got = ctx.alloc(n * 2), ctx.alloc(n * 2)
+        ctx.launch("ipu_stack_add_f16", want, [out, d], [n, n, count])
+        ctx.launch("ipu_stack_gemm_f16_accumulate", got, [da, db, d], sc + strides)
+        assert np.array_equal(got.download(np.uint16), want.download(np.uint16))
+
+
 @pytest.mark.parametrize("M,N,K", [
     # 64 x 64 tiles: partial tiles, a partial last step, one step
     (1000, 1004, 1000), (520, 1160, 72), (1024, 1024, 32),
