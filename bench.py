@@ -424,7 +424,8 @@ def cpu_configs(ipus, oracle, threads):
 # summary, used only when it was measured on the current kernel sources.
 # ---------------------------------------------------------------------------
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "gemm_f16_8192_traffic.json")
-GEMM_SOURCES = ("ipu-stack_amd/csrc/k_gemm_f16.hip", "ipu-stack_amd/csrc/device_common.h")
+GEMM_SOURCES = ("ipu-stack_amd/csrc/k_gemm_f16.hip", "ipu-stack_amd/csrc/gemm_common.h",
+                "ipu-stack_amd/csrc/device_common.h")
 
 
 def source_digest(paths=GEMM_SOURCES) -> str:

@@ -19,7 +19,9 @@
  *
  * Conventions (kernel.rs:14-16, crates/ipu-codegen/src/operator.rs:467-537):
  *   - The caller owns every buffer.  Kernels read inputs and write the output
- *     and allocate nothing.
+ *     and allocate nothing.  A context holds 32 MiB of device memory of its
+ *     own for launches that merge partial results (allocated with it, outside
+ *     ipus_context_live_buffers).
  *   - Launches are ordered on the context's stream (replacing BSP phases).
  *   - Every call returns 0 on success or a negative IPUS_ERROR_* code;
  *     ipus_last_error() returns the message of the calling thread's last
