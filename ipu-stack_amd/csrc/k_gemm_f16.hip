@@ -232,18 +232,22 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_256_kernel(
     for (int j = 0; j < 8; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
   const uint32_t ksteps = (k_len + BK - 1) / BK;
-  // K-contiguous operands mask the chunks past K on the last step (MN-
-  // contiguous rows past K are past the buffer's range).
+  // Chunks and rows past K on the last step are masked (issue_one).
   const uint32_t k_tail = k_len % BK;  // nonzero only on the last split
   auto clamp = [&](uint32_t k) { return k < ksteps ? k : ksteps - 1; };
   // KTail (K % BK != 0) is a separate instantiation, so the tail test never
   // enters the K loop of the common case.
   auto limit = [&](uint32_t k) { return KTail && k == ksteps - 1 ? k_tail : 0u; };
+  // kDwords: on the last step a chunk can run past the operand's end, so the
+  // step's offset moves into the vector offset, which the range check covers.
+  auto in_vector = [&](uint32_t k) { return E == kDwords && k == ksteps - 1; };
   auto dma_a = [&](uint8_t* ta, uint32_t k, uint32_t j) __attribute__((always_inline)) {
-    issue_one<BK, kAK>(a_rsrc, ta, wave, lane, a_voff[j], j, k * a_kstep, limit(k));
+    const uint32_t at = k * a_kstep, v = in_vector(k) ? at : 0u;
+    issue_one<BK, kAK>(a_rsrc, ta, wave, lane, a_voff[j] + v, j, at - v, limit(k));
   };
   auto dma_b = [&](uint8_t* tb, uint32_t k, uint32_t j) __attribute__((always_inline)) {
-    issue_one<BK, kBK_>(b_rsrc, tb, wave, lane, b_voff[j], j, k * b_kstep, limit(k));
+    const uint32_t at = k * b_kstep, v = in_vector(k) ? at : 0u;
+    issue_one<BK, kBK_>(b_rsrc, tb, wave, lane, b_voff[j] + v, j, at - v, limit(k));
   };
   auto fetch = [&](uint8_t* ta, uint8_t* tb, uint32_t k) __attribute__((always_inline)) {
 #pragma unroll

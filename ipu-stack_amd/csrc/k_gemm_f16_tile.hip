@@ -177,7 +177,10 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
         chunk_of.template operator()<KContig, TMN>(inst, &row, &col);
         voff = (KContig ? col : row) < limit ? voff : kPadOffset;
       }
-      dma16(rsrc, tile + inst * 1024, voff, soff);
+      // kDwords: on the last step a chunk can run past the operand's end, so the
+      // step's offset moves into the vector offset, which the range check covers.
+      const uint32_t v = E == kDwords && k == ksteps - 1 ? soff : 0u;
+      dma16(rsrc, tile + inst * 1024, voff + v, soff - v);
     };
 #pragma unroll
     for (int j = 0; j < kDmaA; ++j)
