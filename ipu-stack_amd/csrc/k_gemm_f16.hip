@@ -580,7 +580,7 @@ int launch_gemm_f16(hipStream_t stream, const GemmArgs& args) {
   // do not depend on the epilogue.
   const uint64_t rows = (uint64_t)a.batches * a.rows;
   const bool shared = a.batches > 1 && !a.transpose_left && a.right_batch_stride == 0 &&
-                      a.left_batch_stride == (uint64_t)a.rows * a.inner && rows <= 0xffffffffull;
+                      a.left_batch_stride == (uint64_t)a.rows * a.inner && rows <= 0x7fffffffull;
   if (shared && (!a.addend || a.addend_batch_stride == (uint64_t)a.rows * a.addend_row_stride)) {
     a.rows = (uint32_t)rows;
     a.batches = 1;

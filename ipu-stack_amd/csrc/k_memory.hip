@@ -74,7 +74,7 @@ __device__ __forceinline__ void store16_nt(void* p, u32x4 v) {
 typedef u32x4 __attribute__((aligned(2))) u32x4_elements;
 // Elements c .. c + 7 of a row of `limit` elements, zero past it.
 __device__ __forceinline__ u32x4 load_row8(const uint16_t* row, uint32_t c, uint32_t limit) {
-  if (c + 8 <= limit) return *reinterpret_cast<const u32x4_elements*>(row + c);
+  if (c < limit && limit - c >= 8) return *reinterpret_cast<const u32x4_elements*>(row + c);
   u32x4 v = {0, 0, 0, 0};
 #pragma unroll
   for (uint32_t e = 0; e < 8; ++e)
@@ -82,7 +82,7 @@ __device__ __forceinline__ u32x4 load_row8(const uint16_t* row, uint32_t c, uint
   return v;
 }
 __device__ __forceinline__ void store_row8(uint16_t* row, uint32_t c, uint32_t limit, u32x4 v) {
-  if (c + 8 <= limit) {
+  if (c < limit && limit - c >= 8) {
     *reinterpret_cast<u32x4_elements*>(row + c) = v;
     return;
   }
