@@ -609,8 +609,8 @@ int build_error(const std::string& message) {
 // 64 / tiles), i.e. only for outputs of at most 32 tiles and K >= 6144, with
 // every split keeping >= 1024 k and about 64 workgroups in all.  The line was
 // measured against the unsplit kernel that the tile kernel replaced; today
-// (us, unsplit against split) 256 x 1024 x 16384 43 / 37 and 64 x 64 x 40000 70 /
-// 51 keep the split ahead, 256 x 256 x 8192 20 / 32 and 1024 x 1024 x 8192 29 / 51 do
+// (us, unsplit against split) 256 x 1024 x 16384 43 / 37 keeps the split ahead, 64 x
+// 64 x 40000 13 / 51, 256 x 256 x 8192 11 / 32 and 1024 x 1024 x 8192 29 / 51 do
 // not: callers see the plan's steps, so it stays.  Returns 1 (no split)
 // when the shape is outside the fast kernel's reach.
 uint32_t gemm_splits(uint32_t M, uint32_t N, uint32_t K, uint64_t batches, bool tl, bool tr) {

@@ -596,9 +596,10 @@ int launch_gemm_f16(hipStream_t stream, const GemmArgs& args) {
   // with one 256-k chunk in flight and 2-byte loads: 4095 x 4097 x 4099 1,505 ->
   // 285, 2048 x 2047 x 2048 228 -> 33, 1000 x 1001 x 1003 26.8 -> 10, 129 x 129 x 2001
   // 37 -> 12).
-  const uint32_t tile = gemm_f16_tile(shared ? (uint32_t)rows : a.rows, a.columns, a.inner,
-                                      shared ? 1 : a.batches, access == GemmAccess::kElement ? 128 : 256);
-  if (tile != 256) return launch_gemm_f16_tile(stream, a, tile, access);
+  const uint32_t plan_rows = shared ? (uint32_t)rows : a.rows, plan_batches = shared ? 1 : a.batches;
+  const uint32_t tile = gemm_f16_tile(plan_rows, a.columns, a.inner, plan_batches,
+                                      access == GemmAccess::kElement ? 128 : 256);
+  if (tile != 256) return launch_gemm_f16_tile(stream, a, tile, access, plan_rows, plan_batches);
   const bool dwords = access == GemmAccess::kDword;
   switch (epilogue_of(a)) {
     case kEpiGelu: return dispatch_fast<kEpiGelu, false>(stream, a, 1, a.inner, dwords);

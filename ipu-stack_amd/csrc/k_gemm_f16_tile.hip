@@ -19,6 +19,8 @@
 //     cover each other's waits with the same LDS reads as four waves (128 x
 //     128, 2048^3: 21.6 -> 21.1 us, 1024^3 11.1 -> 9.4, 729 x 4304 x 1152 13.0
 //     -> 11.8); the groups' fp32 sums are added through LDS at the end;
+//   * few 32 x 32 tiles with a long K split K over workgroups, and the last one
+//     adds the partial sums in the order of K (split_plan);
 //   * C leaves through LDS in whole row runs, as in the 256 x 256 kernel.
 // Measured, us per launch, before (256 x 256 kernel or the register-staged
 // small-tile kernel) and now: 2048^3 38.0 -> 21.1 (128 x 128), 729 x 4304 x
@@ -65,6 +67,14 @@ typedef TileShape<128, 128, 64, 64, 2, 64> Tile128;
 typedef TileShape<64, 64, 32, 32, 2, 64> Tile64;
 typedef TileShape<32, 32, 16, 16, 1, 128> Tile32;
 
+// Split launches: workgroup (x, y, z) takes k in [z * chunk, (z + 1) * chunk)
+// of its tile; every split holds at least one k.
+struct SplitK {
+  float* parts = nullptr;        // [batches * tiles][splits][fragments][threads][4]
+  uint32_t* counters = nullptr;  // one per tile, all 0 between launches
+  uint32_t splits = 1, chunk = 0;  // chunk: a multiple of the K step
+};
+
 // LDS tiles.  K-contiguous operand: subtiles of 64 k, each [rows][64 k] with
 // the 16-byte chunk XORed by row & 7.  MN-contiguous: [k][mn], the chunk XORed
 // by mn_swz(k).  A fragment read (ds_read_b64_tr_b16) takes 32 bytes of the 16
@@ -82,11 +92,13 @@ __device__ __forceinline__ uint32_t mn_swz(uint32_t k) {
     return ((k >> 3) & 1u) << 1;
 }
 
-template <class T, bool TransposeLeft, bool TransposeRight, int Epi, int E>
+template <class T, bool TransposeLeft, bool TransposeRight, int Epi, int E, bool Split>
 __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
     uint16_t* out, const uint16_t* __restrict__ left, const uint16_t* __restrict__ right,
     uint32_t M, uint32_t N, uint32_t K, uint64_t left_batch_stride, uint64_t right_batch_stride,
-    const uint16_t* addend, uint64_t addend_batch_stride, uint32_t addend_row_stride) {
+    const uint16_t* addend, uint64_t addend_batch_stride, uint32_t addend_row_stride,
+    SplitK split) {
+  static_assert(!Split || (T::KG == 1 && E != kElements), "splits: one K group, operands by DMA");
   constexpr int TM = T::TM, TN = T::TN, BK = T::BK, S = T::S, KG = T::KG;
   constexpr int kMT = T::kMT, kNT = T::kNT, kSub = T::kSub;
   constexpr int kDmaA = T::kDmaA, kDmaB = T::kDmaB;
@@ -119,8 +131,11 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   const uint16_t* A = left + batch * left_batch_stride;
   const uint16_t* B = right + batch * right_batch_stride;
   uint16_t* C = out + batch * (uint64_t)M * N;
-  const uint16_t* a_base = kAK ? A + (uint64_t)m0 * K : A + m0;
-  const uint16_t* b_base = kBK_ ? B + (uint64_t)n0 * K : B + n0;
+  // This workgroup's K range (the whole of K unless Split).
+  const uint32_t k_begin = Split ? blockIdx.z * split.chunk : 0;
+  const uint32_t k_len = Split ? (K - k_begin < split.chunk ? K - k_begin : split.chunk) : K;
+  const uint16_t* a_base = kAK ? A + (uint64_t)m0 * K + k_begin : A + m0 + (uint64_t)k_begin * M;
+  const uint16_t* b_base = kBK_ ? B + (uint64_t)n0 * K + k_begin : B + n0 + (uint64_t)k_begin * N;
   const uint64_t a_bytes = (uint64_t)M * K * 2 - (uint64_t)(a_base - A) * 2;
   const uint64_t b_bytes = (uint64_t)N * K * 2 - (uint64_t)(b_base - B) * 2;
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -161,8 +176,8 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   const uint32_t a_kstep = kAK ? BK * 2 : BK * M * 2;
   const uint32_t b_kstep = kBK_ ? BK * 2 : BK * N * 2;
 
-  const uint32_t ksteps = (K + BK - 1) / BK;
-  const uint32_t k_tail = K % BK;
+  const uint32_t ksteps = (k_len + BK - 1) / BK;
+  const uint32_t k_tail = k_len % BK;
   auto clamp = [&](uint32_t k) { return k < ksteps ? k : ksteps - 1; };
   // The DMA of step k into a stage.  Past the last step it fetches the last
   // one again (a stage that is never read), so the wait counts stay exact.
@@ -367,6 +382,39 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
         acc[i][j] += *reinterpret_cast<const float4_t*>(theirs + ((i % kRowsT) * kNT + j) * 1024 + lane * 16);
     }
   }
+  if constexpr (Split) {
+    // Every split leaves its sums (one 16-byte slot per thread and fragment);
+    // the last one adds all of them, in the order of K.
+    const uint64_t tile_at = batch * tiles + pid;
+    const uint64_t slots = (uint64_t)T::kThreads * kMT * kNT;
+    float* part = split.parts + (tile_at * split.splits * slots + threadIdx.x) * 4;
+    auto slot = [&](uint32_t z, int i, int j) { return part + (z * slots + (uint64_t)(i * kNT + j) * T::kThreads) * 4; };
+#pragma unroll
+    for (int i = 0; i < kMT; ++i)
+#pragma unroll
+      for (int j = 0; j < kNT; ++j)
+        if (m0 + wm + 16 * i + r16 < M) store_device4(slot(blockIdx.z, i, j), acc[i][j]);
+    __shared__ uint32_t arrived;
+    if (!arrive(split.counters + tile_at, split.splits, &arrived)) return;
+#pragma unroll
+    for (int i = 0; i < kMT; ++i) {
+#pragma unroll
+      for (int j = 0; j < kNT; ++j) {
+        acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        if (m0 + wm + 16 * i + r16 >= M) continue;
+        // Eight loads in flight (past the last split: the last one again, not added).
+        for (uint32_t z0 = 0; z0 < split.splits; z0 += 8) {
+          float4_t x[8];
+#pragma unroll
+          for (uint32_t u = 0; u < 8; ++u)
+            x[u] = load_device4(slot(z0 + u < split.splits ? z0 + u : split.splits - 1, i, j));
+#pragma unroll
+          for (uint32_t u = 0; u < 8; ++u)
+            if (z0 + u < split.splits) acc[i][j] += x[u];
+        }
+      }
+    }
+  }
   // The wave's rows go out through its own slot of LDS as whole runs of
   // 2 * WN bytes: row r, 16-byte chunk c at chunk c ^ (r & (chunks - 1)).
   constexpr uint32_t kRB = 2 * T::WN, kRC = kRB / 16;
@@ -408,23 +456,71 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   }
 }
 
+// K splits for at most 128 tiles of 32 x 32 (decode projections, small products
+// with a long K), where the walk over K of few workgroups leaves CUs and memory
+// idle: at most one workgroup per CU and 8 splits.  Modelled time, us: 0.25 per
+// 128-k step (0.2 from L2, 0.28-0.49 from HBM), and for a split launch 2 for the
+// partial sums, the count and the merge, 0.1 per split and 1.1 per MB of
+// partial sums.  Measured, unsplit and at this choice, weights in HBM: 8 x 4096 x
+// 4096 18.0 -> 13.4 (4 splits 13.9; transposed weights 10.6 -> 10.1), 8 x 2048 x 8192
+// 31.6 -> 13.1 (8 splits 13.4), 16 x 1024 x 4096 11.5 -> 6.8, 8 x 512 x 8192 19.9 ->
+// 7.1, 64 x 64 x 8192 15.5 -> 6.3, 256 x 256 x 4096 10.2 -> 7.4, 8 x 1024 x 2048 6.9 -> 5.8.
+// Not worth it: 320 x 320 x 2000 5.5 -> 6.6, 64 x 2048 x 2048 6.8 -> 7.0, 8 x 4096 x
+// 1024 4.7 -> 6.0.
+// The plan is made for plan_tiles, the tiles of the folded product where the
+// batches could be folded (launch_gemm_f16), so that it does not depend on the
+// epilogue; `launched` tiles (at most 32 per folded one) use the workspace.
+bool split_plan(const GemmArgs& a, uint64_t plan_tiles, uint64_t launched, uint32_t step, SplitK* s) {
+  if (!a.workspace.data || plan_tiles > 128 || launched > a.workspace.counter_count) return false;
+  const uint32_t steps = (a.inner + step - 1) / step;
+  constexpr uint64_t kTileBytes = 32 * 32 * sizeof(float);
+  const uint64_t rows = (uint64_t)a.rows * a.batches;
+  const double stored = (double)plan_tiles * (rows < 32 ? rows : 32) * 32 * sizeof(float);
+  double best_us = steps * 0.25;
+  uint32_t best = 1;
+  for (uint32_t want = 2; want <= 8 && want * plan_tiles <= 256 && want * 2 <= steps; ++want) {
+    const uint32_t per = (steps + want - 1) / want, splits = (steps + per - 1) / per;
+    if (launched * splits * kTileBytes > a.workspace.bytes) break;
+    const double us = per * 0.25 + 2.0 + 0.1 * splits + 1.1e-6 * stored * splits;
+    if (us < best_us) {
+      best_us = us;
+      best = splits;
+      s->chunk = per * step;
+    }
+  }
+  if (best < 2) return false;
+  s->splits = best;
+  s->parts = (float*)a.workspace.data;
+  s->counters = a.workspace.counters;
+  return true;
+}
+
 template <class T, int Epi>
-int launch_tile(hipStream_t stream, const GemmArgs& a, GemmAccess access) {
+int launch_tile(hipStream_t stream, const GemmArgs& a, GemmAccess access, uint64_t plan_tiles) {
   const uint64_t tiles = (uint64_t)((a.rows + T::TM - 1) / T::TM) * ((a.columns + T::TN - 1) / T::TN);
   if (tiles > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
+  SplitK split;
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, a.batches), dim3(T::kThreads), 0, stream,
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, a.batches, split.splits), dim3(T::kThreads), 0, stream,
                        (uint16_t*)a.out, (const uint16_t*)a.left, (const uint16_t*)a.right, a.rows,
                        a.columns, a.inner, a.left_batch_stride, a.right_batch_stride,
-                       (const uint16_t*)a.addend, a.addend_batch_stride, a.addend_row_stride);
+                       (const uint16_t*)a.addend, a.addend_batch_stride, a.addend_row_stride, split);
   };
   const bool tl = a.transpose_left, tr = a.transpose_right;
-  auto layouts = [&]<int E>() {
-    if (!tl && !tr) go(gemm_f16_tile_kernel<T, false, false, Epi, E>);
-    else if (!tl) go(gemm_f16_tile_kernel<T, false, true, Epi, E>);
-    else if (!tr) go(gemm_f16_tile_kernel<T, true, false, Epi, E>);
-    else go(gemm_f16_tile_kernel<T, true, true, Epi, E>);
+  auto layouts = [&]<int E, bool Split = false>() {
+    if (!tl && !tr) go(gemm_f16_tile_kernel<T, false, false, Epi, E, Split>);
+    else if (!tl) go(gemm_f16_tile_kernel<T, false, true, Epi, E, Split>);
+    else if (!tr) go(gemm_f16_tile_kernel<T, true, false, Epi, E, Split>);
+    else go(gemm_f16_tile_kernel<T, true, true, Epi, E, Split>);
   };
+  if constexpr (T::TM == 32) {
+    if (access != GemmAccess::kElement && split_plan(a, plan_tiles, tiles * a.batches, T::BK, &split)) {
+      if (access == GemmAccess::kDword) layouts.template operator()<kDwords, true>();
+      else if (a.inner % T::BK == 0) layouts.template operator()<kWhole, true>();
+      else layouts.template operator()<kKTail, true>();
+      return hip_status(hipGetLastError());
+    }
+  }
   if (access == GemmAccess::kElement) layouts.template operator()<kElements>();
   else if (access == GemmAccess::kDword) layouts.template operator()<kDwords>();
   else if (a.inner % T::BK == 0) layouts.template operator()<kWhole>();
@@ -433,10 +529,10 @@ int launch_tile(hipStream_t stream, const GemmArgs& a, GemmAccess access) {
 }
 
 template <class T>
-int launch_epilogue(hipStream_t stream, const GemmArgs& a, GemmAccess access) {
-  if (a.addend) return launch_tile<T, kEpiAdd>(stream, a, access);
-  if (a.gelu) return launch_tile<T, kEpiGelu>(stream, a, access);
-  return launch_tile<T, kEpiPlain>(stream, a, access);
+int launch_epilogue(hipStream_t stream, const GemmArgs& a, GemmAccess access, uint64_t plan_tiles) {
+  if (a.addend) return launch_tile<T, kEpiAdd>(stream, a, access, plan_tiles);
+  if (a.gelu) return launch_tile<T, kEpiGelu>(stream, a, access, plan_tiles);
+  return launch_tile<T, kEpiPlain>(stream, a, access, plan_tiles);
 }
 
 }  // namespace
@@ -474,10 +570,12 @@ uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t
   return best;
 }
 
-int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, GemmAccess access) {
-  if (tile == 128) return launch_epilogue<Tile128>(stream, a, access);
-  if (tile == 64) return launch_epilogue<Tile64>(stream, a, access);
-  return launch_epilogue<Tile32>(stream, a, access);
+int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, GemmAccess access,
+                         uint32_t plan_rows, uint32_t plan_batches) {
+  const uint64_t plan_tiles = ((uint64_t)plan_rows + tile - 1) / tile * (((uint64_t)a.columns + tile - 1) / tile) * plan_batches;
+  if (tile == 128) return launch_epilogue<Tile128>(stream, a, access, plan_tiles);
+  if (tile == 64) return launch_epilogue<Tile64>(stream, a, access, plan_tiles);
+  return launch_epilogue<Tile32>(stream, a, access, plan_tiles);
 }
 
 }  // namespace ipus

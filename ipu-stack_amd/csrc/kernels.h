@@ -36,6 +36,7 @@ struct GemmArgs {
   const void* addend = nullptr;
   uint64_t addend_batch_stride = 0;
   uint32_t addend_row_stride = 0;
+  Workspace workspace;  // fp16 GEMM only (gemm_f16_may_split)
 };
 
 // The addend of a split-K reduction (launch_reduce_splits_f16): the partials
@@ -68,11 +69,18 @@ int launch_gemm_f16(hipStream_t stream, const GemmArgs& a);
 // kernels' conditions; the smaller ones are launched by launch_gemm_f16_tile
 // (k_gemm_f16_tile.hip), which does not check those conditions again.  access:
 // what every row pitch and address of the operands allows; kElement also
-// takes K = 0 and operands past the DMA's buffer ranges.
+// takes K = 0 and operands past the DMA's buffer ranges.  plan_rows and
+// plan_batches: those the tile was chosen for.
 uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches,
                        uint32_t largest);
 enum class GemmAccess { kChunk, kDword, kElement };  // 16, 4, 2 bytes
-int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, GemmAccess access);
+int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, GemmAccess access,
+                         uint32_t plan_rows, uint32_t plan_batches);
+// Whether launch_gemm_f16 may split K over workgroups in this launch: only then
+// a caller needs to look the workspace up.
+inline bool gemm_f16_may_split(const GemmArgs& a) {
+  return a.inner >= 1536 && ((uint64_t)a.rows * a.batches + 31) / 32 * (((uint64_t)a.columns + 31) / 32) <= 128;
+}
 // Split-K: fp32 partials float[splits][batches][M][N] into a.out (a.gelu must
 // be false), then launch_reduce_splits_f16 to fp16.  gemm_f16_split_chunk
 // gives the k range per split (a multiple of 64); the plan picks splits so
