@@ -3,6 +3,7 @@
 #pragma once
 
 #include "device_common.h"
+#include "kernels.h"
 
 #define LDS_AS __attribute__((address_space(3)))
 
@@ -107,6 +108,94 @@ __device__ __forceinline__ u32x4 keep_elements(u32x4 v, uint32_t valid) {
 __device__ __forceinline__ void clear_chunk_past(uint8_t* chunk, uint32_t valid) {
   u32x4* p = reinterpret_cast<u32x4*>(chunk);
   *p = keep_elements(*p, valid);
+}
+
+// Split launches of the 32 x 32 tile kernels: workgroup (x, y, z) takes k in
+// [z * chunk, (z + 1) * chunk) of its tile; every split holds at least one k.
+struct SplitK {
+  float* parts = nullptr;        // [batches * tiles][splits][fragments][threads][4]
+  uint32_t* counters = nullptr;  // one per tile, all 0 between launches
+  uint32_t splits = 1, chunk = 0;  // chunk: a multiple of the K step
+};
+
+// Every split leaves its sums (one 16-byte slot per thread and fragment, rows
+// past C none); the last one, where this is true, adds all of them into acc, in
+// the order of K.
+template <int Threads, int MT, int NT, class Stored>
+__device__ __forceinline__ bool add_splits(const SplitK& split, uint64_t tile, float4_t (&acc)[MT][NT], Stored stored) {
+  constexpr uint64_t kSlots = (uint64_t)Threads * MT * NT;
+  float* part = split.parts + (tile * split.splits * kSlots + threadIdx.x) * 4;
+  auto slot = [&](uint32_t z, int i, int j) { return part + (z * kSlots + (uint64_t)(i * NT + j) * Threads) * 4; };
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      if (stored(i)) store_device4(slot(blockIdx.z, i, j), acc[i][j]);
+  __shared__ uint32_t arrived;
+  if (!arrive(split.counters + tile, split.splits, &arrived)) return false;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      if (!stored(i)) continue;
+      // Eight loads in flight (past the last split: the last one again, not added).
+      for (uint32_t z0 = 0; z0 < split.splits; z0 += 8) {
+        float4_t x[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+          x[u] = load_device4(slot(z0 + u < split.splits ? z0 + u : split.splits - 1, i, j));
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+          if (z0 + u < split.splits) acc[i][j] += x[u];
+      }
+    }
+  }
+  return true;
+}
+
+// K splits for at most 128 tiles of 32 x 32 (decode projections, small products
+// with a long K), where the walk over K of few workgroups leaves CUs and memory
+// idle: at most one workgroup per CU and 8 splits.  Modelled time, us: step_us
+// per K step of `step` (fp16, 128 k: 0.25; 0.2 from L2, 0.28-0.49 from HBM; fp32,
+// 64 k: 0.30), and for a split launch 2 for the partial sums, the count and the
+// merge, 0.1 per split and 1.1 per MB of partial sums.  Measured, fp16, unsplit
+// and at this choice, weights in HBM: 8 x 4096 x
+// 4096 18.0 -> 13.4 (4 splits 13.9; transposed weights 10.6 -> 10.1), 8 x 2048 x 8192
+// 31.6 -> 13.1 (8 splits 13.4), 16 x 1024 x 4096 11.5 -> 6.8, 8 x 512 x 8192 19.9 ->
+// 7.1, 64 x 64 x 8192 15.5 -> 6.3, 256 x 256 x 4096 10.2 -> 7.4, 8 x 1024 x 2048 6.9 -> 5.8.
+// Not worth it: 320 x 320 x 2000 5.5 -> 6.6, 64 x 2048 x 2048 6.8 -> 7.0, 8 x 4096 x
+// 1024 4.7 -> 6.0.
+// fp32: 8 x 4096 x 4096 21.6 -> 16.6, 16 x 1024 x 4096 21.2 -> 8.6, 8 x 2048 x 2048 12.0 ->
+// 8.3, 8 x 512 x 8192 39.0 -> 10.2, 64 x 64 x 8192 38.3 -> 8.9, 64 x 2048 x 2048 13.5 -> 11.0, 64 x
+// 1024 x 1024 7.1 -> 6.9; 320 x 320 x 1000 stays unsplit (7.3).
+// The plan is made for plan_tiles, the tiles of the folded product where the
+// batches could be folded (launch_gemm_f16), so that it does not depend on the
+// epilogue; `launched` tiles (at most 32 per folded one) use the workspace.
+inline bool split_plan(const GemmArgs& a, uint64_t plan_tiles, uint64_t launched, uint32_t step, double step_us,
+                       SplitK* s) {
+  if (!a.workspace.data || plan_tiles > 128 || launched > a.workspace.counter_count) return false;
+  const uint32_t steps = (a.inner + step - 1) / step;
+  constexpr uint64_t kTileBytes = 32 * 32 * sizeof(float);
+  const uint64_t rows = (uint64_t)a.rows * a.batches;
+  const double stored = (double)plan_tiles * (rows < 32 ? rows : 32) * 32 * sizeof(float);
+  double best_us = steps * step_us;
+  uint32_t best = 1;
+  for (uint32_t want = 2; want <= 8 && want * plan_tiles <= 256 && want * 2 <= steps; ++want) {
+    const uint32_t per = (steps + want - 1) / want, splits = (steps + per - 1) / per;
+    if (launched * splits * kTileBytes > a.workspace.bytes) break;
+    const double us = per * step_us + 2.0 + 0.1 * splits + 1.1e-6 * stored * splits;
+    if (us < best_us) {
+      best_us = us;
+      best = splits;
+      s->chunk = per * step;
+    }
+  }
+  if (best < 2) return false;
+  s->splits = best;
+  s->parts = (float*)a.workspace.data;
+  s->counters = a.workspace.counters;
+  return true;
 }
 
 }  // namespace ipus

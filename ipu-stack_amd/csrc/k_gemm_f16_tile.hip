@@ -20,7 +20,7 @@
 //     128, 2048^3: 21.6 -> 21.1 us, 1024^3 11.1 -> 9.4, 729 x 4304 x 1152 13.0
 //     -> 11.8); the groups' fp32 sums are added through LDS at the end;
 //   * few 32 x 32 tiles with a long K split K over workgroups, and the last one
-//     adds the partial sums in the order of K (split_plan);
+//     adds the partial sums in the order of K (split_plan, gemm_common.h);
 //   * C leaves through LDS in whole row runs, as in the 256 x 256 kernel.
 // Measured, us per launch, before (256 x 256 kernel or the register-staged
 // small-tile kernel) and now: 2048^3 38.0 -> 21.1 (128 x 128), 729 x 4304 x
@@ -66,14 +66,6 @@ struct TileShape {
 typedef TileShape<128, 128, 64, 64, 2, 64> Tile128;
 typedef TileShape<64, 64, 32, 32, 2, 64> Tile64;
 typedef TileShape<32, 32, 16, 16, 1, 128> Tile32;
-
-// Split launches: workgroup (x, y, z) takes k in [z * chunk, (z + 1) * chunk)
-// of its tile; every split holds at least one k.
-struct SplitK {
-  float* parts = nullptr;        // [batches * tiles][splits][fragments][threads][4]
-  uint32_t* counters = nullptr;  // one per tile, all 0 between launches
-  uint32_t splits = 1, chunk = 0;  // chunk: a multiple of the K step
-};
 
 // LDS tiles.  K-contiguous operand: subtiles of 64 k, each [rows][64 k] with
 // the 16-byte chunk XORed by row & 7.  MN-contiguous: [k][mn], the chunk XORed
@@ -383,37 +375,8 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
     }
   }
   if constexpr (Split) {
-    // Every split leaves its sums (one 16-byte slot per thread and fragment);
-    // the last one adds all of them, in the order of K.
-    const uint64_t tile_at = batch * tiles + pid;
-    const uint64_t slots = (uint64_t)T::kThreads * kMT * kNT;
-    float* part = split.parts + (tile_at * split.splits * slots + threadIdx.x) * 4;
-    auto slot = [&](uint32_t z, int i, int j) { return part + (z * slots + (uint64_t)(i * kNT + j) * T::kThreads) * 4; };
-#pragma unroll
-    for (int i = 0; i < kMT; ++i)
-#pragma unroll
-      for (int j = 0; j < kNT; ++j)
-        if (m0 + wm + 16 * i + r16 < M) store_device4(slot(blockIdx.z, i, j), acc[i][j]);
-    __shared__ uint32_t arrived;
-    if (!arrive(split.counters + tile_at, split.splits, &arrived)) return;
-#pragma unroll
-    for (int i = 0; i < kMT; ++i) {
-#pragma unroll
-      for (int j = 0; j < kNT; ++j) {
-        acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        if (m0 + wm + 16 * i + r16 >= M) continue;
-        // Eight loads in flight (past the last split: the last one again, not added).
-        for (uint32_t z0 = 0; z0 < split.splits; z0 += 8) {
-          float4_t x[8];
-#pragma unroll
-          for (uint32_t u = 0; u < 8; ++u)
-            x[u] = load_device4(slot(z0 + u < split.splits ? z0 + u : split.splits - 1, i, j));
-#pragma unroll
-          for (uint32_t u = 0; u < 8; ++u)
-            if (z0 + u < split.splits) acc[i][j] += x[u];
-        }
-      }
-    }
+    auto stored = [&](int i) { return m0 + wm + 16 * i + r16 < M; };
+    if (!add_splits<T::kThreads>(split, batch * tiles + pid, acc, stored)) return;
   }
   // The wave's rows go out through its own slot of LDS as whole runs of
   // 2 * WN bytes: row r, 16-byte chunk c at chunk c ^ (r & (chunks - 1)).
@@ -456,45 +419,6 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   }
 }
 
-// K splits for at most 128 tiles of 32 x 32 (decode projections, small products
-// with a long K), where the walk over K of few workgroups leaves CUs and memory
-// idle: at most one workgroup per CU and 8 splits.  Modelled time, us: 0.25 per
-// 128-k step (0.2 from L2, 0.28-0.49 from HBM), and for a split launch 2 for the
-// partial sums, the count and the merge, 0.1 per split and 1.1 per MB of
-// partial sums.  Measured, unsplit and at this choice, weights in HBM: 8 x 4096 x
-// 4096 18.0 -> 13.4 (4 splits 13.9; transposed weights 10.6 -> 10.1), 8 x 2048 x 8192
-// 31.6 -> 13.1 (8 splits 13.4), 16 x 1024 x 4096 11.5 -> 6.8, 8 x 512 x 8192 19.9 ->
-// 7.1, 64 x 64 x 8192 15.5 -> 6.3, 256 x 256 x 4096 10.2 -> 7.4, 8 x 1024 x 2048 6.9 -> 5.8.
-// Not worth it: 320 x 320 x 2000 5.5 -> 6.6, 64 x 2048 x 2048 6.8 -> 7.0, 8 x 4096 x
-// 1024 4.7 -> 6.0.
-// The plan is made for plan_tiles, the tiles of the folded product where the
-// batches could be folded (launch_gemm_f16), so that it does not depend on the
-// epilogue; `launched` tiles (at most 32 per folded one) use the workspace.
-bool split_plan(const GemmArgs& a, uint64_t plan_tiles, uint64_t launched, uint32_t step, SplitK* s) {
-  if (!a.workspace.data || plan_tiles > 128 || launched > a.workspace.counter_count) return false;
-  const uint32_t steps = (a.inner + step - 1) / step;
-  constexpr uint64_t kTileBytes = 32 * 32 * sizeof(float);
-  const uint64_t rows = (uint64_t)a.rows * a.batches;
-  const double stored = (double)plan_tiles * (rows < 32 ? rows : 32) * 32 * sizeof(float);
-  double best_us = steps * 0.25;
-  uint32_t best = 1;
-  for (uint32_t want = 2; want <= 8 && want * plan_tiles <= 256 && want * 2 <= steps; ++want) {
-    const uint32_t per = (steps + want - 1) / want, splits = (steps + per - 1) / per;
-    if (launched * splits * kTileBytes > a.workspace.bytes) break;
-    const double us = per * 0.25 + 2.0 + 0.1 * splits + 1.1e-6 * stored * splits;
-    if (us < best_us) {
-      best_us = us;
-      best = splits;
-      s->chunk = per * step;
-    }
-  }
-  if (best < 2) return false;
-  s->splits = best;
-  s->parts = (float*)a.workspace.data;
-  s->counters = a.workspace.counters;
-  return true;
-}
-
 template <class T, int Epi>
 int launch_tile(hipStream_t stream, const GemmArgs& a, GemmAccess access, uint64_t plan_tiles) {
   const uint64_t tiles = (uint64_t)((a.rows + T::TM - 1) / T::TM) * ((a.columns + T::TN - 1) / T::TN);
@@ -514,7 +438,7 @@ int launch_tile(hipStream_t stream, const GemmArgs& a, GemmAccess access, uint64
     else go(gemm_f16_tile_kernel<T, true, true, Epi, E, Split>);
   };
   if constexpr (T::TM == 32) {
-    if (access != GemmAccess::kElement && split_plan(a, plan_tiles, tiles * a.batches, T::BK, &split)) {
+    if (access != GemmAccess::kElement && split_plan(a, plan_tiles, tiles * a.batches, T::BK, 0.25, &split)) {
       if (access == GemmAccess::kDword) layouts.template operator()<kDwords, true>();
       else if (a.inner % T::BK == 0) layouts.template operator()<kWhole, true>();
       else layouts.template operator()<kKTail, true>();

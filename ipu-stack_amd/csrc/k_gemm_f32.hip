@@ -264,6 +264,8 @@ int launch_fast(hipStream_t stream, const GemmArgs& a, bool chunked) {
 // 256^3 21 -> 3.6.  Errors against float64 are those of the kernel before (one
 // fp32 sum over K per element: 5.7e-7 normwise at K = 1024) or, with two K
 // groups, lower (4.1e-7).
+// Few 32 x 32 tiles with a long K split K over workgroups (split_plan,
+// gemm_common.h; shorter sums: 8 x 4096 x 4096 1.2e-6 -> 8.1e-7).
 // ---------------------------------------------------------------------------
 // Tile of C (TM x TN), part of one wave (WM x WN), K groups, k per step.
 template <int BM, int BN, int WM_, int WN_, int KG_, int BK_>
@@ -297,10 +299,12 @@ __device__ __forceinline__ uint32_t mn_swz32(uint32_t k) {
   return RowBytes >= 256 ? ((k >> 3) & 3u) << 2 : ((k >> 3) & 1u) << 2;
 }
 
-template <class T, bool TransposeLeft, bool TransposeRight, int E>
+template <class T, bool TransposeLeft, bool TransposeRight, int E, bool Split>
 __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
     float* __restrict__ out, const float* __restrict__ left, const float* __restrict__ right,
-    uint32_t M, uint32_t N, uint32_t K, uint64_t left_batch_stride, uint64_t right_batch_stride) {
+    uint32_t M, uint32_t N, uint32_t K, uint64_t left_batch_stride, uint64_t right_batch_stride,
+    SplitK split) {
+  static_assert(!Split || T::KG == 1, "splits: one K group");
   constexpr int TM = T::TM, TN = T::TN, BK = T::BK, S = T::S, KG = T::KG;
   constexpr int kMT = T::kMT, kNT = T::kNT, kUnits = T::kUnits, kP = T::kP;
   constexpr int kDmaA = T::kDmaA, kDmaB = T::kDmaB;
@@ -332,8 +336,11 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
   const float* A = left + batch * left_batch_stride;
   const float* B = right + batch * right_batch_stride;
   float* C = out + batch * (uint64_t)M * N;
-  const float* a_base = kAK ? A + (uint64_t)m0 * K : A + m0;
-  const float* b_base = kBK_ ? B + (uint64_t)n0 * K : B + n0;
+  // This workgroup's K range (the whole of K unless Split).
+  const uint32_t k_begin = Split ? blockIdx.z * split.chunk : 0;
+  const uint32_t k_len = Split ? (K - k_begin < split.chunk ? K - k_begin : split.chunk) : K;
+  const float* a_base = kAK ? A + (uint64_t)m0 * K + k_begin : A + m0 + (uint64_t)k_begin * M;
+  const float* b_base = kBK_ ? B + (uint64_t)n0 * K + k_begin : B + n0 + (uint64_t)k_begin * N;
   const uint64_t a_bytes = (uint64_t)M * K * 4 - (uint64_t)(a_base - A) * 4;
   const uint64_t b_bytes = (uint64_t)N * K * 4 - (uint64_t)(b_base - B) * 4;
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -376,8 +383,8 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
   const uint32_t a_kstep = kAK ? BK * 4 : BK * M * 4;
   const uint32_t b_kstep = kBK_ ? BK * 4 : BK * N * 4;
 
-  const uint32_t ksteps = (K + BK - 1) / BK;
-  const uint32_t k_tail = K % BK;
+  const uint32_t ksteps = (k_len + BK - 1) / BK;
+  const uint32_t k_tail = k_len % BK;
   auto clamp = [&](uint32_t k) { return k < ksteps ? k : ksteps - 1; };
   // The DMA of step k into a stage; past the last step the last one again (a
   // stage that is never read), so the wait counts stay exact.  KTail: chunks
@@ -519,6 +526,10 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
         acc[i][j] += *reinterpret_cast<const float4_t*>(theirs + ((i % kRowsT) * kNT + j) * 1024 + lane * 16);
     }
   }
+  if constexpr (Split) {
+    auto stored = [&](int i) { return m0 + wm + 16 * i + r16 < M; };
+    if (!add_splits<T::kThreads>(split, batch * tiles + pid, acc, stored)) return;
+  }
 #pragma unroll
   for (int i = 0; i < kMT; ++i) {
     if (KG > 1 && (uint32_t)i / kRowsT != kg) continue;
@@ -549,18 +560,27 @@ template <class T>
 int launch_tile32(hipStream_t stream, const GemmArgs& a, bool chunked) {
   const uint64_t tiles = (uint64_t)((a.rows + T::TM - 1) / T::TM) * ((a.columns + T::TN - 1) / T::TN);
   if (tiles > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
+  SplitK split;
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, a.batches), dim3(T::kThreads), 0, stream,
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, a.batches, split.splits), dim3(T::kThreads), 0, stream,
                        (float*)a.out, (const float*)a.left, (const float*)a.right, a.rows,
-                       a.columns, a.inner, a.left_batch_stride, a.right_batch_stride);
+                       a.columns, a.inner, a.left_batch_stride, a.right_batch_stride, split);
   };
   const bool tl = a.transpose_left, tr = a.transpose_right;
-  auto layouts = [&]<int E>() {
-    if (!tl && !tr) go(gemm_f32_tile_kernel<T, false, false, E>);
-    else if (!tl) go(gemm_f32_tile_kernel<T, false, true, E>);
-    else if (!tr) go(gemm_f32_tile_kernel<T, true, false, E>);
-    else go(gemm_f32_tile_kernel<T, true, true, E>);
+  auto layouts = [&]<int E, bool Split = false>() {
+    if (!tl && !tr) go(gemm_f32_tile_kernel<T, false, false, E, Split>);
+    else if (!tl) go(gemm_f32_tile_kernel<T, false, true, E, Split>);
+    else if (!tr) go(gemm_f32_tile_kernel<T, true, false, E, Split>);
+    else go(gemm_f32_tile_kernel<T, true, true, E, Split>);
   };
+  if constexpr (T::TM == 32) {
+    if (split_plan(a, tiles * a.batches, tiles * a.batches, T::BK, 0.30, &split)) {
+      if (!chunked) layouts.template operator()<kDwords, true>();
+      else if (a.inner % T::BK == 0) layouts.template operator()<kWhole, true>();
+      else layouts.template operator()<kKTail, true>();
+      return hip_status(hipGetLastError());
+    }
+  }
   if (!chunked) layouts.template operator()<kDwords>();
   else if (a.inner % T::BK == 0) layouts.template operator()<kWhole>();
   else layouts.template operator()<kKTail>();

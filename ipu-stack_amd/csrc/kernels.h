@@ -36,7 +36,7 @@ struct GemmArgs {
   const void* addend = nullptr;
   uint64_t addend_batch_stride = 0;
   uint32_t addend_row_stride = 0;
-  Workspace workspace;  // fp16 GEMM only (gemm_f16_may_split)
+  Workspace workspace;  // gemm_may_split
 };
 
 // The addend of a split-K reduction (launch_reduce_splits_f16): the partials
@@ -76,10 +76,11 @@ uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t
 enum class GemmAccess { kChunk, kDword, kElement };  // 16, 4, 2 bytes
 int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, GemmAccess access,
                          uint32_t plan_rows, uint32_t plan_batches);
-// Whether launch_gemm_f16 may split K over workgroups in this launch: only then
-// a caller needs to look the workspace up.
-inline bool gemm_f16_may_split(const GemmArgs& a) {
-  return a.inner >= 1536 && ((uint64_t)a.rows * a.batches + 31) / 32 * (((uint64_t)a.columns + 31) / 32) <= 128;
+// Whether launch_gemm_f16 or launch_gemm_f32 may split K over workgroups in this
+// launch: only then a caller needs to look the workspace up.
+inline bool gemm_may_split(const GemmArgs& a, bool f16) {
+  return a.inner >= (f16 ? 1536u : 640u) &&
+         ((uint64_t)a.rows * a.batches + 31) / 32 * (((uint64_t)a.columns + 31) / 32) <= 128;
 }
 // Split-K: fp32 partials float[splits][batches][M][N] into a.out (a.gelu must
 // be false), then launch_reduce_splits_f16 to fp16.  gemm_f16_split_chunk

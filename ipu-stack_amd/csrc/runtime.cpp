@@ -431,7 +431,7 @@ int run_gemm(ipus_context* ctx, void* out, const void* const* in, const uint32_t
   GemmArgs a;
   if (int e = gemm_args(out, in, s, &a)) return e;
   a.gelu = gelu;
-  if (f16 && gemm_f16_may_split(a)) a.workspace = context_workspace(ctx);
+  if (gemm_may_split(a, f16)) a.workspace = context_workspace(ctx);
   return f16 ? launch_gemm_f16(ctx->stream, a) : launch_gemm_f32(ctx->stream, a);
 }
 
@@ -489,7 +489,7 @@ const std::vector<KernelEntry>& registry() {
          a.addend = i[2];
          a.addend_batch_stride = s[8];
          a.addend_row_stride = s[9];
-         if (gemm_f16_may_split(a)) a.workspace = context_workspace(c);
+         if (gemm_may_split(a, true)) a.workspace = context_workspace(c);
          return launch_gemm_f16(c->stream, a);
        },
        check_gemm_flags},

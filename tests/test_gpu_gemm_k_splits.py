@@ -65,3 +65,27 @@ def test_gemm_f16_k_splits_epilogues(ipus, oracle, ctx, shared, epilogue):
     assert np.array_equal(fused.download(np.uint16), expected)
     for x in (da, db, product, want, fused):
         x.free()
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 4096, 4096), (16, 1000, 1028), (32, 32, 640), (1, 1024, 8192),
+                                   (64, 64, 2049), (10, 515, 1795)])
+@pytest.mark.parametrize("tl,tr", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_f32_k_splits(ipus, ctx, M, N, K, tl, tr):
+    """fp32: an fp32 sum of K rounded products, each within 2^-24 of the running
+    magnitude."""
+    rng = np.random.default_rng(73)
+    a, b = rng.uniform(-1, 1, M * K).astype(np.float32), rng.uniform(-1, 1, K * N).astype(np.float32)
+    af = a.astype(np.float64).reshape((K, M) if tl else (M, K))
+    bf = b.astype(np.float64).reshape((N, K) if tr else (K, N))
+    af, bf = af.T if tl else af, bf.T if tr else bf
+    da, db = ctx.upload(a), ctx.upload(b)
+    outs = [ctx.upload(np.full(M * N + 4, 7.5, np.float32)) for _ in range(3)]
+    for out in outs:
+        ctx.launch("ipu_stack_gemm_f32", out, [da, db], [1, M, N, K, tl, tr, 0, 0])
+    raw = [out.download(np.float32) for out in outs]
+    assert np.all(raw[0][M * N:] == 7.5)  # nothing stored past C
+    got = raw[0][:M * N].reshape(M, N).astype(np.float64)
+    assert np.all(np.abs(got - af @ bf) <= np.abs(af) @ np.abs(bf) * (K + 8) * 2.0 ** -24)
+    assert np.array_equal(raw[0], raw[1]) and np.array_equal(raw[0], raw[2])
+    for x in (da, db, *outs):
+        x.free()
