@@ -734,7 +734,8 @@ __global__ __launch_bounds__(kThreads) void add_vector_kernel(T* __restrict__ ds
   constexpr uint32_t kPer = 16 / sizeof(T);
   const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= total) return;
-  const uint32_t row = i / s.vectors, c = i % s.vectors * kPer;
+  const uint32_t row = i / s.vectors;
+  const uint64_t c = (uint64_t)(i % s.vectors) * kPer;  // a collapsed axis can pass 2^32 elements
   const uint32_t o1 = row / s.outer0, o0 = row % s.outer0;
   const T* l = left + o1 * s.ls[1] + o0 * s.ls[0];
   const T* r = right + o1 * s.rs[1] + o0 * s.rs[0];

@@ -40,3 +40,26 @@ def test_broadcast_add(ipus, ctx, left, right, dtype, swap):
     assert np.array_equal(out.download(t)[:want.size].reshape(shape), want)
     for b in bufs + shifted + [out]:
         b.free()
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+def test_broadcast_add_past_32_bit_columns(ctx, dtype):
+    """A contiguous operand plus one value collapses to a single axis, here of
+    2^32 + 65536 elements: columns past 2^32 read their own elements, not those
+    32 bits of the column away."""
+    t = np.float16 if dtype == "f16" else np.float32
+    rows, columns = 65537, 65536
+    size = np.dtype(t).itemsize
+    left, out = ctx.alloc(rows * columns * size), ctx.alloc(rows * columns * size)
+    first, last = (np.random.default_rng(i).standard_normal(columns).astype(t) for i in (1, 2))
+    ends, value = [ctx.upload(first), ctx.upload(last)], ctx.upload(np.array([0.5], t))
+    offsets = [0, (rows - 1) * columns * size]
+    for end, at in zip(ends, offsets):
+        ctx.launch("ipu_stack_copy", left.ptr + at, [end], [columns * size])
+    scalars = [2, rows, columns, 1, 1, 1, 1, columns, 1, 0, 0, 0, 0] + [0] * 6
+    ctx.launch(f"ipu_stack_add_broadcast_{dtype}", out, [left, value], scalars)
+    for x, end, at in zip((first, last), ends, offsets):
+        ctx.launch("ipu_stack_copy", end, [out.ptr + at], [columns * size])
+        assert np.array_equal(end.download(t), (x.astype(np.float32) + 0.5).astype(t)), at
+    for b in [left, out, value] + ends:
+        b.free()
