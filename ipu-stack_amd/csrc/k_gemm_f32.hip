@@ -32,6 +32,7 @@
 
 #include "gemm_common.h"
 #include "kernels.h"
+#include "tile_grid.h"
 
 namespace ipus {
 namespace {
@@ -320,9 +321,11 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
 
   const uint32_t nbm = (M + TM - 1) / TM, nbn = (N + TN - 1) / TN;
   const uint32_t tiles = nbm * nbn;
+  const uint32_t block = Split ? blockIdx.x : grid_tile(blockIdx.x, blockIdx.z);
+  if (!Split && block >= tiles) return;
   // XCD-contiguous tiles, grouped 8 along M.
-  const uint32_t xcd = blockIdx.x % 8, per = tiles / 8, rest = tiles % 8;
-  const uint32_t pid = xcd * per + (xcd < rest ? xcd : rest) + blockIdx.x / 8;
+  const uint32_t xcd = block % 8, per = tiles / 8, rest = tiles % 8;
+  const uint32_t pid = xcd * per + (xcd < rest ? xcd : rest) + block / 8;
   constexpr uint32_t kGroup = 8;
   const uint32_t group = pid / (kGroup * nbn);
   const uint32_t first_m = group * kGroup;
@@ -560,9 +563,13 @@ template <class T>
 int launch_tile32(hipStream_t stream, const GemmArgs& a, bool chunked) {
   const uint64_t tiles = (uint64_t)((a.rows + T::TM - 1) / T::TM) * ((a.columns + T::TN - 1) / T::TN);
   if (tiles > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
+  static_assert((uint64_t)kTileGridX * T::kThreads < (1ull << 32), "a grid dimension holds fewer than 2^32 work-items");
+  const TileGrid grid = tile_grid(tiles);
   SplitK split;
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, a.batches, split.splits), dim3(T::kThreads), 0, stream,
+    // A split launch has at most 128 tiles a batch (split_plan), so the third
+    // dimension is free for its splits.
+    hipLaunchKernelGGL(kernel, dim3(grid.x, a.batches, split.splits > 1 ? split.splits : grid.z), dim3(T::kThreads), 0, stream,
                        (float*)a.out, (const float*)a.left, (const float*)a.right, a.rows,
                        a.columns, a.inner, a.left_batch_stride, a.right_batch_stride, split);
   };
