@@ -214,7 +214,10 @@ int ipus_session_run(ipus_session *session);
  * replay).  The role of the reference's precompiled device program
  * (HostSession runs, crates/ipu-driver/src/lib.rs:1341-1600) for
  * launch-bound packages; no reference function of its own.  Every step is
- * a kernel (no memset nodes).  A second call is a no-op. */
+ * a kernel (no memset nodes).  A second call is a no-op.  While a caller
+ * records the context's stream into a graph of its own, ipus_session_run
+ * enqueues the steps instead: the captured graph may use device memory of
+ * the context that only launches on its stream share. */
 int ipus_session_capture(ipus_session *session);
 
 #ifdef __cplusplus

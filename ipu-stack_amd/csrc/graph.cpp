@@ -1484,7 +1484,10 @@ int launch_steps(ipus_session* s) {
 extern "C" int ipus_session_run(ipus_session* s) {
   if (!s) return fail(IPUS_ERROR_INVALID_ARGUMENT, "null session");
   if (int status = use_device(s->ctx)) return status;
-  if (s->exec) {
+  // The captured graph splits reductions through the context's workspace, so it
+  // only runs on the context's stream; a caller that records the stream gets
+  // the steps themselves, which do without (context_workspace).
+  if (s->exec && !stream_recorded(s->ctx)) {
     const hipError_t e = hipGraphLaunch(s->exec, s->ctx->stream);
     return e == hipSuccess ? 0 : hip_fail(e, "hipGraphLaunch");
   }

@@ -42,6 +42,8 @@ struct Workspace;
 // into a graph of its own (which it may launch on other streams, several at
 // once): the unsplit kernels run then.
 Workspace context_workspace(const ipus_context* ctx);
+// The context's stream is being recorded into a graph (or cannot tell).
+bool stream_recorded(const ipus_context* ctx);
 
 // Records a formatted message as the thread's last error and returns `code`.
 int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));

@@ -52,14 +52,15 @@ int use_device(const ipus_context* ctx) {
 constexpr size_t kWorkspaceBytes = 32u << 20;
 constexpr uint32_t kWorkspaceCounters = 16384;
 
+bool stream_recorded(const ipus_context* ctx) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+
 Workspace context_workspace(const ipus_context* ctx) {
   Workspace w;
   if (!ctx->workspace) return w;
-  if (!ctx->capturing_session.load(std::memory_order_relaxed)) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone)
-      return w;
-  }
+  if (!ctx->capturing_session.load(std::memory_order_relaxed) && stream_recorded(ctx)) return w;
   w.data = ctx->workspace;
   w.bytes = kWorkspaceBytes;
   w.counters = ctx->workspace_counters;
