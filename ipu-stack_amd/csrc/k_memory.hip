@@ -109,9 +109,9 @@ __device__ __forceinline__ void store_row8(uint16_t* row, uint32_t c, uint32_t l
 // Matrices with too few such tiles for the chip take one wave per workgroup
 // (64 x 64 tiles), so that every CU has some.  Any: rows, columns or addresses
 // that are no multiple of 8 elements, with the same blocks read and written at
-// element alignment and by element at the edges (a kernel with one element per
-// thread, reading a column per wave, before: 4313 x 7213 149 -> 33.7 us, 8191 x
-// 8190 208 -> 47.8, 729 x 1152 5.4 -> 4.3 a launch).
+// element alignment and by element at the edges.  Small totals and matrices
+// that leave most of a tile empty take one element per thread instead (rule
+// and figures at launch_transpose_f16).
 // ---------------------------------------------------------------------------
 constexpr uint32_t kTransposeWaves = 8;
 template <uint32_t Waves, bool Any>
@@ -147,6 +147,19 @@ __global__ __launch_bounds__(64 * Waves) void transpose_f16_kernel(
       store16_nt(d + (uint64_t)(c0 + i) * rows + r0, out[i]);
     }
   }
+}
+
+// One element per thread, in destination order (matrices * rows * columns below
+// 2^32): a wave reads a column, so a matrix past the caches costs a line per
+// element, but nothing is left idle by rows or columns below a tile's.
+__global__ __launch_bounds__(kThreads) void transpose_f16_element_kernel(
+    uint16_t* __restrict__ dst, const uint16_t* __restrict__ src, uint32_t rows, uint32_t columns,
+    uint32_t total) {
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i >= total) return;
+  const uint32_t elements = rows * columns, matrix = i / elements;
+  const uint32_t at = i - matrix * elements, c = at / rows, r = at - c * rows;
+  dst[i] = src[matrix * elements + r * columns + c];
 }
 
 // ---------------------------------------------------------------------------
@@ -922,24 +935,46 @@ inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 int launch_transpose_f16(hipStream_t stream, void* dst, const void* src, uint32_t matrices,
                          uint32_t rows, uint32_t columns) {
   if (matrices == 0 || rows == 0 || columns == 0) return 0;
+  // Aligned extents move whole vectors in any tile; other matrices, and more than
+  // one launch takes, go by the elements there are and how far they fill a tile.
   const bool chunks = rows % 8 == 0 && columns % 8 == 0 && aligned16(dst) && aligned16(src);
+  const bool one_launch = chunks && matrices <= 65535;
   const uint32_t tiles_c = ceil_div(columns, 64);
   const uint64_t tall = (uint64_t)ceil_div(rows, 64 * kTransposeWaves) * tiles_c;
   const uint64_t small = (uint64_t)ceil_div(rows, 64) * tiles_c;
-  if (small > 0x7fffffffu) return IPUS_ERROR_INVALID_ARGUMENT;
+  const uint64_t elements = (uint64_t)rows * columns, total = elements * matrices;
+  // Measured, us, one element per thread against 64 x 64 tiles: 70000 x 3 x 5 3.8 /
+  // 37 (tall tiles 642), 4096 x 17 x 33 5.8 / 11, 5 x 10^6 11.9 / 39, 26 x 50 x 100 2.3 / 6.0,
+  // 120 x 65 x 100 3.1 / 5.6, 238 x 100 x 33 3.1 / 5.2; 729 x 1152 5.0 / 3.8, 2 x 1000 x 1000
+  // 10.8 / 3.8, 41 x 50 x 1000 6.4 / 4.1, 37400 x 20 3.5 / 5.8, 104 x 1000 x 20 5.4 / 6.6, 838 x
+  // 1000 x 20 35 / 26, 2033 x 1000 x 33 175 / 53.
+  const double fill = (double)elements / (4096.0 * (double)small);
+  const bool few = total < 655360 || (total < (1u << 20) && elements < (1u << 17));
+  const bool empty = fill < 0.3 || (fill < 0.4 && total < 2200000);
+  if (!one_launch && (few || empty) && total <= 0xffffff00ull) {
+    hipLaunchKernelGGL(transpose_f16_element_kernel, dim3(ceil_div(total, kThreads)), dim3(kThreads), 0,
+                       stream, (uint16_t*)dst, (const uint16_t*)src, rows, columns, (uint32_t)total);
+    return hip_status(hipGetLastError());
+  }
+  // Up to two rounds of the tall tiles (one workgroup per CU), 64 x 64 tiles
+  // are as fast or faster: 2048^2 5.2 -> 4.4 us a launch, 2048 x 4096 6.8 -> 5.9,
+  // 4096^2 13.4 -> 12.1-13.3; beyond, the tall ones hold (8192^2 45.5), where odd
+  // extents fill them (2001 x 6000 in 5 matrices 50.8 / 45.5, 2001 x 50 in 670 61.5 / 68.6,
+  // 100 x 100 in 6710 82 / 332).
+  const bool full = (double)elements >= 0.8 * 64.0 * 64.0 * kTransposeWaves * (double)tall;
+  const bool tall_tiles = tall * matrices > 512 && (one_launch || full) &&
+                          tall * 64 * kTransposeWaves < (1ull << 32);
+  if (small * 64 >= (1ull << 32)) return IPUS_ERROR_INVALID_ARGUMENT;  // past a grid dimension
   // Matrices beyond the grid's second dimension: one launch per 65535.
   for (uint32_t first = 0; first < matrices; first += 65535) {
     const uint32_t count = matrices - first < 65535 ? matrices - first : 65535;
-    uint16_t* d = (uint16_t*)dst + (uint64_t)first * rows * columns;
-    const uint16_t* s = (const uint16_t*)src + (uint64_t)first * rows * columns;
+    uint16_t* d = (uint16_t*)dst + (uint64_t)first * elements;
+    const uint16_t* s = (const uint16_t*)src + (uint64_t)first * elements;
     auto go = [&](auto kernel, uint64_t tiles, uint32_t waves, uint32_t lds) {
       hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, count), dim3(64 * waves), lds, stream, d, s, rows,
                          columns, tiles_c);
     };
-    // Up to two rounds of the tall tiles (one workgroup per CU), 64 x 64 tiles
-    // are as fast or faster: 2048^2 5.2 -> 4.4 us a launch, 2048 x 4096 6.8 -> 5.9,
-    // 4096^2 13.4 -> 12.1-13.3; beyond, the tall ones hold (8192^2 45.5).
-    if (tall * count > 512) {
+    if (tall_tiles) {
       if (chunks) go(transpose_f16_kernel<kTransposeWaves, false>, tall, kTransposeWaves, occupancy_lds(1, 0));
       else go(transpose_f16_kernel<kTransposeWaves, true>, tall, kTransposeWaves, occupancy_lds(1, 0));
     } else {

@@ -62,3 +62,59 @@ def test_padded_rearrange(ipus, oracle, ctx, order, rb, cb, matrices, lr, pr, lc
         assert np.array_equal(read_guarded(dst, n, dshift), want)
         dst.free()
     src.free()
+
+
+@pytest.mark.parametrize("matrices,rows,cols,shift", [
+    (12, 301, 299, 0), (12, 304, 296, 1),       # 64 x 64 tiles with partial blocks
+    (70, 1001, 255, 0),                         # tall tiles, partial blocks
+    (9, 301, 299, 3), (700, 65, 100, 0),        # by element: a small total, empty tiles
+    (70001, 5, 13, 0), (66000, 8, 24, 0),
+    (65600, 40, 40, 0)])                        # 64 x 64 tiles in two launches
+def test_transpose_routes(ipus, oracle, ctx, matrices, rows, cols, shift):
+    test_transpose_any_size_and_alignment(ipus, oracle, ctx, matrices, rows, cols, shift)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 600_000_007), (600_000_007, 1)])
+def test_transpose_of_a_long_row(ctx, rows, cols):
+    """More 64-column tiles than a grid dimension holds of 512 threads."""
+    n = rows * cols
+    src, dst = ctx.alloc(2 * n), ctx.alloc(2 * n + 16)
+    ends = np.random.default_rng(7).integers(0, 1 << 16, (3, 4096)).astype(np.uint16)
+    window = ctx.alloc(ends[0].nbytes)
+    starts = [0, n // 3, n - 4096]
+    for x, at in zip(ends, starts):
+        ctx.write(window, x)
+        ctx.launch("ipu_stack_copy", src.ptr + 2 * at, [window], [window.nbytes])
+    ctx.memset(dst, 0x5A)
+    ctx.launch("ipu_stack_transpose_f16", dst, [src], [1, rows, cols])
+    for x, at in zip(ends, starts):
+        ctx.launch("ipu_stack_copy", window, [dst.ptr + 2 * at], [window.nbytes])
+        assert np.array_equal(window.download(np.uint16), x), at
+    ctx.launch("ipu_stack_copy", window, [dst.ptr + 2 * n], [16])
+    assert np.all(window.download(np.uint16)[:8] == 0x5A5A)
+    for b in (src, dst, window):
+        b.free()
+
+
+@pytest.mark.parametrize("matrices,rows,cols", [(70000, 3, 5), (4096, 17, 33), (1, 1, 1000000), (69967, 2, 8)])
+def test_transpose_of_small_extents_keeps_the_chip_busy(ctx, matrices, rows, cols):
+    """One tile per small matrix, one workgroup per CU, took 10 to 170 times as long as
+    a transpose of the same elements in one matrix; a launch takes about as long."""
+    n = matrices * rows * cols
+    src, dst = ctx.alloc(2 * n), ctx.alloc(2 * n)
+
+    def us(scalars):
+        best = 1e9
+        for _ in range(5):
+            events = ctx.event_series(2)
+            events.record(0)
+            for _ in range(20):
+                ctx.launch("ipu_stack_transpose_f16", dst, [src], scalars)
+            events.record(1)
+            best = min(best, float(events.durations()[0]) * 1000 / 20)
+        return best
+
+    side = int(n ** 0.5)
+    assert us([matrices, rows, cols]) < 3.0 * us([1, side, side]) + 5.0
+    src.free()
+    dst.free()
