@@ -133,10 +133,8 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   const uint16_t* b_base = kBK_ ? B + (uint64_t)n0 * K + k_begin : B + n0 + (uint64_t)k_begin * N;
   const uint64_t a_bytes = (uint64_t)M * K * 2 - (uint64_t)(a_base - A) * 2;
   const uint64_t b_bytes = (uint64_t)N * K * 2 - (uint64_t)(b_base - B) * 2;
-  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)a_base, 0, (int)(a_bytes > 0x7fffffffull ? 0x7fffffff : a_bytes), kBufferFlags);
-  const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)b_base, 0, (int)(b_bytes > 0x7fffffffull ? 0x7fffffff : b_bytes), kBufferFlags);
+  const int a_range = (int)(a_bytes > 0x7fffffffull ? 0x7fffffff : a_bytes);
+  const int b_range = (int)(b_bytes > 0x7fffffffull ? 0x7fffffff : b_bytes);
 
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t lane = threadIdx.x % kWave;
@@ -173,14 +171,18 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
 
   const uint32_t ksteps = (k_len + BK - 1) / BK;
   const uint32_t k_tail = k_len % BK;
-  auto clamp = [&](uint32_t k) { return k < ksteps ? k : ksteps - 1; };
-  // The DMA of step k into a stage.  Past the last step it fetches the last
-  // one again (a stage that is never read), so the wait counts stay exact.
+  // The DMA of step k into a stage.  Past the last step the descriptors are
+  // empty: no memory is read (the stage is never read either), but the
+  // instructions are issued, so the wait counts stay exact.
   // KTail: on the last step, K-contiguous chunks and MN-contiguous rows past
   // K get an offset past the range and read 0 (the step's K offset travels in
   // the scalar offset, which the range check does not cover).
   auto dma = [&](uint8_t* stage, uint32_t k) __attribute__((always_inline)) {
     const uint32_t limit = KTail && k == ksteps - 1 ? k_tail : 0u;
+    const __amdgpu_buffer_rsrc_t a_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, k < ksteps ? a_range : 0, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t b_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)b_base, 0, k < ksteps ? b_range : 0, kBufferFlags);
     auto one = [&]<bool KContig, int TMN>(__amdgpu_buffer_rsrc_t rsrc, uint8_t* tile, uint32_t inst, uint32_t voff, uint32_t soff) __attribute__((always_inline)) {
       if (KTail && limit != 0) {
         uint32_t row, col;
@@ -243,9 +245,9 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
     load_regs(3, regs[1]);
   } else {
     dma(lds0, 0);
-    dma(lds1, clamp(1));
-    dma(lds2, clamp(2));
-    dma(lds3, clamp(3));
+    dma(lds1, 1);
+    dma(lds2, 2);
+    dma(lds3, 3);
   }
 
   auto k_base = [&](uint32_t w0) { return (w0 + r16) * 128 + ((g4 ^ (r16 & 7)) << 4); };
@@ -313,17 +315,19 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   // kElements: the step stores the chunks of step kt + 2, loaded two steps ago,
   // into their stage (`ahead`, last read in step kt - 2) and loads those of
   // step kt + 4; the barrier publishes the stores of the step before.
-  auto step = [&](uint8_t* cur, uint8_t* next, uint8_t* ahead, int buf, uint32_t kt) __attribute__((always_inline)) {
+  // Tail t (1, 2, 3): the t-th of the at most three steps after the last group of
+  // four, which have nothing left to fetch.
+  auto step = [&]<int Tail>(uint8_t* cur, uint8_t* next, uint8_t* ahead, int buf, uint32_t kt) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (kRegs) {
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-      store_regs(ahead, regs[buf]);
-      load_regs(kt + S, regs[buf]);
+      if constexpr (Tail <= 1) store_regs(ahead, regs[buf]);
+      if constexpr (Tail == 0) load_regs(kt + S, regs[buf]);
     } else {
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * kDma) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((Tail ? S - 1 - Tail : S - 2) * kDma) : "memory");
       __builtin_amdgcn_sched_barrier(0);
-      dma(cur, clamp(kt + S));
+      if constexpr (Tail == 0) dma(cur, kt + S);
     }
     if (E == kDwords && kt + 2 == ksteps) clear_past_k(next);
     __builtin_amdgcn_sched_barrier(0);
@@ -342,15 +346,16 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   };
   uint32_t kt = 0;
   for (; kt + 3 < ksteps; kt += 4) {
-    step(lds0, lds1, lds2, 0, kt);
-    step(lds1, lds2, lds3, 1, kt + 1);
-    step(lds2, lds3, lds0, 0, kt + 2);
-    step(lds3, lds0, lds1, 1, kt + 3);
+    step.template operator()<0>(lds0, lds1, lds2, 0, kt);
+    step.template operator()<0>(lds1, lds2, lds3, 1, kt + 1);
+    step.template operator()<0>(lds2, lds3, lds0, 0, kt + 2);
+    step.template operator()<0>(lds3, lds0, lds1, 1, kt + 3);
   }
-  if (kt < ksteps) step(lds0, lds1, lds2, 0, kt);
-  if (kt + 1 < ksteps) step(lds1, lds2, lds3, 1, kt + 1);
-  if (kt + 2 < ksteps) step(lds2, lds3, lds0, 0, kt + 2);
-  // The redundant prefetches have landed and every wave is done with the stages.
+  if (kt < ksteps) step.template operator()<1>(lds0, lds1, lds2, 0, kt);
+  if (kt + 1 < ksteps) step.template operator()<2>(lds1, lds2, lds3, 1, kt + 1);
+  if (kt + 2 < ksteps) step.template operator()<3>(lds2, lds3, lds0, 0, kt + 2);
+  // Every DMA has landed (those past the last step too) and every wave is done
+  // with the stages.
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   // acc[i][j][e] = C[m0 + wm + 16 i + lane % 16][n0 + wn + 16 j + 4 (lane / 16) + e]

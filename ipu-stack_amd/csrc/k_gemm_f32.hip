@@ -346,10 +346,8 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
   const float* b_base = kBK_ ? B + (uint64_t)n0 * K + k_begin : B + n0 + (uint64_t)k_begin * N;
   const uint64_t a_bytes = (uint64_t)M * K * 4 - (uint64_t)(a_base - A) * 4;
   const uint64_t b_bytes = (uint64_t)N * K * 4 - (uint64_t)(b_base - B) * 4;
-  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)a_base, 0, (int)(a_bytes > 0x7fffffffull ? 0x7fffffff : a_bytes), kBufferFlags);
-  const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)b_base, 0, (int)(b_bytes > 0x7fffffffull ? 0x7fffffff : b_bytes), kBufferFlags);
+  const int a_range = (int)(a_bytes > 0x7fffffffull ? 0x7fffffff : a_bytes);
+  const int b_range = (int)(b_bytes > 0x7fffffffull ? 0x7fffffff : b_bytes);
 
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t lane = threadIdx.x % kWave;
@@ -388,12 +386,16 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
 
   const uint32_t ksteps = (k_len + BK - 1) / BK;
   const uint32_t k_tail = k_len % BK;
-  auto clamp = [&](uint32_t k) { return k < ksteps ? k : ksteps - 1; };
-  // The DMA of step k into a stage; past the last step the last one again (a
-  // stage that is never read), so the wait counts stay exact.  KTail: chunks
-  // and rows past K on the last step get an offset past the range and read 0.
+  // The DMA of step k into a stage.  Past the last step the descriptors are
+  // empty: no memory is read, but the instructions are issued, so the wait
+  // counts stay exact.  KTail: chunks and rows past K on the last step get an
+  // offset past the range and read 0.
   auto dma = [&](uint8_t* stage, uint32_t k) __attribute__((always_inline)) {
     const uint32_t limit = KTail && k == ksteps - 1 ? k_tail : 0u;
+    const __amdgpu_buffer_rsrc_t a_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, k < ksteps ? a_range : 0, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t b_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)b_base, 0, k < ksteps ? b_range : 0, kBufferFlags);
     auto one = [&]<bool KContig, int TMN>(__amdgpu_buffer_rsrc_t rsrc, uint8_t* tile, uint32_t inst, uint32_t voff, uint32_t soff) __attribute__((always_inline)) {
       if (KTail && limit != 0) {
         uint32_t row, col;
@@ -413,9 +415,9 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
       one.template operator()<kBK_, TN>(b_rsrc, stage + T::kABytes, wave * kDmaB + j, b_voff[j], k * b_kstep);
   };
   dma(lds0, 0);
-  dma(lds1, clamp(1));
-  dma(lds2, clamp(2));
-  dma(lds3, clamp(3));
+  dma(lds1, 1);
+  dma(lds2, 2);
+  dma(lds3, 3);
 
   const uint32_t h0 = KG == 2 ? kg : 0;
   auto k_base = [&](uint32_t w0) { return (w0 + r16) * 128 + (((2 * g4 + h0) ^ (r16 & 7)) << 4); };
@@ -474,11 +476,12 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
   for (int r = 0; r < kItems; ++r) read_item(lds0, 0, r);
   // After the barrier every wave's DMA of stage kt + 1 has landed and every
   // wave's reads of stage kt have returned.
-  auto step = [&](uint8_t* cur, uint8_t* next, int buf, uint32_t kt) __attribute__((always_inline)) {
+  // Tail t: as in k_gemm_f16_tile.hip, the steps after the last group of four.
+  auto step = [&]<int Tail>(uint8_t* cur, uint8_t* next, int buf, uint32_t kt) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * kDma) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((Tail ? S - 1 - Tail : S - 2) * kDma) : "memory");
     __builtin_amdgcn_sched_barrier(0);
-    dma(cur, clamp(kt + S));
+    if constexpr (Tail == 0) dma(cur, kt + S);
     if (E == kDwords && kt + 2 == ksteps) clear_past_k(next);
     __builtin_amdgcn_sched_barrier(0);
     int r = 0;
@@ -495,14 +498,14 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f32_tile_kernel(
   };
   uint32_t kt = 0;
   for (; kt + 3 < ksteps; kt += 4) {
-    step(lds0, lds1, 0, kt);
-    step(lds1, lds2, 1, kt + 1);
-    step(lds2, lds3, 0, kt + 2);
-    step(lds3, lds0, 1, kt + 3);
+    step.template operator()<0>(lds0, lds1, 0, kt);
+    step.template operator()<0>(lds1, lds2, 1, kt + 1);
+    step.template operator()<0>(lds2, lds3, 0, kt + 2);
+    step.template operator()<0>(lds3, lds0, 1, kt + 3);
   }
-  if (kt < ksteps) step(lds0, lds1, 0, kt);
-  if (kt + 1 < ksteps) step(lds1, lds2, 1, kt + 1);
-  if (kt + 2 < ksteps) step(lds2, lds3, 0, kt + 2);
+  if (kt < ksteps) step.template operator()<1>(lds0, lds1, 0, kt);
+  if (kt + 1 < ksteps) step.template operator()<2>(lds1, lds2, 1, kt + 1);
+  if (kt + 2 < ksteps) step.template operator()<3>(lds2, lds3, 0, kt + 2);
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   // acc[i][j][e] = C[m0 + wm + 16 i + lane % 16][n0 + wn + 16 j + 4 (lane / 16) + e]
