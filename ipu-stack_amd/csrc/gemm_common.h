@@ -69,14 +69,22 @@ enum Edge : int { kWhole = 0, kKTail = 1, kDwords = 2, kElements = 3 };
 // 16-byte access at element (2-byte) alignment: one global_load/store_dwordx4
 // (the device runs in unaligned access mode).
 typedef u32x4 __attribute__((aligned(2))) u32x4_elements;
-// Elements at .. at + 7 of an operand of `total` elements, zero past its end.
+// The first `valid` elements of a chunk, zero past them.
+__device__ __forceinline__ u32x4 keep_elements(u32x4 v, uint32_t valid) {
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w)
+    v[w] &= (2 * w < valid ? 0xffffu : 0u) | (2 * w + 1 < valid ? 0xffff0000u : 0u);
+  return v;
+}
+// Elements at .. at + 7 (at < total) of an operand of `total` elements, any past
+// its end the last one.  That chunk's elements are eight independent loads,
+// clamped to the operand, not eight tests and loads in turn.
 __device__ __forceinline__ u32x4 load_chunk(const uint16_t* x, uint64_t at, uint64_t total) {
   if (at + 8 <= total) return *reinterpret_cast<const u32x4_elements*>(x + at);
-  u32x4 v = {0, 0, 0, 0};
+  uint32_t e[8];
 #pragma unroll
-  for (uint32_t e = 0; e < 8; ++e)
-    if (at + e < total) v[e / 2] |= (uint32_t)x[at + e] << (16 * (e % 2));
-  return v;
+  for (uint32_t i = 0; i < 8; ++i) e[i] = x[at + i < total ? at + i : total - 1];
+  return u32x4{e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16};
 }
 // 16 bytes of C (8 columns of one row), `valid` columns of them inside the row.
 __device__ __forceinline__ void store_elements(uint16_t* p, u32x4 v, uint32_t valid) {
@@ -95,13 +103,6 @@ __device__ __forceinline__ u32x4 load_elements(const uint16_t* p, uint32_t valid
 #pragma unroll
   for (uint32_t e = 0; e < 8; ++e)
     if (e < valid) v[e / 2] |= (uint32_t)p[e] << (16 * (e % 2));
-  return v;
-}
-// The first `valid` elements of a chunk, zero past them.
-__device__ __forceinline__ u32x4 keep_elements(u32x4 v, uint32_t valid) {
-#pragma unroll
-  for (uint32_t w = 0; w < 4; ++w)
-    v[w] &= (2 * w < valid ? 0xffffu : 0u) | (2 * w + 1 < valid ? 0xffff0000u : 0u);
   return v;
 }
 // The same on a chunk in LDS.

@@ -85,8 +85,10 @@ __device__ __forceinline__ uint32_t mn_swz(uint32_t k) {
     return ((k >> 3) & 1u) << 1;
 }
 
+// Two workgroups share a CU except with 128 x 128 tiles (LDS); the registers of 64
+// x 64 tiles' kElements form have to be held to that (4 waves per SIMD).
 template <class T, bool TransposeLeft, bool TransposeRight, int Epi, int E, bool Split>
-__global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
+__global__ __launch_bounds__(T::kThreads, E == kElements && T::TM == 64 ? 4 : 1) void gemm_f16_tile_kernel(
     uint16_t* out, const uint16_t* __restrict__ left, const uint16_t* __restrict__ right,
     uint32_t M, uint32_t N, uint32_t K, uint64_t left_batch_stride, uint64_t right_batch_stride,
     const uint16_t* addend, uint64_t addend_batch_stride, uint32_t addend_row_stride,
@@ -204,7 +206,7 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
 
   // kElements: this thread's chunks of step k, read at element alignment.  Rows
   // past M or N repeat the last one and chunks run on into the next row (both
-  // reach only elements of C that are not stored); k past K is zero.
+  // reach only elements of C that are not stored); chunks past K are zero.
   auto load_regs = [&](uint32_t k, u32x4 (&v)[kDmaA + kDmaB]) __attribute__((always_inline)) {
     auto one = [&]<bool KContig, int TMN>(const uint16_t* X, uint32_t inst, uint32_t mn0, uint32_t MN) __attribute__((always_inline)) {
       uint32_t row, col;
@@ -214,9 +216,7 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
       if constexpr (KContig) {
         const uint64_t at_k = k0 + col;
         const uint32_t mn = mn0 + row < MN ? mn0 + row : MN - 1;
-        if (at_k >= K) return zero;
-        const u32x4 x = load_chunk(X, (uint64_t)mn * K + at_k, total);
-        return at_k + 8 <= K ? x : keep_elements(x, (uint32_t)(K - at_k));
+        return at_k < K ? load_chunk(X, (uint64_t)mn * K + at_k, total) : zero;
       } else {
         const uint64_t at_k = k0 + row;
         return at_k < K && mn0 + col < MN ? load_chunk(X, at_k * MN + mn0 + col, total) : zero;
@@ -227,7 +227,22 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
 #pragma unroll
     for (int j = 0; j < kDmaB; ++j) v[kDmaA + j] = one.template operator()<kBK_, TN>(B, wave * kDmaB + j, n0, N);
   };
-  auto store_regs = [&](uint8_t* stage, const u32x4 (&v)[kDmaA + kDmaB]) __attribute__((always_inline)) {
+  // Into step k's stage; the chunk that K ends in is cleared past K only here, so
+  // that no load of the last step waits for the one before.
+  auto store_regs = [&](uint8_t* stage, uint32_t k, u32x4 (&v)[kDmaA + kDmaB]) __attribute__((always_inline)) {
+    auto clear = [&]<bool KContig, int TMN>(u32x4& x, uint32_t inst) __attribute__((always_inline)) {
+      if constexpr (KContig) {
+        uint32_t row, col;
+        chunk_of.template operator()<KContig, TMN>(inst, &row, &col);
+        if (k_tail > col && k_tail - col < 8) x = keep_elements(x, k_tail - col);
+      }
+    };
+    if (k + 1 == ksteps && k_tail % 8 != 0) {
+#pragma unroll
+      for (int j = 0; j < kDmaA; ++j) clear.template operator()<kAK, TM>(v[j], wave * kDmaA + j);
+#pragma unroll
+      for (int j = 0; j < kDmaB; ++j) clear.template operator()<kBK_, TN>(v[kDmaA + j], wave * kDmaB + j);
+    }
 #pragma unroll
     for (int j = 0; j < kDmaA; ++j)
       *reinterpret_cast<u32x4*>(stage + (wave * kDmaA + j) * 1024 + lane * 16) = v[j];
@@ -239,8 +254,8 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
   if constexpr (kRegs) {
     load_regs(0, regs[0]);
     load_regs(1, regs[1]);
-    store_regs(lds0, regs[0]);
-    store_regs(lds1, regs[1]);
+    store_regs(lds0, 0, regs[0]);
+    store_regs(lds1, 1, regs[1]);
     load_regs(2, regs[0]);
     load_regs(3, regs[1]);
   } else {
@@ -322,7 +337,7 @@ __global__ __launch_bounds__(T::kThreads, 1) void gemm_f16_tile_kernel(
     if constexpr (kRegs) {
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (Tail <= 1) store_regs(ahead, regs[buf]);
+      if constexpr (Tail <= 1) store_regs(ahead, kt + 2, regs[buf]);
       if constexpr (Tail == 0) load_regs(kt + S, regs[buf]);
     } else {
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((Tail ? S - 1 - Tail : S - 2) * kDma) : "memory");

@@ -56,3 +56,21 @@ def test_gemm_f32_steps(ipus, ctx, M, N, step, steps, tail, tl):
     assert np.all(np.abs(raw[:M * N].reshape(M, N)[rows] - want) <= magnitude * (K + 2) * 2.0 ** -24)
     for x in (da, db, out):
         x.free()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (2, 1, 3), (1, 3, 2), (3, 1, 1), (1, 1, 7), (1, 1, 9), (9, 1, 1),
+                                   (5, 2, 67), (1, 9, 129), (17, 3, 131), (65, 67, 1)])
+@pytest.mark.parametrize("tl,tr", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_f16_operands_near_a_chunk(ipus, oracle, ctx, M, N, K, tl, tr):
+    """Odd rows read at element alignment: operands of fewer elements than a 16-byte
+    chunk, and ends of the operand inside one, with NaN behind them."""
+    a, b, af, bf = operands(ipus, oracle, M, N, K, tl, tr, 1, True)
+    pad = np.full(64, 0x7E00, np.uint16)
+    da, db = (ctx.upload(np.concatenate([pad[:1], x, pad])) for x in (a, b))
+    out = ctx.upload(np.full(M * N + 8, 0x7E00, np.uint16))
+    ctx.launch("ipu_stack_gemm_f16", out, [da.ptr + 2, db.ptr + 2], [1, M, N, K, tl, tr, 0, 0])
+    raw = out.download(np.uint16)
+    assert np.all(raw[M * N:] == 0x7E00)
+    assert_product(oracle.f16_to_f32(raw[:M * N]).reshape(1, M, N), af, bf, K)
+    for x in (da, db, out):
+        x.free()
