@@ -597,8 +597,7 @@ int launch_gemm_f16(hipStream_t stream, const GemmArgs& args) {
   // 285, 2048 x 2047 x 2048 228 -> 33, 1000 x 1001 x 1003 26.8 -> 10, 129 x 129 x 2001
   // 37 -> 12).
   const uint32_t plan_rows = shared ? (uint32_t)rows : a.rows, plan_batches = shared ? 1 : a.batches;
-  const uint32_t tile = gemm_f16_tile(plan_rows, a.columns, a.inner, plan_batches,
-                                      access == GemmAccess::kElement ? 128 : 256);
+  const uint32_t tile = gemm_f16_tile(plan_rows, a.columns, a.inner, plan_batches, access);
   if (tile != 256) return launch_gemm_f16_tile(stream, a, tile, access, plan_rows, plan_batches);
   const bool dwords = access == GemmAccess::kDword;
   switch (epilogue_of(a)) {

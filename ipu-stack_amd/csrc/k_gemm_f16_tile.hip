@@ -41,6 +41,7 @@
 #include "device_common.h"
 #include "gemm_common.h"
 #include "kernels.h"
+#include "tile_choice.h"
 #include "tile_grid.h"
 
 namespace ipus {
@@ -487,39 +488,6 @@ int launch_epilogue(hipStream_t stream, const GemmArgs& a, GemmAccess access, ui
 }
 
 }  // namespace
-
-// Modelled time of each tile size: a start-up (launch, first tiles, store of
-// C) and a time per 64-k step and round of 256 tiles, fitted to launches timed
-// on the chip (ns per step: 256 x 256 1.2 where few CUs work to 1.5 under the
-// power limit, 128 x 128 0.44-0.51, 64 x 64 0.14-0.20, 32 x 32 0.09-0.11 us).
-// Near the lines both sides are close: 3072^3 256 x 256 61.6 us, 128 x 128
-// 71.9; 729 x 4304 x 1152 128 x 128 11.8, 64 x 64 18.6; 1024^3 64 x 64 5.3, 128 x
-// 128 9.4, 32 x 32 9.2; 128 x 4096 x 4096 64 x 64 15.8, 32 x 32 18.3.  The choice
-// does not depend on the epilogue, so a fused epilogue gives the bits of the
-// separate kernels.
-uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches, uint32_t largest) {
-  struct Class {
-    uint32_t tile;
-    double start_us, step_us;
-  };
-  constexpr Class kClasses[] = {{256, 7.0, 1.35}, {128, 5.0, 0.50}, {64, 3.0, 0.19}, {32, 2.4, 0.10}};
-  const uint64_t steps = ((uint64_t)inner + 63) / 64;
-  uint32_t best = 0;
-  double best_us = 0;
-  for (const Class& c : kClasses) {
-    if (c.tile > largest) continue;
-    const uint64_t m = ((uint64_t)rows + c.tile - 1) / c.tile, n = ((uint64_t)columns + c.tile - 1) / c.tile;
-    const double tiles = (double)m * (double)n * (double)batches;
-    // Two workgroups of the smaller tiles share a CU.
-    const double rounds = tiles <= 256 ? 1.0 : c.tile >= 128 ? std::ceil(tiles / 256) : 2.0 * std::ceil(tiles / 512);
-    const double us = c.start_us + rounds * (double)steps * c.step_us;
-    if (best == 0 || us < best_us) {
-      best = c.tile;
-      best_us = us;
-    }
-  }
-  return best;
-}
 
 int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, GemmAccess access,
                          uint32_t plan_rows, uint32_t plan_batches) {

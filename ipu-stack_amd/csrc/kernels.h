@@ -7,6 +7,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "tile_choice.h"
+
 namespace ipus {
 
 // Device memory that launches on one stream share: partial results of kernels
@@ -65,15 +67,8 @@ struct AttentionArgs {
 
 // Dense products (k_gemm_f16.hip, k_gemm_f32.hip).
 int launch_gemm_f16(hipStream_t stream, const GemmArgs& a);
-// Tile edge (256, 128, 64 or 32) for an fp16 product that meets the LDS-DMA
-// kernels' conditions; the smaller ones are launched by launch_gemm_f16_tile
-// (k_gemm_f16_tile.hip), which does not check those conditions again.  access:
-// what every row pitch and address of the operands allows; kElement also
-// takes K = 0 and operands past the DMA's buffer ranges.  plan_rows and
-// plan_batches: those the tile was chosen for.
-uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches,
-                       uint32_t largest);
-enum class GemmAccess { kChunk, kDword, kElement };  // 16, 4, 2 bytes
+// The smaller tiles of gemm_f16_tile (tile_choice.h); the access is not checked
+// again.  plan_rows and plan_batches: those the tile was chosen for.
 int launch_gemm_f16_tile(hipStream_t stream, const GemmArgs& a, uint32_t tile, GemmAccess access,
                          uint32_t plan_rows, uint32_t plan_batches);
 // Whether launch_gemm_f16 or launch_gemm_f32 may split K over workgroups in this
