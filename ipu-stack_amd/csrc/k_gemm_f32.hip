@@ -3,8 +3,9 @@
 // output and accumulates in fp32 (gemm_f32_64_amp.S:40-56).
 //
 // Every shape runs the tile kernel (v_mfma_f32_16x16x4_f32, at the end of this
-// file) except K = 0 and operands past its 31-bit buffer ranges.  Those run
-// the 128 x 128 kernel (v_mfma_f32_32x32x2_f32): 16-byte aligned operands whose
+// file) except many tiles of a short sum (tile_f32), K = 0 and operands past
+// its 31-bit buffer ranges.  Those run the 128 x 128 kernel
+// (v_mfma_f32_32x32x2_f32): 16-byte aligned operands whose
 // contiguous axes, and N, are multiples of 4 with 16-byte loads (the kEdge
 // mode, off the 128 x 128 x 32 grid, zero-fills loads past M, N or K and stores
 // only rows < M and 4-column chunks < N), others in its kScalar mode with
@@ -28,10 +29,9 @@
 //     of C (one 16-byte store).
 #include "../../include/ipus.h"
 
-#include <cmath>
-
 #include "gemm_common.h"
 #include "kernels.h"
+#include "tile_choice.h"
 #include "tile_grid.h"
 
 namespace ipus {
@@ -597,17 +597,6 @@ int launch_tile32(hipStream_t stream, const GemmArgs& a, bool chunked) {
   return hip_status(hipGetLastError());
 }
 
-// Modelled time of the two tile sizes: start-up and time per 32-k step and
-// round of 256 tiles (us).  729 x 1152 x 1152: 64 x 64 20.9, 32 x 32 21.7; 512^3
-// 10.6 / 5.1; 1000 x 1004 x 1000 20.9 / 23.1.
-bool smaller_tiles(const GemmArgs& a) {
-  auto us = [&](uint32_t tile, double start, double step) {
-    const double tiles = (double)((a.rows + tile - 1) / tile) * ((a.columns + tile - 1) / tile) * a.batches;
-    return start + std::ceil(tiles / 256) * ((a.inner + 31) / 32) * step;
-  };
-  return us(32, 2.5, 0.15) < us(64, 3.0, 0.50);
-}
-
 }  // namespace
 
 int launch_gemm_f32(hipStream_t stream, const GemmArgs& a) {
@@ -631,8 +620,11 @@ int launch_gemm_f32(hipStream_t stream, const GemmArgs& a) {
   const uint64_t a_span = (a.transpose_left ? (uint64_t)a.rows : 64ull) * a.inner * 4;
   const uint64_t b_span = (a.transpose_right ? 64ull : (uint64_t)a.columns) * a.inner * 4;
   const bool floats = (uintptr_t)a.left % 4 == 0 && (uintptr_t)a.right % 4 == 0 && (uintptr_t)a.out % 4 == 0;
-  if (floats && a.inner > 0 && a_span < (1ull << 31) && b_span < (1ull << 31))
-    return smaller_tiles(a) ? launch_tile32<TileF32x32>(stream, a, vec) : launch_tile32<TileF32x64>(stream, a, vec);
+  if (floats && a.inner > 0 && a_span < (1ull << 31) && b_span < (1ull << 31)) {
+    const TileF32 tile = tile_f32(a.rows, a.columns, a.inner, a.batches, vec);
+    if (tile == TileF32::k64) return launch_tile32<TileF32x64>(stream, a, vec);
+    if (tile == TileF32::k32) return launch_tile32<TileF32x32>(stream, a, vec);
+  }
   if (!a.transpose_left && !a.transpose_right) return launch_fast<false, false>(stream, a, vec);
   if (!a.transpose_left && a.transpose_right) return launch_fast<false, true>(stream, a, vec);
   if (a.transpose_left && !a.transpose_right) return launch_fast<true, false>(stream, a, vec);

@@ -59,4 +59,24 @@ inline uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, u
   return best;
 }
 
+// Modelled time of the kernels, us, as gemm_f16_tile's: a start-up, and per round
+// of 256 tiles a fixed part and one per 32-k step (32 x 32 tiles: 64-k).  Kernel
+// times (128 x 128 with 16-byte loads, 64 x 64, 32 x 32) of M x N x K:
+//   4096 x 4096 x 32    20.6  30.3  67.2    1024 x 1024 x 64   7.9  4.8  6.0
+//   4096 x 4096 x 256   79.5  80.6   112    1024 x 1024 x 1000  76  21.6 24.1
+//   2392 x 2688 x 8     12.2  16.6  29.5    256 x 256 x 1000    76  19.5  6.9
+//   2760 x 960 x 64      9.4   8.8  12.8    800 x 1088 x 8 x 4 batches 8.1 9.3 15.8
+// The 128 x 128 kernel holds where C is most of the traffic (a short sum of many
+// tiles; 1960 x 1400 x 144 x 17 batches 152, 185, 263) and operands are whole chunks (element loads: 2392 x 2688 x 1 24.9 against 17.1).
+enum class TileF32 { k128, k64, k32 };
+inline TileF32 tile_f32(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches, bool chunked) {
+  auto us = [&](uint32_t tile, uint32_t step, double start, double round, double step_us) {
+    const double tiles = (double)(((uint64_t)rows + tile - 1) / tile) * (double)(((uint64_t)columns + tile - 1) / tile) * (double)batches;
+    return start + std::ceil(tiles / 256) * (round + (double)(((uint64_t)inner + step - 1) / step) * step_us);
+  };
+  const double us64 = us(64, 32, 3.0, 1.3, 0.45), us32 = us(32, 64, 2.5, 0.75, 0.245);
+  if (chunked && inner <= 256 && us(128, 32, 4.5, 2.0, 2.1) < std::fmin(us64, us32)) return TileF32::k128;
+  return us32 < us64 ? TileF32::k32 : TileF32::k64;
+}
+
 }  // namespace ipus

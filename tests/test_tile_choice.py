@@ -20,6 +20,8 @@ int main(int argc, char** argv) {
     auto n = [&](int k) { return (uint32_t)strtoul(argv[i + k], nullptr, 10); };
     if (argv[1][0] == '1')
       printf("%u\n", gemm_f16_tile(n(0), n(1), n(2), n(3), (GemmAccess)n(4)));
+    else
+      printf("%d\n", (int)tile_f32(n(0), n(1), n(2), n(3), n(4) != 0));
   }
 }
 """
@@ -57,6 +59,18 @@ F16 = {
     (1023, 1025, 441, 1, ELEMENT): {128: 10.2, 64: 7.9, 32: 15.5},
     (255, 257, 251, 1, ELEMENT): {128: 7.6, 64: 5.6, 32: 4.3},
 }
+# (M, N, K, batches, whole 16-byte chunks): kernel us on 128 x 128, 64 x 64 and 32 x
+# 32 tiles (128 x 128 only where the operands are whole chunks).
+F32 = {
+    (4096, 4096, 8, 1, 1): (21.0, 31.8, 67.6), (4096, 4096, 64, 1, 1): (29.2, 38.3, 63.0),
+    (4096, 4096, 1000, 1, 1): (273.8, 272.6, 330.2), (4096, 4096, 2, 1, 0): (48.1, 32.4, 78.8),
+    (2392, 2688, 8, 1, 1): (12.2, 16.6, 29.5), (2392, 2688, 256, 1, 1): (42.7, 37.7, 46.5),
+    (2760, 960, 64, 1, 1): (9.4, 8.8, 12.8), (1024, 1024, 8, 1, 1): (6.8, 4.2, 6.2),
+    (1024, 1024, 1000, 1, 1): (76.0, 21.6, 24.1), (256, 256, 256, 1, 1): (21.0, 7.0, 4.0),
+    (256, 256, 1000, 1, 1): (75.5, 19.5, 6.9), (8192, 64, 256, 1, 1): (21.5, 7.2, 5.9),
+    (800, 1088, 8, 4, 1): (8.1, 9.3, 15.8), (3336, 298, 8, 8, 0): (33.8, 19.4, 39.7),
+    (108, 384, 2, 26, 0): (11.1, 5.8, 8.2), (1960, 1400, 144, 17, 1): (152.3, 185.0, 262.9),
+}
 
 
 @pytest.fixture(scope="module")
@@ -88,3 +102,9 @@ def test_f16_tile_of_the_longest_rows(choose):
     shapes = [(2 ** 31 - 1, 2 ** 31 - 1, 8, 1, CHUNK), (2 ** 31 - 1, 8, 8, 1, CHUNK), (8, 8, 0, 1, ELEMENT),
               (2 ** 31 - 1, 2 ** 20, 2 ** 20, 65535, ELEMENT)]
     assert choose("16", shapes) == [256, 64, 32, 128]
+
+
+def test_f32_tile_is_near_the_fastest(choose):
+    for (shape, us), kernel in zip(F32.items(), choose("32", F32)):
+        assert shape[4] or kernel != 0, shape
+        assert us[kernel] <= 1.1 * min(us) + 0.3, (shape, kernel)
