@@ -727,7 +727,8 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd_kernel(
   const uint32_t group = Causal && QT == 2 ? 2 : group_arg;
   constexpr uint32_t kQPB = Fast<W, QT>::kQueriesPerBlock;
   const uint32_t qblocks = (query_rows + kQPB - 1) / kQPB;
-  const uint32_t per_stream = (qblocks + group - 1) / group;
+  const uint32_t shift = group - 1;  // group is 1 or 2
+  const uint32_t per_stream = (qblocks + shift) >> shift;
   const uint32_t total = per_stream * streams;
   uint32_t pid = blockIdx.x;
   if (total % 8 == 0) pid = (pid % 8) * (total / 8) + pid / 8;  // XCD-contiguous
@@ -741,7 +742,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd_kernel(
     if (group == 1) return qblocks - 1 - pos;
     return pos % 2 == 0 ? qblocks - 1 - pos / 2 : pos / 2;
   };
-  const uint32_t pos0 = i * group;
+  const uint32_t pos0 = i << shift;
   const uint32_t reps = qblocks - pos0 < group ? qblocks - pos0 : group;
   half8_t qf[QT][DC / 32];
   load_q<W, QT, DC>(qf, query, stream, qb_at(pos0), query_rows, width, q_heads);
