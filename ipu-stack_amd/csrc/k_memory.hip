@@ -1039,7 +1039,11 @@ bool launch_padded(hipStream_t stream, void* dst, const void* src, uint32_t orde
   const uint64_t rows = left ? (uint64_t)matrices * physical_rows : physical_rows;
   const uint32_t tiles_c = ceil_div(physical_columns, 64);
   const uint64_t tiles = ceil_div(rows, 32) * (uint64_t)tiles_c;
-  if (rows > 0xffffffffull || tiles > 0x7fffffffull || (!left && matrices > 65535)) return false;
+  if (rows > 0xffffffffull || tiles * kThreads >= (1ull << 32) || (!left && matrices > 65535)) return false;
+  // Few elements: one per thread fills the chip sooner (us, elements against
+  // chunks: 4096 x 9 to 16 columns 2.2 / 2.6, 8192 x 20 to 32 2.4 / 2.7, 32768 x 3
+  // to 16 3.2 / 2.9, 729 x 1152 5.3 / 3.5).
+  if ((uint64_t)matrices * physical_rows * physical_columns < 400000) return false;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles, left ? 1 : matrices), dim3(kThreads), 0, stream,
                        (uint16_t*)dst, (const uint16_t*)src, (uint32_t)rows, logical_rows, physical_rows,

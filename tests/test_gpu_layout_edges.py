@@ -118,3 +118,28 @@ def test_transpose_of_small_extents_keeps_the_chip_busy(ctx, matrices, rows, col
     assert us([matrices, rows, cols]) < 3.0 * us([1, side, side]) + 5.0
     src.free()
     dst.free()
+
+
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("matrices,lr,pr,lc,pc", [
+    (1, 24989, 24992, 3, 16), (1, 25008, 25008, 9, 16),    # either side of 400,000 elements
+    (3, 2085, 2096, 50, 64), (40, 200, 208, 20, 64), (1, 1, 16, 25001, 25008)])
+def test_padded_rearrange_routes(ipus, oracle, ctx, order, matrices, lr, pr, lc, pc):
+    test_padded_rearrange(ipus, oracle, ctx, order, 0, 0, matrices, lr, pr, lc, pc, 3)
+
+
+def test_padded_rearrange_of_one_long_row(ctx):
+    """AMP-Left tiles of 32 rows for a single one: more of them than a grid dimension
+    holds of 256 threads."""
+    n, pc = 1_100_000_007, 1_100_000_016
+    src, dst = ctx.alloc(2 * n), ctx.alloc(2 * pc)
+    window = ctx.alloc(32)
+    ctx.memset(src, 0x11)
+    ctx.launch("ipu_stack_rearrange_row_major_f16", dst, [src], [1, 1, 0, n, pc, 0, 0, 1])
+    for at in (0, n // 2 // 16 * 16, pc - 32):
+        ctx.launch("ipu_stack_copy", window, [dst.ptr + 2 * at], [32])
+        assert np.all(window.download(np.uint16) == 0x1111), at
+    ctx.launch("ipu_stack_copy", window, [dst.ptr + 2 * (pc - 16)], [32])
+    assert window.download(np.uint16).tolist() == [0x1111] * 7 + [0] * 9
+    for b in (src, dst, window):
+        b.free()
