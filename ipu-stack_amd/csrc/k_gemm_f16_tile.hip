@@ -205,9 +205,9 @@ __global__ __launch_bounds__(T::kThreads, E == kElements && T::TM == 64 ? 4 : 1)
       one.template operator()<kBK_, TN>(b_rsrc, stage + T::kABytes, wave * kDmaB + j, b_voff[j], k * b_kstep);
   };
 
-  // kElements: this thread's chunks of step k, read at element alignment.  Rows
-  // past M or N repeat the last one and chunks run on into the next row (both
-  // reach only elements of C that are not stored); chunks past K are zero.
+  // kElements: this thread's chunks of step k, read at element alignment.  Chunks
+  // run on into the next row (which reaches only elements of C that are not
+  // stored); rows past M or N and chunks past K are zero.
   auto load_regs = [&](uint32_t k, u32x4 (&v)[kDmaA + kDmaB]) __attribute__((always_inline)) {
     auto one = [&]<bool KContig, int TMN>(const uint16_t* X, uint32_t inst, uint32_t mn0, uint32_t MN) __attribute__((always_inline)) {
       uint32_t row, col;
@@ -216,8 +216,8 @@ __global__ __launch_bounds__(T::kThreads, E == kElements && T::TM == 64 ? 4 : 1)
       const u32x4 zero = {0, 0, 0, 0};
       if constexpr (KContig) {
         const uint64_t at_k = k0 + col;
-        const uint32_t mn = mn0 + row < MN ? mn0 + row : MN - 1;
-        return at_k < K ? load_chunk(X, (uint64_t)mn * K + at_k, total) : zero;
+        const uint32_t mn = mn0 + row;
+        return at_k < K && mn < MN ? load_chunk(X, (uint64_t)mn * K + at_k, total) : zero;
       } else {
         const uint64_t at_k = k0 + row;
         return at_k < K && mn0 + col < MN ? load_chunk(X, at_k * MN + mn0 + col, total) : zero;

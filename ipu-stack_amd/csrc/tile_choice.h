@@ -25,14 +25,15 @@ enum class GemmAccess { kChunk, kDword, kElement };  // 16, 4, 2 bytes
 // (a model without the fixed part of a round had taken small tiles for many
 // short sums: 4096 x 4096 x 64 22.8, 2592 x 4368 x 440 27.2.)  kElements, whose loads
 // pass through registers: 4095 x 4097 x 441 45.5 (128 x 128) 56.1 136, 1023 x 1025 x
-// 65 6.4 4.9 7.9.  The choice does not depend on the epilogue, so a fused epilogue
+// 65 6.4 4.9 7.9; operands past the buffer ranges: 32
+// x 49152 x 49152 1,027 on 64 x 64, 1,290 on 32 x 32.  The choice does not depend on the epilogue, so a fused epilogue
 // gives the bits of the separate kernels.
 inline uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches, GemmAccess access) {
   struct Class {
     uint32_t tile;
     double start_us, round_us, step_us, element_step_us;
   };
-  constexpr Class kClasses[] = {{128, 1.7, 3.6, 0.40, 0.90}, {64, 2.2, 1.2, 0.152, 0.33}, {32, 2.0, 0.75, 0.155, 0.40}};
+  constexpr Class kClasses[] = {{128, 1.7, 3.6, 0.40, 0.90}, {64, 2.2, 1.2, 0.152, 0.33}, {32, 2.0, 0.75, 0.155, 0.55}};
   auto tiles_of = [&](uint32_t tile) {
     return (double)(((uint64_t)rows + tile - 1) / tile) * (double)(((uint64_t)columns + tile - 1) / tile) * (double)batches;
   };
