@@ -23,11 +23,11 @@ enum class GemmAccess { kChunk, kDword, kElement };  // 16, 4, 2 bytes
 //   3072 x 3072 x 128     9.3  14.6  15.4  34.6    1024 x 1024 x 2048 35.5 15.4  7.8 15.9
 //   3093 x 1976 x 640    17.6  16.3  19.2  40.9    256 x 256 x 1024   21.2  8.6  5.2  4.0
 // (a model without the fixed part of a round had taken small tiles for many
-// short sums: 4096 x 4096 x 64 22.8, 2592 x 4368 x 440 27.2.)  kElements, whose loads
+// short sums: 4096 x 4096 x 64 22.8, 2592 x 4368 x 440 27.2).  kElements, whose loads
 // pass through registers: 4095 x 4097 x 441 45.5 (128 x 128) 56.1 136, 1023 x 1025 x
-// 65 6.4 4.9 7.9; operands past the buffer ranges: 32
-// x 49152 x 49152 1,027 on 64 x 64, 1,290 on 32 x 32.  The choice does not depend on the epilogue, so a fused epilogue
-// gives the bits of the separate kernels.
+// 65 6.4 4.9 7.9, and past the buffer ranges 32 x 49152 x 49152 1,027 on 64 x 64, 1,290
+// on 32 x 32.  The choice does not depend on the epilogue, so a fused epilogue gives
+// the bits of the separate kernels.
 inline uint32_t gemm_f16_tile(uint32_t rows, uint32_t columns, uint32_t inner, uint64_t batches, GemmAccess access) {
   struct Class {
     uint32_t tile;

@@ -17,7 +17,7 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 BUILD = os.path.join(ROOT, "ipu-stack_amd", "_build")
-SOURCES = ("k_memory", "k_gemm_f16", "k_gemm_f32", "k_attention", "k_calibrate")
+SOURCES = ("k_memory", "k_gemm_f16", "k_gemm_f16_tile", "k_gemm_f32", "k_attention", "k_calibrate")
 LINE = re.compile(r"remark:\s+(?P<key>[^:]+?):\s+(?P<value>\S+)\s+\[-Rpass-analysis")
 
 
@@ -75,8 +75,11 @@ def test_no_kernel_uses_scratch_memory(kernels):
     # Some instantiations of the 256 x 256 GEMM spill two or three values
     # across their K loop (stored before it, reloaded in the epilogue; no
     # scratch access inside the loop); nothing else may touch scratch.
+    # So do the 64 x 64 tiles' element form with the left operand transposed (three
+    # epilogues), held to 128 registers for two workgroups per CU.
+    element64 = re.compile(r"gemm_f16_tile_kernel\S*ILi64ELi64E\S*ELb1ELb0ELi\dELi3ELb0E")
     for name, f in kernels.items():
-        limit = 16 if "gemm_f16_256_kernel" in name else 0
+        limit = 16 if "gemm_f16_256_kernel" in name else 24 if element64.search(name) else 0
         assert int(f["ScratchSize [bytes/lane]"]) <= limit, (name, f)
         assert f.get("Dynamic Stack", "False") == "False", name
 
@@ -105,3 +108,13 @@ def test_memory_kernels_need_no_agprs_or_scratch(kernels):
             continue
         assert int(f["AGPRs"]) == 0, (name, f)
         assert int(f["VGPRs Spill"]) == 0 and int(f["SGPRs Spill"]) == 0, (name, f)
+
+
+def test_gemm_tile_kernels_share_a_cu(kernels):
+    # 64 x 64 and 32 x 32 tiles: two workgroups per CU by LDS and registers
+    # (512 threads: 4 waves per SIMD, 256 threads: 2).
+    for name, f in matching(kernels, "_tile_kernel").items():
+        m = re.search(r"TileShape(?:F32)?ILi(\d+)E", name)
+        if int(m.group(1)) < 128:
+            assert int(f["LDS Size [bytes/block]"]) <= 81920, (name, f)
+            assert int(f["Occupancy [waves/SIMD]"]) >= (4 if m.group(1) == "64" else 2), (name, f)
