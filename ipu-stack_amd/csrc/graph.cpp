@@ -608,11 +608,11 @@ int build_error(const std::string& message) {
 // Split-K count for an fp16 GEMM on the 256 x 256 kernel: min(16, K / 1024,
 // 64 / tiles), i.e. only for outputs of at most 32 tiles and K >= 6144, with
 // every split keeping >= 1024 k and about 64 workgroups in all.  The line was
-// measured against the unsplit kernel that the tile kernel replaced; today
-// (us, unsplit against split) 256 x 1024 x 16384 43 / 37 keeps the split ahead, 64 x
-// 64 x 40000 13 / 51, 256 x 256 x 8192 11 / 32 and 1024 x 1024 x 8192 29 / 51 do
-// not: callers see the plan's steps, so it stays.  Returns 1 (no split)
-// when the shape is outside the fast kernel's reach.
+// measured against the unsplit kernel that the tile kernels replaced, and now
+// lies too low: (us, unsplit against split) 256 x 1024 x 16384 43 / 37 keeps the
+// split ahead, but 64 x 64 x 40000 13 / 51, 256 x 256 x 8192 11 / 32 and 1024 x 1024 x
+// 8192 29 / 51 do not, so a session runs those slower than a launch of the
+// product.  Returns 1 (no split) when the shape is outside the fast kernel's reach.
 uint32_t gemm_splits(uint32_t M, uint32_t N, uint32_t K, uint64_t batches, bool tl, bool tr) {
   if (K < 6144 || K % 8 != 0 || N % 8 != 0 || (tl && M % 8 != 0)) return 1;
   const uint64_t a_span = tl ? (uint64_t)K * M * 2 : 256ull * K * 2;
