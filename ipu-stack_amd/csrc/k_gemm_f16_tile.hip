@@ -259,11 +259,6 @@ __global__ __launch_bounds__(T::kThreads, E == kElements && T::TM == 64 ? 4 : 1)
     store_regs(lds1, 1, regs[1]);
     load_regs(2, regs[0]);
     load_regs(3, regs[1]);
-  } else {
-    dma(lds0, 0);
-    dma(lds1, 1);
-    dma(lds2, 2);
-    dma(lds3, 3);
   }
 
   auto k_base = [&](uint32_t w0) { return (w0 + r16) * 128 + ((g4 ^ (r16 & 7)) << 4); };
@@ -319,11 +314,14 @@ __global__ __launch_bounds__(T::kThreads, E == kElements && T::TM == 64 ? 4 : 1)
 
   constexpr int kDma = T::kDma;
   constexpr int kMfma = kSub * kMT * kNT, kReads = kSub * kItems;
-  if constexpr (kRegs) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * kDma) : "memory");
-  if (E == kDwords && ksteps == 1) clear_past_k(lds0);
+  // The first step's fragments, with the DMA of `Behind` stages still in flight.
+  auto start = [&]<int Behind>() __attribute__((always_inline)) {
+    if constexpr (kRegs) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(Behind * kDma) : "memory");
+    if (E == kDwords && ksteps == 1) clear_past_k(lds0);
 #pragma unroll
-  for (int r = 0; r < kReads; ++r) read_item(lds0, 0, r);
+    for (int r = 0; r < kReads; ++r) read_item(lds0, 0, r);
+  };
   // Step kt: its fragments are in register buffer buf.  After the barrier
   // every wave's DMA of stage kt + 1 (`next`) has landed and every wave's
   // reads of stage kt (`cur`) have returned, so cur takes the DMA of step
@@ -360,16 +358,32 @@ __global__ __launch_bounds__(T::kThreads, E == kElements && T::TM == 64 ? 4 : 1)
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  uint32_t kt = 0;
-  for (; kt + 3 < ksteps; kt += 4) {
-    step.template operator()<0>(lds0, lds1, lds2, 0, kt);
-    step.template operator()<0>(lds1, lds2, lds3, 1, kt + 1);
-    step.template operator()<0>(lds2, lds3, lds0, 0, kt + 2);
-    step.template operator()<0>(lds3, lds0, lds1, 1, kt + 3);
+  if (!kRegs && ksteps <= 2) {
+    // Nothing to issue past the second stage: 256^3 replayed 3.01 -> 2.91 us.
+    dma(lds0, 0);
+    dma(lds1, 1);
+    start.template operator()<1>();
+    step.template operator()<3>(lds0, lds1, lds2, 0, 0);
+    if (ksteps == 2) step.template operator()<3>(lds1, lds2, lds3, 1, 1);
+  } else {
+    if constexpr (!kRegs) {
+      dma(lds0, 0);
+      dma(lds1, 1);
+      dma(lds2, 2);
+      dma(lds3, 3);
+    }
+    start.template operator()<S - 1>();
+    uint32_t kt = 0;
+    for (; kt + 3 < ksteps; kt += 4) {
+      step.template operator()<0>(lds0, lds1, lds2, 0, kt);
+      step.template operator()<0>(lds1, lds2, lds3, 1, kt + 1);
+      step.template operator()<0>(lds2, lds3, lds0, 0, kt + 2);
+      step.template operator()<0>(lds3, lds0, lds1, 1, kt + 3);
+    }
+    if (kt < ksteps) step.template operator()<1>(lds0, lds1, lds2, 0, kt);
+    if (kt + 1 < ksteps) step.template operator()<2>(lds1, lds2, lds3, 1, kt + 1);
+    if (kt + 2 < ksteps) step.template operator()<3>(lds2, lds3, lds0, 0, kt + 2);
   }
-  if (kt < ksteps) step.template operator()<1>(lds0, lds1, lds2, 0, kt);
-  if (kt + 1 < ksteps) step.template operator()<2>(lds1, lds2, lds3, 1, kt + 1);
-  if (kt + 2 < ksteps) step.template operator()<3>(lds2, lds3, lds0, 0, kt + 2);
   // Every DMA has landed (those past the last step too) and every wave is done
   // with the stages.
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
