@@ -73,3 +73,11 @@ def test_traffic_table_scales_by_the_copy_kernel(tmp_path):
     assert float(cells[3]) == pytest.approx(2 * copy_bytes / 1e6, abs=0.01)
     assert float(cells[4]) == pytest.approx(copy_bytes / 1e6, abs=0.01)
     assert "    a" in text and "    b" in text
+
+
+def test_committed_traffic_is_of_the_current_sources():
+    """roofline.traffic of bench.py is null once a source that the headline kernel
+    includes, or that chooses it, has changed without the counters measured again."""
+    traffic, note = bench.committed_traffic()
+    assert traffic is not None, note
+    assert traffic == pytest.approx(1.745e9, rel=0.02)
