@@ -36,8 +36,6 @@
 // element alignment two steps before they are stored to LDS.
 #include "../../include/ipus.h"
 
-#include <cmath>
-
 #include "device_common.h"
 #include "gemm_common.h"
 #include "kernels.h"
